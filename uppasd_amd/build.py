@@ -25,10 +25,15 @@ ARCH = "gfx950"
 HIP_COMMON = [f"--offload-arch={ARCH}", "-O3", "-fPIC", "-std=c++17",
               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
               "-Wno-unused-command-line-argument"]
+# (source, object, flags); the tile kernels one solver and arithmetic type at a time
 UNITS = [
-    ("uasd_kernels_f64.hip", ["-ffp-contract=off"]),
-    ("uasd_kernels_f32.hip", ["-ffp-contract=fast"]),
-    ("uasd_engine.hip", ["-ffp-contract=off"]),
+    ("uasd_kernels_f64.hip", "uasd_kernels_f64.o", ["-ffp-contract=off"]),
+    ("uasd_kernels_f32.hip", "uasd_kernels_f32.o", ["-ffp-contract=fast"]),
+    ("uasd_engine.hip", "uasd_engine.o", ["-ffp-contract=off"]),
+] + [
+    ("uasd_tile.hip", f"uasd_tile_{r}_{alg}.o", [f"-DUASD_REAL={r}", f"-DUASD_ALG={alg}", fp])
+    for r, fp in (("double", "-ffp-contract=off"), ("float", "-ffp-contract=fast"))
+    for alg in (1, 4, 5, 6, 7)
 ]
 
 
@@ -50,15 +55,15 @@ def build(verbose: bool = False) -> str:
     before = _source_digest()
     # the translation units are independent: compile them side by side
     cmds, objs = [], []
-    for src, extra in UNITS:
-        obj = os.path.join(objdir, src.replace(".hip", ".o"))
+    for src, name, extra in UNITS:
+        obj = os.path.join(objdir, name)
         cmds.append([HIPCC, *HIP_COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
     setup_obj = os.path.join(objdir, "uasd_setup.o")
     cmds.append(["g++", "-O2", "-fPIC", "-std=c++17", "-fopenmp", "-ffp-contract=off",
                  "-c", os.path.join(CSRC, "uasd_setup.cpp"), "-o", setup_obj])
     objs.append(setup_obj)
-    with ThreadPoolExecutor(max_workers=len(cmds)) as pool:
+    with ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 8)) as pool:
         for f in [pool.submit(_run, c, verbose) for c in cmds]:
             f.result()
     tmp = LIB + ".tmp"

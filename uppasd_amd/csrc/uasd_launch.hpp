@@ -7,6 +7,13 @@
 
 namespace uasd {
 
+// Grid for n work items, padded to a multiple of the XCD count (the kernels
+// remap blockIdx so each XCD takes a contiguous range; padding blocks exit).
+inline unsigned grid_for(int64_t n, int block) {
+  const int64_t b = (n + block - 1) / block;
+  return (unsigned)((b + kXCD - 1) / kXCD * kXCD);
+}
+
 constexpr int kBlock = 256;  // largest workgroup the kernels are built for
 
 // Launch shape of the gathering kernels (chosen by the autotuner):
@@ -71,6 +78,11 @@ template <typename R>
 hipError_t launch_llg_tile(hipStream_t s, TileDev t, int pipe, int alg, int half,
                            const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e,
                            Quad<R> *p, Quad<R> *b2, Quad<R> *out);
+// The same for one solver; uasd_tile.hip instantiates each (R, ALG).
+template <typename R, int ALG>
+hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, const HamDev<R> &h,
+                               const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p, Quad<R> *b2,
+                               Quad<R> *out);
 // LDS bytes the tile kernel needs for a halo tile of hv cells
 // Component plane size of k_llg_tile for NA*HV halo values: the smallest of
 // kTilePlanes that holds them, or 0.
