@@ -678,9 +678,11 @@ int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
   return toc(c, half);
 }
 
-// parts: also write beff1 and beff2 into quad arrays 1 and 2 of c->field.
+// parts: also write beff1 and beff2 into quad arrays 1 and 2 of c->field;
+// want_beff = false: the energy alone.
 template <typename R>
-int run_field(uasd_ctx *c, bool from_scratch, bool want_energy, bool parts = false) {
+int run_field(uasd_ctx *c, bool from_scratch, bool want_energy, bool parts = false,
+              bool want_beff = true) {
   uasd::HamDev<R> h = ham_view<R>(c);
   const uasd::Quad<R> *src = from_scratch ? quads<R>(c, c->scratch) : quads<R>(c, c->spins, 0);
   HIP_TRY(c->field.ensure(std::max(c->field.bytes, (parts ? 3 : 1) * quad_bytes(c))));
@@ -690,7 +692,7 @@ int run_field(uasd_ctx *c, bool from_scratch, bool want_energy, bool parts = fal
     en = c->energy.as<double>();
   }
   tic(c, 2);
-  HIP_TRY(uasd::launch_field<R>(c->stream, c->tune[1], h, src, quads<R>(c, c->field), en,
+  HIP_TRY(uasd::launch_field<R>(c->stream, c->tune[1], h, src, want_beff ? quads<R>(c, c->field) : nullptr, en,
                                 parts ? quads<R>(c, c->field, 1) : nullptr));
   return toc(c, 2);
 }
@@ -700,7 +702,7 @@ int run_field(uasd_ctx *c, bool from_scratch, bool want_energy, bool parts = fal
 template <typename R>
 int reduce_moments(uasd_ctx *c, bool with_energy, bool from_scratch, std::vector<double> &out) {
   const int nv = with_energy ? 4 : 3;
-  const int nblocks = std::max(1, std::min(1024, (c->N + 4095) / 4096));
+  const int nblocks = std::max(1, std::min(1024, (c->N + 255) / 256));
   HIP_TRY(c->partial.ensure((size_t)c->M * nblocks * nv * sizeof(double)));
   HIP_TRY(c->redout.ensure((size_t)c->M * nv * sizeof(double)));
   const uasd::Quad<R> *s = from_scratch ? quads<R>(c, c->scratch) : quads<R>(c, c->spins, 0);
@@ -960,14 +962,32 @@ int make_tile(uasd_ctx *c, int k, uasd::TileDev &t) {
 }
 
 // ------------------------------------------------------------ segments
-constexpr int kSegChunk = 4096;  // sites per reduction chunk
+// Sites per reduction chunk, one workgroup each: the fewest, from 256 (a site
+// per thread) up to 4096, whose partial sums fit the fixed scratch of
+// uasd_energy_terms_noalloc, so that entry point sums in the same order as
+// uasd_energy_terms.  Small chunks fill the chip: calc_energy's terms of
+// 221,184 sites with 58 neighbours took 202 us in 54 chunks of 4096 sites (54
+// workgroups cannot fill 256 CUs); 864 chunks of 256 took 166 us off a pass of
+// field, energy terms and moment sums (1012 -> 846 us, host copies included).
+constexpr int kSegChunkMax = 4096;
+
+int seg_chunk_size(int nseg, const int *off, int M) {
+  int size = 256;
+  for (; size < kSegChunkMax; size *= 2) {
+    size_t n = nseg;
+    for (int s = 0; s < nseg; ++s) n += ((size_t)(off[s + 1] - off[s]) + size - 1) / size;
+    if (n * M * 4 <= kScratchDoubles) break;
+  }
+  return size;
+}
 
 int set_segments(uasd_ctx *c, int nseg, const int *off) {
   std::vector<int> chunks, seg_chunk(1, 0), seg_n;
+  const int size = seg_chunk_size(nseg, off, c->M);
   for (int s = 0; s < nseg; ++s) {
-    for (int a = off[s]; a < off[s + 1]; a += kSegChunk) {
+    for (int a = off[s]; a < off[s + 1]; a += size) {
       chunks.push_back(a);
-      chunks.push_back(std::min(off[s + 1], a + kSegChunk));
+      chunks.push_back(std::min(off[s + 1], a + size));
     }
     seg_chunk.push_back((int)chunks.size() / 2);
     seg_n.push_back(off[s + 1] - off[s]);
@@ -2091,8 +2111,8 @@ int uasd_measure(uasd_ctx *c, double *msum, double *energy) {
   if (energy) {
     if (!c->have_ex) return fail(UASD_ERR_STATE, "exchange not set");
     if (int r = rebuild_classes(c)) return r;
-    int r = c->prec == UASD_FP64 ? run_field<double>(c, false, true)
-                                 : run_field<float>(c, false, true);
+    int r = c->prec == UASD_FP64 ? run_field<double>(c, false, true, false, false)
+                                 : run_field<float>(c, false, true, false, false);
     if (r) return r;
   }
   std::vector<double> red;
@@ -2169,8 +2189,8 @@ int uasd_measure_segments(uasd_ctx *c, double *msum, double *energy) {
   if (energy) {
     if (!c->have_ex) return fail(UASD_ERR_STATE, "exchange not set");
     if (int r = rebuild_classes(c)) return r;
-    int r = c->prec == UASD_FP64 ? run_field<double>(c, false, true)
-                                 : run_field<float>(c, false, true);
+    int r = c->prec == UASD_FP64 ? run_field<double>(c, false, true, false, false)
+                                 : run_field<float>(c, false, true, false, false);
     if (r) return r;
   }
   int r = c->prec == UASD_FP64 ? segment_sums<double>(c, energy != nullptr)
@@ -2269,8 +2289,8 @@ int uasd_accumulate(uasd_ctx *c, int with_energy) {
   if (with_energy) {
     if (!c->have_ex) return fail(UASD_ERR_STATE, "exchange not set");
     if (int r = rebuild_classes(c)) return r;
-    int r = c->prec == UASD_FP64 ? run_field<double>(c, false, true)
-                                 : run_field<float>(c, false, true);
+    int r = c->prec == UASD_FP64 ? run_field<double>(c, false, true, false, false)
+                                 : run_field<float>(c, false, true, false, false);
     if (r) return r;
   }
   int r = c->prec == UASD_FP64 ? segment_sums<double>(c, with_energy != 0)

@@ -1003,8 +1003,8 @@ __device__ __forceinline__ void midpoint_solve(R A0, R A1, R A2, R e0, R e1, R e
 
 // =================================================================== kernels
 
-// effective_field_full over all (site, ens): beff (quads, w unused) and, when
-// en != null, the per-site field-routine energy -m.(0.5*(bs+2bq+2bext)) in FP64;
+// effective_field_full over all (site, ens): beff (quads, w unused; null where
+// only the energy is wanted) and, when en != null, the per-site field-routine energy -m.(0.5*(bs+2bq+2bext)) in FP64;
 // when parts != null also beff1 = bs into parts[q] and beff2 = bq + bext into
 // parts[N*M + q] (hamiltonianactions.f90:240-241).
 template <typename R, int G>
@@ -1017,12 +1017,9 @@ __global__ void __launch_bounds__(256) k_field(HamDev<R> h, const Quad<R> *__res
   const int site = (int)fast_div((uint32_t)q, h.mdiv), ens = (int)q - site * h.M;
   R s0, s1, s2, q0, q1, q2, x0, x1, x2;
   site_field<R, G>(h, src, site, ens, s0, s1, s2, q0, q1, q2, x0, x1, x2);
-  Quad<R> b;
-  b.x = (R)0 + s0 + (q0 + x0 + (R)0);
-  b.y = (R)0 + s1 + (q1 + x1 + (R)0);
-  b.z = (R)0 + s2 + (q2 + x2 + (R)0);
-  b.w = (R)0;
-  beff[q] = b;
+  if (beff)
+    beff[q] = Quad<R>{(R)0 + s0 + (q0 + x0 + (R)0), (R)0 + s1 + (q1 + x1 + (R)0),
+                      (R)0 + s2 + (q2 + x2 + (R)0), (R)0};
   if (parts) {
     parts[q] = Quad<R>{s0, s1, s2, (R)0};
     parts[total + q] = Quad<R>{q0 + x0 + (R)0, q1 + x1 + (R)0, q2 + x2 + (R)0, (R)0};
@@ -1975,6 +1972,38 @@ __global__ void __launch_bounds__(256) k_mc_colour(HamDev<R> h, MCParams mp, Qua
 }
 
 // ---------------------------------------------------------- FP64 reductions
+// The measurement sums are short: what bounds them is how many workgroups they
+// fill the chip with and the length of their serial chains, not memory.  A
+// workgroup therefore sums a few hundred sites (chunks of 256 where the
+// partial sums fit, see set_segments), its threads' values meet in a tree, and
+// the partials of a sum are added by a whole wavefront.  Both orders are fixed
+// by the sizes alone, so a sum gives the same bits every time.
+
+// Adds the values a[0..NV) of the threads t, t + S, t + 2S, ... of a workgroup
+// of 256 (S a power of two): thread t < S ends up with their sum.  A tree in
+// LDS, every halving step the same for all sums.
+template <int NV>
+__device__ __forceinline__ void block_sum(double (&a)[NV], int S) {
+  __shared__ double red[NV][256];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) red[v][threadIdx.x] = a[v];
+  for (int w = 128; w >= S; w >>= 1) {
+    __syncthreads();
+    if ((int)threadIdx.x < w) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) red[v][threadIdx.x] = a[v] = a[v] + red[v][threadIdx.x + w];
+    }
+  }
+}
+
+// Sum over groups of LW adjacent lanes of a wavefront, in the first lane of each.
+template <int LW>
+__device__ __forceinline__ double lane_sum(double x) {
+#pragma unroll
+  for (int off = LW / 2; off > 0; off >>= 1) x += __shfl_down(x, off, LW);
+  return x;
+}
+
 // Stage 1: block b sums sites [b*chunk, (b+1)*chunk) of ensemble blockIdx.y:
 // the three components of emomM = xyz*w (and the energy term when en != null).
 template <typename R, int NV>
@@ -1984,49 +2013,37 @@ __global__ void __launch_bounds__(256)
   const int ens = blockIdx.y;
   const int b = blockIdx.x;
   const int s0 = b * chunk, s1 = min(N, s0 + chunk);
-  double a0 = 0.0, a1 = 0.0, a2 = 0.0, a3 = 0.0;
+  double a[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) a[v] = 0.0;
   for (int i = s0 + (int)threadIdx.x; i < s1; i += blockDim.x) {
     const size_t q = (size_t)i * M + ens;
     const Quad<R> v = s[q];
     const double m = (double)v.w;
-    a0 += (double)v.x * m;
-    a1 += (double)v.y * m;
-    a2 += (double)v.z * m;
-    if (NV > 3) a3 += en[q];
+    a[0] += (double)v.x * m;
+    a[1] += (double)v.y * m;
+    a[2] += (double)v.z * m;
+    if (NV > 3) a[3] += en[q];
   }
-  __shared__ double red[4][256 / 64];
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  block_sum<NV>(a, 1);
+  if (threadIdx.x == 0) {
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    a0 += __shfl_down(a0, off, 64);
-    a1 += __shfl_down(a1, off, 64);
-    a2 += __shfl_down(a2, off, 64);
-    if (NV > 3) a3 += __shfl_down(a3, off, 64);
-  }
-  if (lane == 0) {
-    red[0][wid] = a0;
-    red[1][wid] = a1;
-    red[2][wid] = a2;
-    red[3][wid] = a3;
-  }
-  __syncthreads();
-  if (threadIdx.x < NV) {
-    double x = 0.0;
-    for (int w = 0; w < (int)(blockDim.x / 64); ++w) x += red[threadIdx.x][w];
-    partial[((size_t)ens * gridDim.x + b) * NV + threadIdx.x] = x;
+    for (int v = 0; v < NV; ++v) partial[((size_t)ens * gridDim.x + b) * NV + v] = a[v];
   }
 }
 
-// Stage 2: one thread per (ensemble, value) sums the block partials in order.
+// Stage 2: one wavefront per (ensemble, value) adds the block partials.
 template <int NV>
-__global__ void k_reduce_stage2(int M, int nblocks, const double *__restrict__ partial,
-                                double *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) k_reduce_stage2(int M, int nblocks,
+                                                       const double *__restrict__ partial,
+                                                       double *__restrict__ out) {
+  const int t = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64, lane = threadIdx.x & 63;
   if (t >= M * NV) return;
   const int ens = t / NV, v = t - ens * NV;
   double x = 0.0;
-  for (int b = 0; b < nblocks; ++b) x += partial[((size_t)ens * nblocks + b) * NV + v];
-  out[t] = x;
+  for (int b = lane; b < nblocks; b += 64) x += partial[((size_t)ens * nblocks + b) * NV + v];
+  x = lane_sum<64>(x);
+  if (lane == 0) out[t] = x;
 }
 
 // ------------------------------------------------- per-replica reductions
@@ -2054,16 +2071,11 @@ __global__ void __launch_bounds__(256)
     a[2] += (double)x.z * m;
     if (NV > 3) a[3] += en[q];
   }
-  __shared__ double red[256][NV];
+  block_sum<NV>(a, M);
+  if ((int)threadIdx.x < M) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) red[threadIdx.x][v] = a[v];
-  __syncthreads();
-  // M*NV partials: more than the workgroup's threads once M > blockDim/NV
-  for (int t = (int)threadIdx.x; t < M * NV; t += (int)blockDim.x) {
-    const int ens = t / NV, v = t - ens * NV;
-    double x = 0.0;
-    for (int j = ens; j < (int)blockDim.x; j += M) x += red[j][v];
-    partial[((size_t)blockIdx.x * M + ens) * NV + v] = x;
+    for (int v = 0; v < NV; ++v)
+      partial[((size_t)blockIdx.x * M + threadIdx.x) * NV + v] = a[v];
   }
 }
 
@@ -2086,29 +2098,33 @@ __global__ void __launch_bounds__(256)
     a[2] += (double)x.z * m;
     if (NV > 3) a[3] += en[q];
   }
-  __shared__ double red[256][NV];
+  block_sum<NV>(a, 1);
+  if (threadIdx.x == 0) {
 #pragma unroll
-  for (int v = 0; v < NV; ++v) red[threadIdx.x][v] = a[v];
-  __syncthreads();
-  if ((int)threadIdx.x < NV) {
-    double x = 0.0;
-    for (int j = 0; j < (int)blockDim.x; ++j) x += red[j][threadIdx.x];
-    partial[((size_t)blockIdx.x * M + ens) * NV + threadIdx.x] = x;
+    for (int v = 0; v < NV; ++v) partial[((size_t)blockIdx.x * M + ens) * NV + v] = a[v];
   }
 }
 
-// One thread per (segment, ensemble, value): the segment's chunk partials
-// summed in chunk order into out[(seg*M + ens)*NV + v].
-template <int NV>
-__global__ void k_segsum_final(int nseg, int M, const int *__restrict__ seg_chunk,
-                               const double *__restrict__ partial, double *__restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nseg * M * NV) return;
-  const int v = t % NV, se = t / NV, ens = se % M, seg = se / M;
-  double x = 0.0;
-  for (int c = seg_chunk[seg]; c < seg_chunk[seg + 1]; ++c)
-    x += partial[((size_t)c * M + ens) * NV + v];
-  out[t] = x;
+// LW lanes per (segment, ensemble, value): the segment's chunk partials added
+// into out[(seg*M + ens)*NV + v].  A whole wavefront where a segment has many
+// chunks, eight lanes where it has few (batches of many small segments).
+template <int NV, int LW>
+__global__ void __launch_bounds__(256)
+    k_segsum_final(int nseg, int M, const int *__restrict__ seg_chunk,
+                   const double *__restrict__ partial, double *__restrict__ out) {
+  const int lane = threadIdx.x & (LW - 1);
+  const int64_t total = (int64_t)nseg * M * NV, stride = (int64_t)gridDim.x * (256 / LW);
+  for (int64_t t = (int64_t)blockIdx.x * (256 / LW) + threadIdx.x / LW; t < total; t += stride) {
+    const int v = (int)(t % NV);
+    const int64_t se = t / NV;
+    const int ens = (int)(se % M), seg = (int)(se / M);
+    const int c1 = seg_chunk[seg + 1];
+    double x = 0.0;
+    for (int c = seg_chunk[seg] + lane; c < c1; c += LW)
+      x += partial[((size_t)c * M + ens) * NV + v];
+    x = lane_sum<LW>(x);
+    if (lane == 0) out[t] = x;
+  }
 }
 
 // ------------------------------------------------- term-resolved energies
@@ -2180,14 +2196,10 @@ __global__ void __launch_bounds__(256)
       a[3] += update_ene(m0, m1, m2, v.x, v.y, v.z, 1.0);
     }
   }
-  __shared__ double red[256][4];
+  block_sum<4>(a, 1);
+  if (threadIdx.x == 0) {
 #pragma unroll
-  for (int v = 0; v < 4; ++v) red[threadIdx.x][v] = a[v];
-  __syncthreads();
-  if ((int)threadIdx.x < 4) {
-    double x = 0.0;
-    for (int j = 0; j < (int)blockDim.x; ++j) x += red[j][threadIdx.x];
-    partial[((size_t)blockIdx.x * M + ens) * 4 + threadIdx.x] = x;
+    for (int v = 0; v < 4; ++v) partial[((size_t)blockIdx.x * M + ens) * 4 + v] = a[v];
   }
 }
 

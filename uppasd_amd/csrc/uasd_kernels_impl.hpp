@@ -2,6 +2,7 @@
 // uasd_launch.hpp, instantiated for one arithmetic type by the including
 // translation unit.
 #pragma once
+#include <algorithm>
 #include <type_traits>
 
 #include "uasd_launch.hpp"
@@ -138,14 +139,30 @@ hipError_t launch_reduce(hipStream_t s, int N, int M, const Quad<R> *spins, cons
   if (nv == 4) {
     hipLaunchKernelGGL((k_reduce_stage1<R, 4>), g1, dim3(kBlock), 0, s, N, M, chunk, spins, en,
                        partial);
-    hipLaunchKernelGGL(k_reduce_stage2<4>, dim3((M * 4 + 63) / 64), dim3(64), 0, s, M, nblocks,
+    hipLaunchKernelGGL(k_reduce_stage2<4>, dim3(M), dim3(kBlock), 0, s, M, nblocks,
                        partial, out);
   } else {
     hipLaunchKernelGGL((k_reduce_stage1<R, 3>), g1, dim3(kBlock), 0, s, N, M, chunk, spins, en,
                        partial);
-    hipLaunchKernelGGL(k_reduce_stage2<3>, dim3((M * 3 + 63) / 64), dim3(64), 0, s, M, nblocks,
+    hipLaunchKernelGGL(k_reduce_stage2<3>, dim3((M * 3 + 3) / 4), dim3(kBlock), 0, s, M, nblocks,
                        partial, out);
   }
+  return hipGetLastError();
+}
+
+// The chunk partials of every (segment, ensemble, value) summed.
+template <int NV>
+static hipError_t segsum_final(hipStream_t s, int nseg, int M, int nchunks, const int *seg_chunk,
+                               const double *partial, double *out) {
+  const bool wave = nchunks >= 16 * (int64_t)nseg;  // many chunks per segment
+  const int64_t per = wave ? 4 : 32, n = (int64_t)nseg * M * NV;  // sums per workgroup
+  const dim3 grid((unsigned)std::min<int64_t>((n + per - 1) / per, 1 << 16));
+  if (wave)
+    hipLaunchKernelGGL((k_segsum_final<NV, 64>), grid, dim3(kBlock), 0, s, nseg, M, seg_chunk,
+                       partial, out);
+  else
+    hipLaunchKernelGGL((k_segsum_final<NV, 8>), grid, dim3(kBlock), 0, s, nseg, M, seg_chunk,
+                       partial, out);
   return hipGetLastError();
 }
 
@@ -163,19 +180,14 @@ hipError_t launch_segsum(hipStream_t s, int M, int nseg, int nchunks, const int2
     else
       hipLaunchKernelGGL((k_segsum_strided<R, 4>), g, dim3(kBlock), 0, s, M, chunks, spins, en,
                          partial);
-    hipLaunchKernelGGL(k_segsum_final<4>, dim3((nseg * M * 4 + 255) / 256), dim3(256), 0, s, nseg,
-                       M, seg_chunk, partial, out);
-  } else {
-    if (wide)
-      hipLaunchKernelGGL((k_segsum_wide<R, 3>), g, dim3(kBlock), 0, s, M, chunks, spins, en,
-                         partial);
-    else
-      hipLaunchKernelGGL((k_segsum_strided<R, 3>), g, dim3(kBlock), 0, s, M, chunks, spins, en,
-                         partial);
-    hipLaunchKernelGGL(k_segsum_final<3>, dim3((nseg * M * 3 + 255) / 256), dim3(256), 0, s, nseg,
-                       M, seg_chunk, partial, out);
+    return segsum_final<4>(s, nseg, M, nchunks, seg_chunk, partial, out);
   }
-  return hipGetLastError();
+  if (wide)
+    hipLaunchKernelGGL((k_segsum_wide<R, 3>), g, dim3(kBlock), 0, s, M, chunks, spins, en, partial);
+  else
+    hipLaunchKernelGGL((k_segsum_strided<R, 3>), g, dim3(kBlock), 0, s, M, chunks, spins, en,
+                       partial);
+  return segsum_final<3>(s, nseg, M, nchunks, seg_chunk, partial, out);
 }
 
 template <typename R>
@@ -185,9 +197,7 @@ hipError_t launch_energy_terms(hipStream_t s, const HamDev<R> &h, int nseg, int 
   if (nseg == 0 || h.M == 0 || nchunks == 0) return hipSuccess;
   hipLaunchKernelGGL((k_energy_terms<R>), dim3(nchunks, h.M), dim3(kBlock), 0, s, h, chunks,
                      spins, partial);
-  hipLaunchKernelGGL(k_segsum_final<4>, dim3((nseg * h.M * 4 + 255) / 256), dim3(256), 0, s,
-                     nseg, h.M, seg_chunk, partial, out);
-  return hipGetLastError();
+  return segsum_final<4>(s, nseg, h.M, nchunks, seg_chunk, partial, out);
 }
 
 #define UASD_INSTANTIATE(R)                                                                   \
