@@ -1,0 +1,41 @@
+"""Host arrays in and out of the device quads: site orders, ensembles, both
+precisions, and more (site, ensemble) pairs than one transfer takes at a time
+(2^22).  Directions and moments come back bit for bit: FP64 values unchanged,
+FP32 values rounded once."""
+import numpy as np
+import pytest
+
+import uppasd_amd as U
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("N,M,na", [(2, 1, 1), (6, 5, 3), (255, 2, 5), (65536, 65, 2), (4194305, 1, 1)])
+def test_moments_round_trip(N, M, na, precision):
+    rng = np.random.default_rng(N + M)
+    e = rng.normal(size=(M, N, 3))
+    mm = rng.uniform(0.5, 2.5, size=(M, N))
+    eng = U.Engine(N, M, precision, site_order=na)
+    eng.set_moments(e, mm)
+    if precision == "fp32":
+        e, mm = (a.astype(np.float32).astype(np.float64) for a in (e, mm))
+    got, gotM = eng.get_moments()
+    assert np.array_equal(got, e)
+    assert np.array_equal(gotM, e * mm[..., None])
+
+
+@pytest.mark.parametrize("N,M,na", [(6, 5, 3), (65536, 65, 2)])
+def test_field_of_host_moments(N, M, na):
+    rng = np.random.default_rng(N)
+    nl = (np.arange(N)[:, None] + 1) % N + 1           # one bond per site, J = 2
+    eng = U.Engine(N, M, site_order=na)
+    eng.set_exchange(nl.astype(np.int32), np.ones(N, np.int32), np.full((N, 1), 2.0))
+    ext = rng.normal(size=(M, N, 3))
+    eng.set_external_field(ext)
+    eng.set_moments(rng.normal(size=(M, N, 3)), np.ones((M, N)))
+    eM = rng.normal(size=(M, N, 3))
+    beff, _, b1, b2 = eng.effective_field(eM, parts=True)
+    assert np.array_equal(b1, 2.0 * np.roll(eM, -1, axis=1))
+    assert np.array_equal(b2, ext)
+    assert np.array_equal(beff, b1 + b2)

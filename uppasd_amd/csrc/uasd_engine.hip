@@ -155,6 +155,7 @@ struct uasd_ctx {
   DevBuf spins;   // quad arrays: e, p, b2
   DevBuf field;   // beff quads for the unfused path
   DevBuf scratch; // emomM quads (w = 1) for host field calls
+  DevBuf hostio;  // host arrays on their way in or out (upload_vec, download_vec)
   DevBuf noise;   // injected N(0,1) quads
   DevBuf nsave;   // fused steps: deviates drawn by the predictor for the corrector
   DevBuf llgarr;  // lambda, temp, lande (double, N each)
@@ -355,67 +356,132 @@ int upload_raw(uasd_ctx *c, DevBuf &dst, const std::vector<T> &src) {
   return UASD_OK;
 }
 
-// (3,N,M) Fortran array (+ w per (N,M) Fortran array, or a constant) -> quads
-// in device site order
-std::vector<double> to_quads(const uasd_ctx *c, const double *a, const double *w, double wconst) {
-  const int N = c->N, M = c->M;
-  std::vector<double> out((size_t)4 * N * M);
-  for (int k = 0; k < M; ++k)
-    for (int i = 0; i < N; ++i) {
-      const double *v = a + 3 * ((size_t)i + (size_t)N * k);
-      const size_t q = (size_t)slot_of(c, i) * M + k;
-      out[4 * q] = v[0];
-      out[4 * q + 1] = v[1];
-      out[4 * q + 2] = v[2];
-      out[4 * q + 3] = w ? w[(size_t)i + (size_t)N * k] : wconst;
-    }
-  return out;
+// Host (3,N,M) Fortran arrays cross as they are and are turned into quads, or
+// made from them, by a kernel: p = i + N*k is the pair of reference site i and
+// ensemble k, q its quad in device order.  A transfer's bound is then the copy
+// itself; the host threads convert nothing.  Arrays pass through a device
+// buffer of at most kIoPairs pairs, in stream order.  Against conversion on a
+// host thread with pageable quads in between: a step of the host-array halves
+// at 65,536 spins 2.13 -> 1.55 ms, moments of 4.1e6 pairs read back 95 -> 34 ms.
+constexpr size_t kIoPairs = (size_t)1 << 22;
+
+// the w of the quads an upload writes
+struct PackW {
+  const double *host = nullptr;  // an (N,M) Fortran array, or nullptr:
+  int from_state = 0;            // 1: the moment magnitudes of the state's quads
+  double value = 0.0;            // else this constant
+};
+
+// In device order, the quad of reference site i, ensemble k.
+struct PairMap {
+  int M, na, nc;
+  uasd::FastDiv ndiv;  // division by N
+  int N;
+  __device__ __forceinline__ size_t quad(size_t p) const {
+    const uint32_t k = uasd::fast_div((uint32_t)p, ndiv), i = (uint32_t)p - k * (uint32_t)N;
+    const uint32_t d = na == 1 ? i : (i % na) * (uint32_t)nc + i / na;
+    return (size_t)d * M + k;
+  }
+};
+
+// Pairs [p0, p0 + n) of a staged array a (and w) into their quads.  wsrc and
+// dst may be the same array: each thread reads and writes its own quad.
+template <typename R>
+__global__ void __launch_bounds__(256)
+    k_pack(PairMap m, size_t p0, size_t n, const double *__restrict__ a,
+           const double *__restrict__ w, const uasd::Quad<R> *wsrc, double wconst,
+           uasd::Quad<R> *dst) {
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const size_t q = m.quad(p0 + t);
+  dst[q] = uasd::Quad<R>{(R)a[3 * t], (R)a[3 * t + 1], (R)a[3 * t + 2],
+                         w ? (R)w[t] : wsrc ? wsrc[q].w : (R)wconst};
 }
 
-// upload host quads (double) into quad array k of buffer b (converted to R)
-int upload_quads(uasd_ctx *c, DevBuf &b, int k, const std::vector<double> &hq) {
+// The reverse: xyz, or xyz*w (emomM), of pairs [p0, p0 + n) in FP64.
+template <typename R>
+__global__ void __launch_bounds__(256)
+    k_unpack(PairMap m, size_t p0, size_t n, const uasd::Quad<R> *__restrict__ src, int times_w,
+             double *__restrict__ out) {
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const uasd::Quad<R> v = src[m.quad(p0 + t)];
+  const double w = times_w ? (double)v.w : 1.0;
+  out[3 * t] = (double)v.x * w;
+  out[3 * t + 1] = (double)v.y * w;
+  out[3 * t + 2] = (double)v.z * w;
+}
+
+PairMap pair_map(const uasd_ctx *c) {
+  return PairMap{c->M, c->order_na, c->order_na == 1 ? c->N : c->order_nc,
+                 uasd::make_fast_div((uint32_t)c->N), c->N};
+}
+
+// Host array a into quad array k of buffer b.  Asynchronous: a (and w.host)
+// must stay as they are until the stream has been waited for.
+int upload_vec(uasd_ctx *c, DevBuf &b, int k, const double *a, PackW w) {
   HIP_TRY(b.ensure(std::max(b.bytes, (size_t)(k + 1) * quad_bytes(c))));
-  if (c->prec == UASD_FP64) {
-    HIP_TRY(hipMemcpyAsync(quads<double>(c, b, k), hq.data(), hq.size() * 8,
-                           hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-  } else {
-    std::vector<float> f(hq.begin(), hq.end());
-    HIP_TRY(hipMemcpyAsync(quads<float>(c, b, k), f.data(), f.size() * 4, hipMemcpyHostToDevice,
+  const size_t total = (size_t)c->N * c->M, step = std::min(total, kIoPairs);
+  HIP_TRY(c->hostio.ensure(4 * step * sizeof(double)));
+  double *sa = c->hostio.as<double>(), *sw = w.host ? sa + 3 * step : nullptr;
+  for (size_t p0 = 0; p0 < total; p0 += step) {
+    const size_t n = std::min(step, total - p0);
+    HIP_TRY(hipMemcpyAsync(sa, a + 3 * p0, 3 * n * sizeof(double), hipMemcpyHostToDevice,
                            c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    if (sw)
+      HIP_TRY(hipMemcpyAsync(sw, w.host + p0, n * sizeof(double), hipMemcpyHostToDevice,
+                             c->stream));
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    if (c->prec == UASD_FP64)
+      hipLaunchKernelGGL(k_pack<double>, grid, block, 0, c->stream, pair_map(c), p0, n, sa, sw,
+                         w.from_state ? quads<double>(c, c->spins, 0) : nullptr, w.value,
+                         quads<double>(c, b, k));
+    else
+      hipLaunchKernelGGL(k_pack<float>, grid, block, 0, c->stream, pair_map(c), p0, n, sa, sw,
+                         w.from_state ? quads<float>(c, c->spins, 0) : nullptr, w.value,
+                         quads<float>(c, b, k));
+    HIP_TRY(hipGetLastError());
   }
   return UASD_OK;
 }
 
-int download_quads(uasd_ctx *c, const DevBuf &b, int k, std::vector<double> &hq) {
-  const size_t n = (size_t)4 * c->N * c->M;
-  if (c->prec == UASD_FP64) {
-    hq.resize(n);
-    HIP_TRY(hipMemcpyAsync(hq.data(), quads<double>(c, b, k), n * 8, hipMemcpyDeviceToHost,
+// Quad array k of buffer b into host array out (times_w: emomM = xyz*w).
+// Asynchronous: out is complete once the stream has been waited for.
+int download_vec(uasd_ctx *c, const DevBuf &b, int k, double *out, bool times_w) {
+  const size_t total = (size_t)c->N * c->M, step = std::min(total, kIoPairs);
+  HIP_TRY(c->hostio.ensure(4 * step * sizeof(double)));
+  double *so = c->hostio.as<double>();
+  for (size_t p0 = 0; p0 < total; p0 += step) {
+    const size_t n = std::min(step, total - p0);
+    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+    if (c->prec == UASD_FP64)
+      hipLaunchKernelGGL(k_unpack<double>, grid, block, 0, c->stream, pair_map(c), p0, n,
+                         quads<double>(c, b, k), times_w ? 1 : 0, so);
+    else
+      hipLaunchKernelGGL(k_unpack<float>, grid, block, 0, c->stream, pair_map(c), p0, n,
+                         quads<float>(c, b, k), times_w ? 1 : 0, so);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(out + 3 * p0, so, 3 * n * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-  } else {
-    std::vector<float> f(n);
-    HIP_TRY(hipMemcpyAsync(f.data(), quads<float>(c, b, k), n * 4, hipMemcpyDeviceToHost,
-                           c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    hq.assign(f.begin(), f.end());
   }
   return UASD_OK;
 }
 
-// quads (device site order) -> Fortran (3,N,M); times_w gives emomM = xyz*w
-void from_quads(const uasd_ctx *c, const std::vector<double> &hq, double *out, bool times_w) {
-  const int N = c->N, M = c->M;
-  for (int k = 0; k < M; ++k)
-    for (int i = 0; i < N; ++i) {
-      const size_t q = (size_t)slot_of(c, i) * M + k;
-      double *v = out + 3 * ((size_t)i + (size_t)N * k);
-      const double w = hq[4 * q + 3];
-      for (int d = 0; d < 3; ++d) v[d] = times_w ? hq[4 * q + d] * w : hq[4 * q + d];
-    }
-}
+// A call's host arrays are in transfer while this is open: wait() ends the
+// call, and a call that ends early waits before its caller gets them back.
+struct HostIo {
+  uasd_ctx *c;
+  bool open = true;
+  explicit HostIo(uasd_ctx *cc) : c(cc) {}
+  ~HostIo() {
+    if (open) (void)hipStreamSynchronize(c->stream);  // the call's own error is reported
+  }
+  int wait() {
+    open = false;
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    return UASD_OK;
+  }
+};
 
 // Whether every site's DM neighbours are its exchange neighbours, in the same
 // order and number, at most kFusedW of them (or there is no DM term): the
@@ -1320,7 +1386,9 @@ int uasd_set_external_field(uasd_ctx *c, const double *field) {
   }
   c->ext_mode = 2;
   if (int r = upload_real(c, c->ext_u, c->ext_u_host)) return r;
-  return upload_quads(c, c->ext_full, 0, to_quads(c, field, nullptr, 0.0));
+  HostIo io(c);
+  if (int r = upload_vec(c, c->ext_full, 0, field, PackW{})) return r;
+  return io.wait();
 }
 
 int uasd_set_llg(uasd_ctx *c, const double *lambda1, const double *temp, const double *landeg,
@@ -1371,7 +1439,9 @@ int uasd_set_noise(uasd_ctx *c, int mode, uint64_t seed, const double *normals) 
     return fail(UASD_ERR_ARG, "unknown noise mode");
   if (mode == UASD_NOISE_INJECTED) {
     if (!normals) return fail(UASD_ERR_ARG, "injected noise needs the normals array");
-    if (int r = upload_quads(c, c->noise, 0, to_quads(c, normals, nullptr, 0.0))) return r;
+    HostIo io(c);
+    if (int r = upload_vec(c, c->noise, 0, normals, PackW{})) return r;
+    if (int r = io.wait()) return r;
   }
   if (mode == UASD_NOISE_PHILOX && (seed != c->seed || c->noise_mode != mode)) c->step = 0;
   c->noise_mode = mode;
@@ -1382,9 +1452,12 @@ int uasd_set_noise(uasd_ctx *c, int mode, uint64_t seed, const double *normals) 
 int uasd_set_moments(uasd_ctx *c, const double *emom, const double *mmom) {
   if (int r = check_ctx(c)) return r;
   if (!emom || !mmom) return fail(UASD_ERR_ARG, "uasd_set_moments: null array");
-  std::vector<double> hq = to_quads(c, emom, mmom, 0.0);
-  if (int r = upload_quads(c, c->spins, 0, hq)) return r;
-  if (int r = upload_quads(c, c->spins, 1, hq)) return r;  // emom2 starts as emom
+  HostIo io(c);
+  if (int r = upload_vec(c, c->spins, 0, emom, PackW{mmom})) return r;
+  HIP_TRY(hipMemcpyAsync(static_cast<char *>(c->spins.p) + quad_bytes(c), c->spins.p,
+                         quad_bytes(c), hipMemcpyDeviceToDevice,
+                         c->stream));  // emom2 starts as emom
+  if (int r = io.wait()) return r;
   c->have_state = true;
   const size_t nm = (size_t)c->N * c->M;
   c->m_uniform = std::all_of(mmom, mmom + nm, [&](double v) { return v == mmom[0]; });
@@ -1396,47 +1469,22 @@ int uasd_set_moments(uasd_ctx *c, const double *emom, const double *mmom) {
 int uasd_get_moments(uasd_ctx *c, double *emom, double *emomM) {
   if (int r = check_ctx(c)) return r;
   if (!c->have_state) return fail(UASD_ERR_STATE, "moments not set");
-  std::vector<double> hq;
-  if (int r = download_quads(c, c->spins, 0, hq)) return r;
-  if (emom) from_quads(c, hq, emom, false);
-  if (emomM) from_quads(c, hq, emomM, true);
-  return UASD_OK;
+  HostIo io(c);
+  if (emom)
+    if (int r = download_vec(c, c->spins, 0, emom, false)) return r;
+  if (emomM)
+    if (int r = download_vec(c, c->spins, 0, emomM, true)) return r;
+  return io.wait();
 }
 
 // ---------------------------------------------------------- drop-in (host)
 // Host vec3 arrays are uploaded as quads; spin quads keep the resident mmom
 // in w, the others carry a constant.
-// dst[q] = (src[q].xyz, wsrc[q].w): uploaded directions merged with the
-// moment magnitudes already on the device
-extern "C++" {
-template <typename R>
-__global__ void __launch_bounds__(256)
-    k_merge_xyz(const uasd::Quad<R> *__restrict__ src, const uasd::Quad<R> *wsrc,
-                uasd::Quad<R> *dst, size_t n) {  // wsrc and dst may be the same array
-  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const uasd::Quad<R> v = src[q];
-  dst[q] = uasd::Quad<R>{v.x, v.y, v.z, wsrc[q].w};
-}
-}
 
 // quad array k of the spins <- the (3,N,M) array a, with w = mmom of the
-// state (quad array 0): a goes to the scratch quads, the merge runs on the
-// device, so the magnitudes are not read back to the host
+// state (quad array 0): the magnitudes stay on the device
 static int upload_vec_keep_w(uasd_ctx *c, int k, const double *a) {
-  if (int r = upload_quads(c, c->scratch, 0, to_quads(c, a, nullptr, 0.0))) return r;
-  const size_t n = (size_t)c->N * c->M;
-  const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-  if (c->prec == UASD_FP64)
-    hipLaunchKernelGGL(k_merge_xyz<double>, grid, block, 0, c->stream,
-                       quads<double>(c, c->scratch), quads<double>(c, c->spins, 0),
-                       quads<double>(c, c->spins, k), n);
-  else
-    hipLaunchKernelGGL(k_merge_xyz<float>, grid, block, 0, c->stream,
-                       quads<float>(c, c->scratch), quads<float>(c, c->spins, 0),
-                       quads<float>(c, c->spins, k), n);
-  HIP_TRY(hipGetLastError());
-  return UASD_OK;
+  return upload_vec(c, c->spins, k, a, PackW{nullptr, 1, 0.0});
 }
 
 int uasd_effective_field_host(uasd_ctx *c, const double *emomM, double *beff, double *beff1,
@@ -1445,22 +1493,15 @@ int uasd_effective_field_host(uasd_ctx *c, const double *emomM, double *beff, do
   if (!c->have_ex) return fail(UASD_ERR_STATE, "exchange not set");
   if (!emomM || !beff) return fail(UASD_ERR_ARG, "null array");
   if (int r = rebuild_classes(c)) return r;
-  if (int r = upload_quads(c, c->scratch, 0, to_quads(c, emomM, nullptr, 1.0))) return r;
+  HostIo io(c);
+  if (int r = upload_vec(c, c->scratch, 0, emomM, PackW{nullptr, 0, 1.0})) return r;
   const bool parts = beff1 || beff2;
   int r = c->prec == UASD_FP64 ? run_field<double>(c, true, energy != nullptr, parts)
                                : run_field<float>(c, true, energy != nullptr, parts);
   if (r) return r;
-  std::vector<double> hq;
-  if ((r = download_quads(c, c->field, 0, hq))) return r;
-  from_quads(c, hq, beff, false);
-  if (beff1) {
-    if ((r = download_quads(c, c->field, 1, hq))) return r;
-    from_quads(c, hq, beff1, false);
-  }
-  if (beff2) {
-    if ((r = download_quads(c, c->field, 2, hq))) return r;
-    from_quads(c, hq, beff2, false);
-  }
+  if ((r = download_vec(c, c->field, 0, beff, false))) return r;
+  if (beff1 && (r = download_vec(c, c->field, 1, beff1, false))) return r;
+  if (beff2 && (r = download_vec(c, c->field, 2, beff2, false))) return r;
   if (energy) {
     std::vector<double> red;
     r = c->prec == UASD_FP64 ? reduce_moments<double>(c, true, true, red)
@@ -1470,7 +1511,7 @@ int uasd_effective_field_host(uasd_ctx *c, const double *emomM, double *beff, do
     for (int k = 0; k < c->M; ++k) e += red[4 * (size_t)k + 3];
     *energy = e * uasd::kMub / uasd::kMry;
   }
-  return UASD_OK;
+  return io.wait();
 }
 
 int uasd_evolve_first_host(uasd_ctx *c, int alg, const double *beff, double *emom, double *emom2,
@@ -1481,37 +1522,31 @@ int uasd_evolve_first_host(uasd_ctx *c, int alg, const double *beff, double *emo
   if (!beff || !emom || !emom2 || !emomM || (sde_b2eff(alg) && !b2eff))
     return fail(UASD_ERR_ARG, "null array");
   if (int r = ready_for_llg(c)) return r;
-  if (int r = upload_quads(c, c->field, 0, to_quads(c, beff, nullptr, 0.0))) return r;
+  HostIo io(c);
+  if (int r = upload_vec(c, c->field, 0, beff, PackW{})) return r;
   // heun4p starts from emom2 (heun_proper.f90:309-311), the others from emom
   if (int r = upload_vec_keep_w(c, 0, alg == UASD_SDE_HEUN ? emom2 : emom)) return r;
   int r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 0, false, false)
                                : run_llg_half<float>(c, alg, 0, false, false);
   if (r) return r;
-  std::vector<double> pq;
-  if ((r = download_quads(c, c->spins, 1, pq))) return r;
   if (alg == UASD_SDE_DEPONDT) {
     // depondt.f90:182-187: emom2 = m(t), emom = rotated, emomM = emom*mmom, b2eff = bdup
+    if ((r = io.wait())) return r;  // emom has been read before it is written
     std::memcpy(emom2, emom, sizeof(double) * 3 * (size_t)c->N * c->M);
-    from_quads(c, pq, emom, false);
-    from_quads(c, pq, emomM, true);
-    std::vector<double> bq;
-    if ((r = download_quads(c, c->spins, 2, bq))) return r;
-    from_quads(c, bq, b2eff, false);
+    if ((r = download_vec(c, c->spins, 1, emom, false))) return r;
+    if ((r = download_vec(c, c->spins, 2, b2eff, false))) return r;
   } else if (alg == UASD_SDE_HEUN) {
     // heun_proper.f90:303-365: b2eff = beff, emom = predictor, emomM =
     // emom*mmom, emom2 unchanged
-    from_quads(c, pq, emom, false);
-    from_quads(c, pq, emomM, true);
-    std::vector<double> bq;
-    if ((r = download_quads(c, c->spins, 2, bq))) return r;
-    from_quads(c, bq, b2eff, false);
+    if ((r = download_vec(c, c->spins, 1, emom, false))) return r;
+    if ((r = download_vec(c, c->spins, 2, b2eff, false))) return r;
   } else {
     // midpoint.f90:167-175 (and sibt / sispht, sphmidpoint.f90:247-258,
     // 698-710): emom2 = et', emomM = et'*mmom, emom unchanged
-    from_quads(c, pq, emom2, false);
-    from_quads(c, pq, emomM, true);
+    if ((r = download_vec(c, c->spins, 1, emom2, false))) return r;
   }
-  return UASD_OK;
+  if ((r = download_vec(c, c->spins, 1, emomM, true))) return r;
+  return io.wait();
 }
 
 int uasd_evolve_second_host(uasd_ctx *c, int alg, const double *beff, const double *b2eff,
@@ -1522,12 +1557,13 @@ int uasd_evolve_second_host(uasd_ctx *c, int alg, const double *beff, const doub
   if (!beff || !emom || !emom2 || (sde_b2eff(alg) && !b2eff))
     return fail(UASD_ERR_ARG, "null array");
   if (int r = ready_for_llg(c)) return r;
-  if (int r = upload_quads(c, c->field, 0, to_quads(c, beff, nullptr, 0.0))) return r;
+  HostIo io(c);
+  if (int r = upload_vec(c, c->field, 0, beff, PackW{})) return r;
   if (alg == UASD_SDE_DEPONDT || alg == UASD_SDE_HEUN) {
     // reference on entry: emom = predicted, emom2 = m(t)
     if (int r = upload_vec_keep_w(c, 1, emom)) return r;
     if (int r = upload_vec_keep_w(c, 0, emom2)) return r;
-    if (int r = upload_quads(c, c->spins, 2, to_quads(c, b2eff, nullptr, 0.0))) return r;
+    if (int r = upload_vec(c, c->spins, 2, b2eff, PackW{})) return r;
   } else {
     if (int r = upload_vec_keep_w(c, 0, emom)) return r;
     if (int r = upload_vec_keep_w(c, 1, emom2)) return r;
@@ -1535,10 +1571,12 @@ int uasd_evolve_second_host(uasd_ctx *c, int alg, const double *beff, const doub
   int r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 1, false, false)
                                : run_llg_half<float>(c, alg, 1, false, false);
   if (r) return r;
-  if (alg == UASD_SDE_DEPONDT) std::memcpy(emom, emom2, sizeof(double) * 3 * (size_t)c->N * c->M);
-  std::vector<double> pq;
-  if ((r = download_quads(c, c->spins, 1, pq))) return r;
-  from_quads(c, pq, emom2, false);
+  if (alg == UASD_SDE_DEPONDT) {
+    if ((r = io.wait())) return r;  // both have been read before they are written
+    std::memcpy(emom, emom2, sizeof(double) * 3 * (size_t)c->N * c->M);
+  }
+  if ((r = download_vec(c, c->spins, 1, emom2, false))) return r;
+  if ((r = io.wait())) return r;
   c->step += 1;
   return UASD_OK;
 }
@@ -1682,14 +1720,12 @@ int uasd_effective_field(uasd_ctx *c, double *beff, double *energy) {
   if (int r = check_ctx(c)) return r;
   if (!c->have_ex || !c->have_state) return fail(UASD_ERR_STATE, "exchange or moments not set");
   if (int r = rebuild_classes(c)) return r;
-  int r = c->prec == UASD_FP64 ? run_field<double>(c, false, energy != nullptr)
-                               : run_field<float>(c, false, energy != nullptr);
+  int r = c->prec == UASD_FP64
+              ? run_field<double>(c, false, energy != nullptr, false, beff != nullptr)
+              : run_field<float>(c, false, energy != nullptr, false, beff != nullptr);
   if (r) return r;
-  if (beff) {
-    std::vector<double> hq;
-    if ((r = download_quads(c, c->field, 0, hq))) return r;
-    from_quads(c, hq, beff, false);
-  }
+  HostIo io(c);
+  if (beff && (r = download_vec(c, c->field, 0, beff, false))) return r;
   if (energy) {
     std::vector<double> red;
     r = c->prec == UASD_FP64 ? reduce_moments<double>(c, true, false, red)
@@ -1699,8 +1735,7 @@ int uasd_effective_field(uasd_ctx *c, double *beff, double *energy) {
     for (int k = 0; k < c->M; ++k) e += red[4 * (size_t)k + 3];
     *energy = e * uasd::kMub / uasd::kMry;
   }
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return UASD_OK;
+  return io.wait();
 }
 
 // Uploads the per-ensemble MC constants and the colour lists and fills mp.
