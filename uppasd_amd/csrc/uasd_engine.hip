@@ -230,6 +230,18 @@ struct uasd_ctx {
   std::vector<int> color_start, color_stride;
   bool coloring_dirty = true;
 
+  // the independent systems of the lattice and their tables for the resident
+  // MC kernel (built with the first MC call after a Hamiltonian change)
+  struct Resident {
+    bool ok = false;
+    int ncomp = 0, nmax = 0;
+    DevBuf buf;
+    uasd::ResDev dev{};
+    int64_t cls_version = -1;
+    int64_t col_version = -1;
+  } res;
+  int64_t col_version = 0;  // bumped by every colouring rebuild
+
   // Per-kernel timing: an event pair is recorded around each launch without
   // a host wait; pairs are resolved when the totals are read.
   bool timing = false;
@@ -843,6 +855,7 @@ int build_coloring(uasd_ctx *c) {
     c->color_stride[k] = ap ? d : 0;
   }
   c->coloring_dirty = false;
+  c->col_version += 1;
   c->gen += 1;
   return UASD_OK;
 }
@@ -1738,6 +1751,108 @@ int uasd_effective_field(uasd_ctx *c, double *beff, double *energy) {
   return io.wait();
 }
 
+// Contiguous ranges of device slots that no bond crosses, as first slots.
+static std::vector<int> independent_ranges(const uasd_ctx *c) {
+  const int N = c->N;
+  std::vector<int> reach(N);  // furthest slot bonded to slot i or to one before it
+  auto add = [&](const std::vector<int> &row, const std::vector<int> &len,
+                 const std::vector<int> &nb, int W) {
+    if (W == 0 || row.empty()) return;
+    for (int j = 0; j < W; ++j)
+      for (int i = 0; i < N; ++i)
+        if (j < len[row[i]]) {
+          const int n = nb[(size_t)j * N + i];
+          reach[std::min(i, n)] = std::max(reach[std::min(i, n)], std::max(i, n));
+        }
+  };
+  for (int i = 0; i < N; ++i) reach[i] = i;
+  add(c->ex_row_of_site, c->ex_len_host, c->nbr_host, c->W);
+  add(c->dm_row_of_site, c->dm_len_host, c->dnbr_host, c->Wd);
+  std::vector<int> off(1, 0);
+  for (int i = 0, far = 0; i < N; ++i) {
+    far = std::max(far, reach[i]);
+    if (far == i) off.push_back(i + 1);
+  }
+  return off;
+}
+
+// Builds c->res for the current lists, classes and colouring.
+static int build_resident(uasd_ctx *c) {
+  auto &r = c->res;
+  if (r.cls_version == c->cls_version && r.col_version == c->col_version) return UASD_OK;
+  r.ok = false;
+  r.cls_version = c->cls_version;
+  r.col_version = c->col_version;
+  const int N = c->N, ncol = c->ncolors;
+  const std::vector<int> off = independent_ranges(c);
+  const int ncomp = (int)off.size() - 1;
+  int nmax = 0;
+  for (int k = 0; k < ncomp; ++k) nmax = std::max(nmax, off[k + 1] - off[k]);
+  if (uasd::res_lds_spins(c->rsize, nmax) > (size_t)c->lds_max || nmax > 65536) return UASD_OK;
+  std::vector<int> ptr((size_t)ncomp * (ncol + 1)), pos(N);
+  std::vector<int> site(N);
+  int cmax = 1;
+  for (int k = 0; k < ncomp; ++k) {
+    int *pc = ptr.data() + (size_t)k * (ncol + 1);
+    for (int i = off[k]; i < off[k + 1]; ++i) pc[c->color_of_site[i] + 1]++;
+    for (int q = 1; q <= ncol; ++q) {
+      cmax = std::max(cmax, pc[q]);
+      pc[q] += pc[q - 1];
+    }
+    std::vector<int> at(pc, pc + ncol);
+    for (int i = off[k]; i < off[k + 1]; ++i) {
+      pos[i] = at[c->color_of_site[i]]++;
+      site[off[k] + pos[i]] = i;
+    }
+  }
+  const int W = c->W, Wd = c->Wd;
+  std::vector<uint16_t> nb((size_t)(W + Wd) * N);
+  auto fill = [&](const std::vector<int> &list, int w, uint16_t *out) {
+    for (int k = 0; k < ncomp; ++k)
+      for (int p = off[k]; p < off[k + 1]; ++p)
+        for (int j = 0; j < w; ++j) out[(size_t)j * N + p] = (uint16_t)pos[list[(size_t)j * N + site[p]]];
+  };
+  fill(c->nbr_host, W, nb.data());
+  fill(c->dnbr_host, Wd, nb.data() + (size_t)W * N);
+  std::vector<uasd::SiteClass> cls(N);
+  for (int p = 0; p < N; ++p) {
+    const int i = site[p];
+    cls[p] = uasd::SiteClass{c->ex_row_of_site.empty() ? 0 : c->ex_row_of_site[i],
+                             c->dm_row_of_site.empty() ? -1 : c->dm_row_of_site[i],
+                             c->an_row_of_site.empty() ? -1 : c->an_row_of_site[i], 0};
+  }
+  // one allocation: classes, offsets, colour pointers, sites, lists
+  std::vector<char> all;
+  auto put = [&](const void *p, size_t n) {
+    const size_t at = all.size();
+    all.resize(at + (n + 15) / 16 * 16);
+    std::memcpy(all.data() + at, p, n);
+    return at;
+  };
+  const size_t ocls = put(cls.data(), cls.size() * sizeof(cls[0])),
+               ooff = put(off.data(), off.size() * sizeof(int)),
+               optr = put(ptr.data(), ptr.size() * sizeof(int)),
+               osite = put(site.data(), site.size() * sizeof(int)),
+               onb = put(nb.data(), nb.size() * sizeof(uint16_t));
+  if (int e = upload_raw(c, r.buf, all)) return e;
+  const char *base = r.buf.as<char>();
+  r.dev = uasd::ResDev{ncomp,
+                       ncol,
+                       nmax,
+                       cmax,
+                       reinterpret_cast<const int *>(base + ooff),
+                       reinterpret_cast<const int *>(base + optr),
+                       reinterpret_cast<const int *>(base + osite),
+                       reinterpret_cast<const uasd::SiteClass *>(base + ocls),
+                       reinterpret_cast<const uint16_t *>(base + onb),
+                       reinterpret_cast<const uint16_t *>(base + onb) + (size_t)W * N};
+  r.ncomp = ncomp;
+  r.nmax = nmax;
+  r.ok = true;
+  c->gen += 1;  // captured sweeps hold the old tables
+  return UASD_OK;
+}
+
 // Uploads the per-ensemble MC constants and the colour lists and fills mp.
 static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed,
                       uasd::MCParams &mp) {
@@ -1748,6 +1863,7 @@ static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed
     return fail(UASD_ERR_UNSUPPORTED, "MC takes a uniform external field (as mc_evolve's extfield)");
   if (int r = rebuild_classes(c)) return r;
   if (int r = build_coloring(c)) return r;
+  if (int r = build_resident(c)) return r;
   const int M = c->M;
   for (int k = 0; k < M; ++k)
     if (!(temps[k] > 0.0)) return fail(UASD_ERR_ARG, "MC temperatures must be > 0");
@@ -1780,9 +1896,55 @@ static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed
   return UASD_OK;
 }
 
+// Whether the sweeps run in k_mc_resident: systems that fit in LDS, whose
+// colours hold no more sites on average than its workgroup has threads, and
+// few enough updates per colour that a launch of them is mostly launch.
+//  - Sites per colour: a colour costs 1.4-2.2 us (14 neighbours) against 5-7
+//    us for its launch; with more sites than threads the one CU needs longer
+//    for a phase than the whole chip for a launch.  Per sweep, launches ->
+//    resident, 14 neighbours: 432 sites FP64 54 -> 18 us (FP32 40 -> 13), 2000
+//    sites 63 -> 27 (44 -> 17), heat bath 57 -> 26, 4394 sites (10 colours,
+//    439 sites each) 77 -> 47.
+//  - Updates per colour: 2^18 of them take the launch path 6-17 us.  At 228k
+//    (1024 ensembles of 2000 sites, 9 colours) 158 -> 113 us a sweep, at 262k
+//    (alloy pairs of 1024 sites, 256 ensembles, 2 colours) 29 -> 21 us; at
+//    600k (64 alloys, 32 ensembles) 54 -> 61 us, slower.
+static bool mc_use_resident(const uasd_ctx *c) {
+  return c->res.ok && c->res.nmax <= uasd::kResThreads * c->ncolors &&
+         (int64_t)c->N * c->M <= (int64_t)c->ncolors << 18;
+}
+
+// nsweeps sweeps in resident launches of at most kResSweeps, from mp.sweep on.
+// The predicted moments (quad array 1), which every LLG step writes before it
+// reads them, lend their memory to the trial moves.
+static int mc_resident(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
+  constexpr int64_t kResSweeps = 1024;
+  for (int64_t s = 0; s < nsweeps; s += kResSweeps) {
+    const int n = (int)std::min(kResSweeps, nsweeps - s);
+    tic(c, 3);
+    if (c->prec == UASD_FP64)
+      HIP_TRY(uasd::launch_mc_resident<double>(c->stream, ham_view<double>(c), mp, c->res.dev, n,
+                                               (size_t)c->lds_max, quads<double>(c, c->spins, 0),
+                                               quads<double>(c, c->spins, 1)));
+    else
+      HIP_TRY(uasd::launch_mc_resident<float>(c->stream, ham_view<float>(c), mp, c->res.dev, n,
+                                              (size_t)c->lds_max, quads<float>(c, c->spins, 0),
+                                               quads<float>(c, c->spins, 1)));
+    if (int r = toc(c, 3)) return r;
+    mp.sweep += (uint64_t)n;
+  }
+  return UASD_OK;
+}
+
 // nsweeps colour-ordered sweeps; every launch is asynchronous on the stream.
 static int mc_run(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
   const int *sites_dev = mp.sites;
+  if (mc_use_resident(c)) {
+    mp.sweep = c->mc_sweep;
+    if (int r = mc_resident(c, mp, nsweeps)) return r;
+    c->mc_sweep += (uint64_t)nsweeps;
+    return UASD_OK;
+  }
   for (int64_t s = 0; s < nsweeps; ++s) {
     mp.sweep = c->mc_sweep;
     for (int col = 0; col < c->ncolors; ++col) {
@@ -1827,7 +1989,12 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
     auto body = [&]() -> int {
       uasd::MCParams g = mp;
       g.sweep_dev = c->ctr.as<uint64_t>() + 1;
-      for (int j = 0; j < K; ++j) {
+      const bool resident = mc_use_resident(c);
+      if (resident) {
+        g.sweep = 0;
+        if (int r = mc_resident(c, g, K)) return r;
+      }
+      for (int j = 0; j < K && !resident; ++j) {
         g.sweep = (uint64_t)j;
         for (int col = 0; col < c->ncolors; ++col) {
           g.sites = mp.sites + c->color_ptr[col];

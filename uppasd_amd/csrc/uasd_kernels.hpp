@@ -390,6 +390,13 @@ struct NbDec1 {
   }
 };
 
+// Lists whose entries are the gather index itself (the resident MC kernel).
+struct NbDecId {
+  template <typename R>
+  __device__ __forceinline__ NbDecId(const HamDev<R> &, int) {}
+  __device__ __forceinline__ int operator()(uint16_t v) const { return v; }
+};
+
 template <bool NT, typename I>
 __device__ __forceinline__ I nb_load(const I *p) {
   if constexpr (NT) return __builtin_nontemporal_load(p);
@@ -521,12 +528,12 @@ __device__ __forceinline__ void exchange_sum(const HamDev<R> &h, const I *__rest
 }
 
 // DM sum of site_field: field += m_j x D_ij (hamiltonianactions.f90:565-578).
-template <typename R, int G, typename I>
+template <typename R, int G, typename I, typename D = NbDec>
 __device__ __forceinline__ void dm_sum(const HamDev<R> &h, const I *__restrict__ nb,
                                        const Quad<R> *__restrict__ src, int site, int ens,
                                        int row, R &s0, R &s1, R &s2) {
   const int M = h.M, N = h.N;
-  const NbDec dec(h, site);
+  const D dec(h, site);
   const int len = h.dm_len[row];
   const size_t rs = (size_t)h.dm_rows;
   for (int j = 0; j < len; j += G) {
@@ -693,6 +700,32 @@ __device__ __forceinline__ void site_field(const HamDev<R> &h, const Quad<R> *__
   }
 }
 
+// The anisotropy field of the moment at quad q, added to s (uniaxial, cubic)
+// and qf (type 7's cubic part times sb) as site_field adds it.
+template <typename R>
+__device__ __forceinline__ void anisotropy(const HamDev<R> &h, const SiteClass &sc,
+                                           const Quad<R> *__restrict__ src, size_t q, R (&s)[3],
+                                           R (&qf)[3]) {
+  if (sc.an_row < 0) return;
+  const int t = h.an_type[sc.an_row];
+  if (t != 1 && t != 2 && t != 7) return;
+  R m0, m1, m2;
+  moment(src, q, m0, m1, m2);
+  if (t == 1) {
+    uniaxial(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
+  } else if (t == 2) {
+    cubic(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
+  } else {
+    R t0 = 0, t1 = 0, t2 = 0;
+    uniaxial(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
+    cubic(h, sc.an_row, m0, m1, m2, t0, t1, t2);
+    const R sb = h.an_sb[sc.an_row];
+    qf[0] = qf[0] + t0 * sb;
+    qf[1] = qf[1] + t1 * sb;
+    qf[2] = qf[2] + t2 * sb;
+  }
+}
+
 // The pair, DM and anisotropy parts of site_field for the U adjacent
 // ensembles e0 .. e0+U-1 of one site: the exchange terms of all U from one
 // read of the neighbour entries and couplings, then each ensemble's DM and
@@ -727,26 +760,7 @@ __device__ __forceinline__ void site_field_u(const HamDev<R> &h, const Quad<R> *
         dm_sum<R, G>(h, h.dnbr + site, src, site, e0 + k, sc.dm_row, sf[k][0], sf[k][1],
                      sf[k][2]);
     }
-    if (sc.an_row >= 0) {
-      const int t = h.an_type[sc.an_row];
-      if (t == 1 || t == 2 || t == 7) {
-        R m0, m1, m2;
-        moment(src, (size_t)site * M + e0 + k, m0, m1, m2);
-        if (t == 1) {
-          uniaxial(h, sc.an_row, m0, m1, m2, sf[k][0], sf[k][1], sf[k][2]);
-        } else if (t == 2) {
-          cubic(h, sc.an_row, m0, m1, m2, sf[k][0], sf[k][1], sf[k][2]);
-        } else {
-          R t0 = 0, t1 = 0, t2 = 0;
-          uniaxial(h, sc.an_row, m0, m1, m2, sf[k][0], sf[k][1], sf[k][2]);
-          cubic(h, sc.an_row, m0, m1, m2, t0, t1, t2);
-          const R sb = h.an_sb[sc.an_row];
-          qf[k][0] = qf[k][0] + t0 * sb;
-          qf[k][1] = qf[k][1] + t1 * sb;
-          qf[k][2] = qf[k][2] + t2 * sb;
-        }
-      }
-    }
+    anisotropy(h, sc, src, (size_t)site * M + e0 + k, sf[k], qf[k]);
   }
 }
 
@@ -1648,41 +1662,57 @@ __global__ void __launch_bounds__(1024)
 }
 
 // ----------------------------------------------------------------- MC
-// choose_random_flip (montecarlo_common.f90:25-79)
+// choose_random_flip (montecarlo_common.f90:25-79): a uniform direction, a
+// Gaussian step or the reversed moment, chosen by floor(3 u0).
+template <typename R>
+__device__ __forceinline__ void trial_uniform(double u1, double u2, R &n0, R &n1, R &n2) {
+  // phi = 2 pi u1, theta = acos(1 - 2 u2) (montecarlo_common.f90:55-59):
+  // cos(theta) = z and sin(theta) = sqrt(1 - z^2) >= 0 on [0, pi], and
+  // sincospi(2 u1) is sin and cos of phi, all equal to the library forms to
+  // rounding without the acos, sin and cos of theta
+  const double z = 1 - 2 * u2;
+  const double st = sqrt(fmax(0.0, 1 - z * z));
+  double sp, cp;
+  sincospi(2 * u1, &sp, &cp);
+  n0 = (R)(st * cp);
+  n1 = (R)(st * sp);
+  n2 = (R)z;
+}
+
+template <typename R>
+__device__ __forceinline__ void trial_gauss(R e0, R e1, R e2, double delta, double g0, double g1,
+                                           double g2, R &n0, R &n1, R &n2) {
+  R a0 = e0 + (R)(g0 * delta), a1 = e1 + (R)(g1 * delta), a2 = e2 + (R)(g2 * delta);
+  // one reciprocal for the three divisions by the length (equal to rounding)
+  const R il = (R)1 / fsqrt(a0 * a0 + a1 * a1 + a2 * a2);
+  n0 = a0 * il;
+  n1 = a1 * il;
+  n2 = a2 * il;
+}
+
+// Spin flip, newmom = -emom.  Written as a subtraction: hipcc (clang 22,
+// -O1 and above) drops a bare negation of a loaded value when it merges
+// the three branches of trial_move, turning every flip into a no-op.
+// 0 - e equals -e except that a +0 component stays +0, which changes no
+// energy or later arithmetic.
+template <typename R>
+__device__ __forceinline__ void trial_flip(R e0, R e1, R e2, R &n0, R &n1, R &n2) {
+  n0 = (R)0 - e0;
+  n1 = (R)0 - e1;
+  n2 = (R)0 - e2;
+}
+
 template <typename R>
 __device__ __forceinline__ void trial_move(R e0, R e1, R e2, double delta, double u0, double u1,
                                           double u2, double g0, double g1, double g2, R &n0,
                                           R &n1, R &n2) {
   const int ftype = (int)floor(3 * u0);
-  if (ftype == 0) {
-    // phi = 2 pi u1, theta = acos(1 - 2 u2) (montecarlo_common.f90:55-59):
-    // cos(theta) = z and sin(theta) = sqrt(1 - z^2) >= 0 on [0, pi], and
-    // sincospi(2 u1) is sin and cos of phi, all equal to the library forms to
-    // rounding without the acos, sin and cos of theta
-    const double z = 1 - 2 * u2;
-    const double st = sqrt(fmax(0.0, 1 - z * z));
-    double sp, cp;
-    sincospi(2 * u1, &sp, &cp);
-    n0 = (R)(st * cp);
-    n1 = (R)(st * sp);
-    n2 = (R)z;
-  } else if (ftype == 1) {
-    R a0 = e0 + (R)(g0 * delta), a1 = e1 + (R)(g1 * delta), a2 = e2 + (R)(g2 * delta);
-    // one reciprocal for the three divisions by the length (equal to rounding)
-    const R il = (R)1 / fsqrt(a0 * a0 + a1 * a1 + a2 * a2);
-    n0 = a0 * il;
-    n1 = a1 * il;
-    n2 = a2 * il;
-  } else {
-    // Spin flip, newmom = -emom.  Written as a subtraction: hipcc (clang 22,
-    // -O1 and above) drops a bare negation of a loaded value when it merges
-    // the three branches of this function, turning every flip into a no-op.
-    // 0 - e equals -e except that a +0 component stays +0, which changes no
-    // energy or later arithmetic.
-    n0 = (R)0 - e0;
-    n1 = (R)0 - e1;
-    n2 = (R)0 - e2;
-  }
+  if (ftype == 0)
+    trial_uniform(u1, u2, n0, n1, n2);
+  else if (ftype == 1)
+    trial_gauss(e0, e1, e2, delta, g0, g1, g2, n0, n1, n2);
+  else
+    trial_flip(e0, e1, e2, n0, n1, n2);
 }
 
 template <typename R>
@@ -1690,37 +1720,19 @@ __device__ __forceinline__ R sq(R x) {
   return x * x;
 }
 
-// calculate_energy (montecarlo_common.f90:431-865), exchange + anisotropy +
-// DM + external field, for the U adjacent ensembles e0 .. e0+U-1 of one site:
-// de[k] = mub*(E_trial - E_current) of ensemble e0+k, whose current moment is
-// me[k], trial direction tr[k] and uniform field x[k].  The site's class, its
-// neighbour entries and its couplings are read once for the U ensembles.
-template <typename R, int G, int U>
-__device__ __forceinline__ void mc_delta_e(const HamDev<R> &h, const Quad<R> *__restrict__ s,
-                                           int site, int e0, const Quad<R> (&me)[U],
-                                           const R (&tr)[U][3], const R (&x)[U][3],
-                                           R (&de)[U]) {
-  const SiteClass sc = h.classes[h.cls[site]];
-  const int M = h.M, N = h.N;
-  // The exchange energy of the current and the trial moment, -sum_j J_j
-  // m.m_j (montecarlo_common.f90:512-520), is formed as -m.f with the
-  // exchange field f = sum_j J_j m_j of site_field: the same quantity with a
-  // third of the arithmetic, equal to the term-by-term sums to rounding.
-  R f[U][3];
-#pragma unroll
-  for (int k = 0; k < U; ++k) f[k][0] = f[k][1] = f[k][2] = (R)0;
-  const int row = sc.ex_row;
-  if (h.nbr16) {
-    if (h.nt)
-      mc_exchange_fields<R, G, true, int16_t, U>(h, h.nbr16 + site, s, site, e0, row, f);
-    else
-      mc_exchange_fields<R, G, false, int16_t, U>(h, h.nbr16 + site, s, site, e0, row, f);
-  } else {
-    if (h.nt)
-      mc_exchange_fields<R, G, true, int, U>(h, h.nbr + site, s, site, e0, row, f);
-    else
-      mc_exchange_fields<R, G, false, int, U>(h, h.nbr + site, s, site, e0, row, f);
-  }
+// The energy difference of calculate_energy (montecarlo_common.f90:431-865)
+// once the exchange fields f of the U ensembles are known: exchange,
+// anisotropy, DM (nbf(j) = the site's j-th DM neighbour) and external field; de[k] = mub*(E_trial - E_current).  The exchange energy of the
+// current and the trial moment, -sum_j J_j m.m_j (512-520), is formed as -m.f
+// with the exchange field f = sum_j J_j m_j of site_field: the same quantity
+// with a third of the arithmetic, equal to the term-by-term sums to rounding.
+template <typename R, int U, typename F>
+__device__ __forceinline__ void mc_energy_diff(const HamDev<R> &h, const SiteClass &sc,
+                                               const Quad<R> *__restrict__ s, int e0, F &&nbf,
+                                               const R (&f)[U][3], const Quad<R> (&me)[U],
+                                               const R (&tr)[U][3], const R (&x)[U][3],
+                                               R (&de)[U]) {
+  const int M = h.M;
   R c0[U], c1[U], c2[U], t0[U], t1[U], t2[U], e_c[U], e_t[U];
 #pragma unroll
   for (int k = 0; k < U; ++k) {
@@ -1764,8 +1776,7 @@ __device__ __forceinline__ void mc_delta_e(const HamDev<R> &h, const Quad<R> *__
   if (h.Wd > 0 && sc.dm_row >= 0) {
     const int len = h.dm_len[sc.dm_row];
     for (int j = 0; j < len; ++j) {
-      const int nb = h.dnbr16 ? NbDec(h, site)(h.dnbr16[(size_t)j * N + site])
-                              : h.dnbr[(size_t)j * N + site];
+      const int nb = nbf(j);
       const size_t r = (size_t)j * h.dm_rows + sc.dm_row;
       const R D0 = h.dvx[r], D1 = h.dvy[r], D2 = h.dvz[r];
 #pragma unroll
@@ -1788,6 +1799,42 @@ __device__ __forceinline__ void mc_delta_e(const HamDev<R> &h, const Quad<R> *__
     const R tt = e_t[k] - e_c[k];
     de[k] = (R)kMub * tt;
   }
+}
+
+// calculate_energy (montecarlo_common.f90:431-865), exchange + anisotropy +
+// DM + external field, for the U adjacent ensembles e0 .. e0+U-1 of one site:
+// de[k] = mub*(E_trial - E_current) of ensemble e0+k, whose current moment is
+// me[k], trial direction tr[k] and uniform field x[k].  The site's class, its
+// neighbour entries and its couplings are read once for the U ensembles.
+template <typename R, int G, int U>
+__device__ __forceinline__ void mc_delta_e(const HamDev<R> &h, const Quad<R> *__restrict__ s,
+                                           int site, int e0, const Quad<R> (&me)[U],
+                                           const R (&tr)[U][3], const R (&x)[U][3],
+                                           R (&de)[U]) {
+  const SiteClass sc = h.classes[h.cls[site]];
+  R f[U][3];
+#pragma unroll
+  for (int k = 0; k < U; ++k) f[k][0] = f[k][1] = f[k][2] = (R)0;
+  const int row = sc.ex_row;
+  if (h.nbr16) {
+    if (h.nt)
+      mc_exchange_fields<R, G, true, int16_t, U>(h, h.nbr16 + site, s, site, e0, row, f);
+    else
+      mc_exchange_fields<R, G, false, int16_t, U>(h, h.nbr16 + site, s, site, e0, row, f);
+  } else {
+    if (h.nt)
+      mc_exchange_fields<R, G, true, int, U>(h, h.nbr + site, s, site, e0, row, f);
+    else
+      mc_exchange_fields<R, G, false, int, U>(h, h.nbr + site, s, site, e0, row, f);
+  }
+  const int N = h.N;
+  mc_energy_diff<R, U>(
+      h, sc, s, e0,
+      [&](int j) {
+        return h.dnbr16 ? NbDec(h, site)(h.dnbr16[(size_t)j * N + site])
+                        : h.dnbr[(size_t)j * N + site];
+      },
+      f, me, tr, x, de);
 }
 
 // flip_h (montecarlo_common.f90:371-422)
@@ -1881,6 +1928,31 @@ __device__ __forceinline__ void trial_f32(const MCParams &mp, uint64_t sweep, ui
   }
 }
 
+// The Metropolis trial direction tr and acceptance uniform of one (site,
+// ensemble): hs is the site's reference index, me its current moment.
+template <typename R>
+__device__ __forceinline__ void metropolis_trial(const MCParams &mp, uint64_t sweep, uint32_t hs,
+                                                 int ens, const Quad<R> &me, R (&tr)[3],
+                                                 R &acc) {
+  if constexpr (std::is_same<R, float>::value) {
+    trial_f32(mp, sweep, hs, ens, me.x, me.y, me.z, tr[0], tr[1], tr[2], acc);
+  } else {
+    double u0, u1, u2, u3;
+    uniform4(mp.seed, kTagMCU, sweep, hs, (uint32_t)ens, u0, u1, u2, u3);
+    double g0 = 0.0, g1 = 0.0, g2 = 0.0;
+    if ((int)floor(3 * u0) == 1) normal3_f64(mp.seed, kTagMCG, sweep, hs, (uint32_t)ens, g0, g1, g2);
+    trial_move<R>(me.x, me.y, me.z, mp.delta[ens], u0, u1, u2, g0, g1, g2, tr[0], tr[1], tr[2]);
+    acc = u3;
+  }
+}
+
+template <typename R>
+__device__ __forceinline__ bool metropolis_take(double beta, R de, R acc) {
+  if (std::is_same<R, float>::value)
+    return de <= (R)0 || (float)acc < expf(-(float)beta * (float)de);
+  return de <= (R)0 || acc < exp(-beta * (double)de);
+}
+
 // One colour of a sweep.  HB selects heat bath (mp.heat_bath) or Metropolis
 // at compile time, so each mode's registers are allocated for its own code
 // alone.  A thread updates the U adjacent ensembles e0 .. e0+U-1 of one site
@@ -1932,43 +2004,210 @@ __global__ void __launch_bounds__(256) k_mc_colour(HamDev<R> h, MCParams mp, Qua
       s[q0 + k] = Quad<R>{o0, o1, o2, me[k].w};
     }
   } else {
-    R tr[U][3];
-    double acc[U];
+    R tr[U][3], acc[U];
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int ens = e0 + k;
-      if (std::is_same<R, float>::value) {
-        float n0, n1, n2, a;
-        trial_f32(mp, sweep, hs, ens, (float)me[k].x, (float)me[k].y, (float)me[k].z, n0, n1, n2,
-                  a);
-        tr[k][0] = (R)n0;
-        tr[k][1] = (R)n1;
-        tr[k][2] = (R)n2;
-        acc[k] = a;
-      } else {
-        double u0, u1, u2, u3;
-        uniform4(mp.seed, kTagMCU, sweep, hs, (uint32_t)ens, u0, u1, u2, u3);
-        double g0 = 0.0, g1 = 0.0, g2 = 0.0;
-        if ((int)floor(3 * u0) == 1)
-          normal3_f64(mp.seed, kTagMCG, sweep, hs, (uint32_t)ens, g0, g1, g2);
-        trial_move<R>(me[k].x, me[k].y, me[k].z, mp.delta[ens], u0, u1, u2, g0, g1, g2, tr[k][0],
-                      tr[k][1], tr[k][2]);
-        acc[k] = u3;
-      }
-    }
+    for (int k = 0; k < U; ++k) metropolis_trial<R>(mp, sweep, hs, e0 + k, me[k], tr[k], acc[k]);
     R de[U];
     mc_delta_e<R, G, U>(h, (const Quad<R> *)s, site, e0, me, tr, x, de);
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const int ens = e0 + k;
-      bool take;
-      if (std::is_same<R, float>::value)
-        take = de[k] <= (R)0 || (float)acc[k] < expf(-(float)mp.beta[ens] * (float)de[k]);
-      else
-        take = de[k] <= (R)0 || acc[k] < exp(-mp.beta[ens] * (double)de[k]);
-      if (take) s[q0 + k] = Quad<R>{tr[k][0], tr[k][1], tr[k][2], me[k].w};
+    for (int k = 0; k < U; ++k)
+      if (metropolis_take<R>(mp.beta[e0 + k], de[k], acc[k]))
+        s[q0 + k] = Quad<R>{tr[k][0], tr[k][1], tr[k][2], me[k].w};
+  }
+}
+
+// ------------------------------------------------- resident MC of small systems
+// A system is one independent part of the lattice (no bond leaves it) in one
+// ensemble.  A small one is swept by one workgroup with its spins in LDS, all
+// the sweeps of a call in one launch: the colours of a sweep then cost a
+// barrier each instead of a launch each, which is what a small system's sweep
+// consists of (a launch of a few hundred updates takes 6-7 us, the updates
+// themselves a fraction of one).
+//
+// The spins lie in LDS in colour order (position p; the sites of a colour are
+// adjacent), so the waves of a phase are full.  The neighbour lists hold
+// positions, 16 bits each, and sit in LDS where they fit beside the spins.
+// The Metropolis trial moves of a whole sweep depend on a site's own moment
+// alone: they are made before its first colour by all waves at once (into LDS,
+// TRL, or into a global buffer), so a phase is the field gather and the
+// acceptance only.  In FP64 the sites are first sorted by their move: a wave
+// whose lanes chose freely would run the arithmetic of all three moves.  Every
+// update is arithmetically the one of k_mc_colour, from the same counters.
+//
+// What bounds it: instruction issue of the one CU for the trials, and for the
+// phases the latency of their chain (class, couplings, LDS gather, exp).
+struct ResDev {
+  int ncomp, ncol;                      // systems per ensemble, colours
+  int nmax, cmax;                       // sites of the largest system, of the largest phase
+  const int *__restrict__ off;          // (ncomp+1) first position of each system
+  const int *__restrict__ ptr;          // (ncomp, ncol+1) positions of its colours, local
+  const int *__restrict__ site;         // (N) device slot at each position
+  const SiteClass *__restrict__ cls;    // (N) class at each position
+  const uint16_t *__restrict__ nbr;     // (W, N) local positions of the neighbours
+  const uint16_t *__restrict__ dnbr;    // (Wd, N)
+};
+
+constexpr int kResThreads = 512;
+
+// Appends v to a list in LDS at *count (one atomic per wavefront).
+__device__ __forceinline__ void lds_append(bool on, uint16_t v, uint16_t *list, int *count,
+                                           int dir) {
+  const uint64_t m = __ballot(on);
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  if (m != 0 && lane == __ffsll((unsigned long long)m) - 1) base = atomicAdd(count, __popcll(m));
+  base = __shfl(base, m ? __ffsll((unsigned long long)m) - 1 : 0, 64);
+  if (on) list[dir * (base + __popcll(m & (((uint64_t)1 << lane) - 1)))] = v;
+}
+
+// The trial moves of sweep `sweep` at every position.  list: n entries of LDS
+// for the sorted positions (FP64), uniform moves from its front, Gaussian
+// steps from its back; count: two counters in LDS.
+template <typename R, typename T>
+__device__ __forceinline__ void resident_trials(const HamDev<R> &h, const MCParams &mp,
+                                                const ResDev &rd, uint64_t sweep, int off, int n,
+                                                int ens, const Quad<R> *sp, T *tr,
+                                                uint16_t *list, int *count) {
+  const int tid = threadIdx.x, nt = blockDim.x;
+  if constexpr (std::is_same<R, float>::value) {
+    for (int p = tid; p < n; p += nt) {
+      R d[3], acc;
+      metropolis_trial<R>(mp, sweep, host_site(h, rd.site[off + p]), ens, sp[p], d, acc);
+      tr[p] = Quad<R>{d[0], d[1], d[2], acc};
+    }
+  } else {
+    if (tid < 2) count[tid] = 0;
+    __syncthreads();
+    for (int p0 = 0; p0 < n; p0 += nt) {  // every lane takes part in the appends
+      const int p = p0 + tid;
+      int ftype = -1;
+      if (p < n) {
+        const uint32_t hs = host_site(h, rd.site[off + p]);
+        double u0, u1, u2, u3;
+        uniform4(mp.seed, kTagMCU, sweep, hs, (uint32_t)ens, u0, u1, u2, u3);
+        ftype = (int)floor(3 * u0);
+        Quad<R> t{u1, u2, (R)hs, u3};  // what the move still needs
+        if (ftype != 0 && ftype != 1) {
+          const Quad<R> e = sp[p];
+          trial_flip(e.x, e.y, e.z, t.x, t.y, t.z);
+        }
+        tr[p] = t;
+      }
+      lds_append(ftype == 0, (uint16_t)p, list, count, 1);
+      lds_append(ftype == 1, (uint16_t)p, list + (n - 1), count + 1, -1);
+    }
+    __syncthreads();
+    const int nu = count[0], ng = count[1];
+    for (int i = nt - 1 - tid; i < ng; i += nt) {  // from the last wave on
+      const int p = list[n - 1 - i];
+      const Quad<R> t = tr[p], e = sp[p];
+      double g0, g1, g2;
+      normal3_f64(mp.seed, kTagMCG, sweep, (uint32_t)t.z, (uint32_t)ens, g0, g1, g2);
+      Quad<R> o;
+      o.w = t.w;
+      trial_gauss(e.x, e.y, e.z, mp.delta[ens], g0, g1, g2, o.x, o.y, o.z);
+      tr[p] = o;
+    }
+    for (int i = tid; i < nu; i += nt) {
+      const int p = list[i];
+      const Quad<R> t = tr[p];
+      Quad<R> o;
+      o.w = t.w;
+      trial_uniform(t.x, t.y, o.x, o.y, o.z);
+      tr[p] = o;
     }
   }
+}
+
+// trg: (M, N) trials in global memory, used where they do not fit in LDS.
+template <typename R, bool HB, bool TRL, bool LNB>
+__global__ void __launch_bounds__(kResThreads, !HB && sizeof(R) == 4 ? 4 : 2)
+    k_mc_resident(HamDev<R> h, MCParams mp, ResDev rd, int nsweeps, Quad<R> *s, Quad<R> *trg) {
+  constexpr int G = 4;  // LDS gathers: eight in flight cost registers and gain nothing
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_res[];
+  __shared__ int count[2];
+  Quad<R> *sp = reinterpret_cast<Quad<R> *>(lds_res);
+  Quad<R> *trl = sp + rd.nmax;
+  uint16_t *list = reinterpret_cast<uint16_t *>(sp + (TRL ? 2 : 1) * rd.nmax);  // FP64 Metropolis
+  uint16_t *lnb = list + (!HB && sizeof(R) == 8 ? rd.nmax : 0);
+  const int M = h.M, W = h.W, Wd = h.Wd, N = h.N;
+  const int comp = blockIdx.x / M, ens = blockIdx.x - comp * M;
+  const int off = rd.off[comp], n = rd.off[comp + 1] - off;
+  const int *ptr = rd.ptr + (size_t)comp * (rd.ncol + 1);
+  const int tid = threadIdx.x, T = blockDim.x;
+  trg += (size_t)ens * N + off;
+  for (int p = tid; p < n; p += T) sp[p] = s[(size_t)rd.site[off + p] * M + ens];
+  if (LNB) {
+    for (int j = 0; j < W; ++j)
+      for (int p = tid; p < n; p += T) lnb[j * n + p] = rd.nbr[(size_t)j * N + off + p];
+    for (int j = 0; j < Wd; ++j)
+      for (int p = tid; p < n; p += T) lnb[(W + j) * n + p] = rd.dnbr[(size_t)j * N + off + p];
+  }
+  // the lists as the gathers see them: one ensemble, stride lh.N
+  HamDev<R> lh = h;
+  lh.M = 1;
+  lh.N = LNB ? n : N;
+  const uint16_t *nb = LNB ? lnb : rd.nbr + off;
+  const uint16_t *dnb = LNB ? lnb + W * n : rd.dnbr + off;
+  const R x[1][3] = {{(R)mp.ext[3 * ens], (R)mp.ext[3 * ens + 1], (R)mp.ext[3 * ens + 2]}};
+  const double beta = HB ? mp.hbeta[ens] : mp.beta[ens];
+  const uint64_t sweep0 = mp.sweep_dev ? *mp.sweep_dev + mp.sweep : mp.sweep;
+  __syncthreads();
+  for (int k = 0; k < nsweeps; ++k) {
+    const uint64_t sweep = sweep0 + (uint64_t)k;
+    if (!HB) {
+      if (TRL)
+        resident_trials<R>(h, mp, rd, sweep, off, n, ens, sp, trl, list, count);
+      else
+        resident_trials<R>(h, mp, rd, sweep, off, n, ens, sp, trg, list, count);
+      __syncthreads();
+    }
+    // the class of this thread's first position of the next colour is loaded
+    // before the barrier that ends the current one
+    SiteClass first = tid < ptr[1] ? rd.cls[off + tid] : SiteClass{0, 0, 0, 0};
+    for (int c = 0; c < rd.ncol; ++c) {
+      const int p0 = ptr[c] + tid, p1 = ptr[c + 1];
+      const int pn = p1 + tid;
+      const SiteClass mine = first;
+      if (c + 1 < rd.ncol && pn < ptr[c + 2]) first = rd.cls[off + pn];
+      for (int p = p0; p < p1; p += T) {
+        const SiteClass sc = p == p0 ? mine : rd.cls[off + p];
+        const Quad<R> me[1] = {sp[p]};
+        const int len = h.ex_full ? W : h.ex_len[sc.ex_row];
+        if constexpr (HB) {
+          R f[1][3] = {{(R)0, (R)0, (R)0}}, qf[3] = {(R)0, (R)0, (R)0};
+          exchange_run<R, G, false, uint16_t, 1, false, NbDecId>(lh, nb + p, sp, p, 0, sc.ex_row,
+                                                                 len, f);
+          if (Wd > 0 && sc.dm_row >= 0)
+            dm_sum<R, G, uint16_t, NbDecId>(lh, dnb + p, sp, p, 0, sc.dm_row, f[0][0], f[0][1],
+                                            f[0][2]);
+          anisotropy(h, sc, (const Quad<R> *)sp, (size_t)p, f[0], qf);
+          double u0, u1, u2, u3;
+          uniform4(mp.seed, kTagMCU, sweep, host_site(h, rd.site[off + p]), (uint32_t)ens, u0, u1,
+                   u2, u3);
+          const R f0 = (R)0 + f[0][0] + (qf[0] + x[0][0] + (R)0);
+          const R f1 = (R)0 + f[0][1] + (qf[1] + x[0][1] + (R)0);
+          const R f2 = (R)0 + f[0][2] + (qf[2] + x[0][2] + (R)0);
+          R o0, o1, o2;
+          heat_bath<R>(beta, me[0].w, f0, f1, f2, u1, u0, o0, o1, o2);
+          sp[p] = Quad<R>{o0, o1, o2, me[0].w};
+        } else {
+          const Quad<R> t = TRL ? trl[p] : trg[p];
+          const R d[1][3] = {{t.x, t.y, t.z}};
+          R f[1][3] = {{(R)0, (R)0, (R)0}}, de[1];
+          exchange_run<R, G, false, uint16_t, 1, true, NbDecId>(lh, nb + p, sp, p, 0, sc.ex_row,
+                                                                len, f);
+          mc_energy_diff<R, 1>(
+              lh, sc, (const Quad<R> *)sp, 0, [&](int j) { return (int)dnb[j * lh.N + p]; }, f, me,
+              d, x, de);
+          if (metropolis_take<R>(beta, de[0], t.w))
+            sp[p] = Quad<R>{d[0][0], d[0][1], d[0][2], me[0].w};
+        }
+      }
+      __syncthreads();
+    }
+  }
+  for (int p = tid; p < n; p += T) s[(size_t)rd.site[off + p] * M + ens] = sp[p];
 }
 
 // ---------------------------------------------------------- FP64 reductions

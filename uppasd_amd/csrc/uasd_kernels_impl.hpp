@@ -116,6 +116,52 @@ hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCP
   });
 }
 
+template <typename R, bool HB, bool TRL, bool LNB>
+static hipError_t mc_resident_one(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
+                                  const ResDev &rd, int nsweeps, size_t bytes, int threads,
+                                  Quad<R> *spins, Quad<R> *trials) {
+  const void *kern = (const void *)&k_mc_resident<R, HB, TRL, LNB>;
+  // dynamic LDS above 64 KiB must be requested
+  const hipError_t err =
+      hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((k_mc_resident<R, HB, TRL, LNB>), dim3((unsigned)(rd.ncomp * h.M)),
+                     dim3(threads), bytes, s, h, mp, rd, nsweeps, spins, trials);
+  return hipGetLastError();
+}
+
+template <typename R>
+hipError_t launch_mc_resident(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
+                              const ResDev &rd, int nsweeps, size_t lds, Quad<R> *spins,
+                              Quad<R> *trials) {
+  const size_t sp = res_lds_spins(sizeof(R), rd.nmax), lists = res_lds_lists(rd.nmax, h.W + h.Wd);
+  const size_t tr = 4 * sizeof(R) * (size_t)rd.nmax;
+  if (sp > lds || nsweeps <= 0) return hipErrorInvalidValue;
+  // A phase needs a thread per site of its colour.  Only the trial moves of a
+  // sweep can use more, and only while the chip has CUs to spare (256 of
+  // them): with more systems than that the waves are better spent on other
+  // workgroups (1024 heat-bath systems of 432 sites: 83 -> 30 us a sweep).
+  const bool wide = !mp.heat_bath && (int64_t)rd.ncomp * h.M <= 512;
+  const int threads = std::min(kResThreads, ((wide ? rd.nmax : rd.cmax) + 63) / 64 * 64);
+  // the trials of a sweep in LDS where they fit, then the lists
+  const bool trl = !mp.heat_bath && sp + tr <= lds;
+  const size_t base = sp + (trl ? tr : 0);
+  const bool lnb = base + lists <= lds;
+  const size_t bytes = base - 16 + (lnb ? lists : 0);  // the counters are static
+#define UASD_RES_CASE(HB_, TRL_, LNB_)                                                          \
+  if ((mp.heat_bath != 0) == HB_ && trl == TRL_ && lnb == LNB_)                                 \
+    return mc_resident_one<R, HB_, TRL_, LNB_>(s, h, mp, rd, nsweeps, bytes, threads, spins,    \
+                                               trials);
+  UASD_RES_CASE(true, false, true)
+  UASD_RES_CASE(true, false, false)
+  UASD_RES_CASE(false, true, true)
+  UASD_RES_CASE(false, true, false)
+  UASD_RES_CASE(false, false, true)
+  UASD_RES_CASE(false, false, false)
+#undef UASD_RES_CASE
+  return hipErrorInvalidValue;
+}
+
 template <typename R>
 hipError_t launch_llg_tile(hipStream_t s, TileDev t, int pipe, int alg, int half,
                            const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e,
@@ -208,6 +254,8 @@ hipError_t launch_energy_terms(hipStream_t s, const HamDev<R> &h, int nseg, int 
                                     Quad<R> *, Quad<R> *, const Quad<R> *, Quad<R> *);        \
   template hipError_t launch_mc<R>(hipStream_t, const Tune &, const HamDev<R> &,              \
                                    const MCParams &, Quad<R> *);                              \
+  template hipError_t launch_mc_resident<R>(hipStream_t, const HamDev<R> &, const MCParams &,  \
+                                            const ResDev &, int, size_t, Quad<R> *, Quad<R> *); \
   template hipError_t launch_llg_tile<R>(hipStream_t, TileDev, int, int, int,              \
                                          const HamDev<R> &, const LLGDev<R> &,                \
                                          const Quad<R> *, Quad<R> *, Quad<R> *, Quad<R> *);   \

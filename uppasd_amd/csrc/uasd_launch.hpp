@@ -72,6 +72,21 @@ template <typename R>
 hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
                      Quad<R> *spins);
 
+// nsweeps sweeps of every system with k_mc_resident; lds = LDS bytes a
+// workgroup may use, trials = N*M quads of scratch for the trial moves that do
+// not fit in them (not read before they are written).
+template <typename R>
+hipError_t launch_mc_resident(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
+                              const ResDev &rd, int nsweeps, size_t lds, Quad<R> *spins,
+                              Quad<R> *trials);
+
+// LDS of k_mc_resident with nmax sites: what it cannot do without (the spins,
+// the sorted positions and two counters), and w list entries per site.
+inline size_t res_lds_lists(int nmax, int w) { return sizeof(uint16_t) * (size_t)nmax * w; }
+inline size_t res_lds_spins(size_t rsize, int nmax) {
+  return 4 * rsize * (size_t)nmax + res_lds_lists(nmax, rsize == 8 ? 1 : 0) + 16;
+}
+
 // Fused LLG half-step with the LDS-tiled stencil kernel, work units (tile,
 // ensemble).
 template <typename R>
