@@ -1,5 +1,6 @@
 """Host arrays in and out of the device quads: site orders, ensembles, both
-precisions, and more (site, ensemble) pairs than one transfer takes at a time
+precisions, the most pairs that pass through pinned memory (16,384) and one
+more, and more (site, ensemble) pairs than one transfer takes at a time
 (2^22).  Directions and moments come back bit for bit: FP64 values unchanged,
 FP32 values rounded once."""
 import numpy as np
@@ -11,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
-@pytest.mark.parametrize("N,M,na", [(2, 1, 1), (6, 5, 3), (255, 2, 5), (65536, 65, 2), (4194305, 1, 1)])
+@pytest.mark.parametrize("N,M,na", [(2, 1, 1), (6, 5, 3), (255, 2, 5), (16384, 1, 1),
+                                    (16385, 1, 5), (65536, 65, 2), (4194305, 1, 1)])
 def test_moments_round_trip(N, M, na, precision):
     rng = np.random.default_rng(N + M)
     e = rng.normal(size=(M, N, 3))

@@ -88,6 +88,17 @@ hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fuse
 }
 
 template <typename R>
+hipError_t launch_draw(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
+                       Quad<R> *out) {
+  const int64_t n = (int64_t)h.N * h.M;
+  if (n == 0 || steps <= 0) return hipSuccess;
+  const int block = n <= 64 * 256 ? 64 : kBlock;
+  hipLaunchKernelGGL((k_draw<R>), dim3((unsigned)((n + block - 1) / block), (unsigned)steps),
+                     dim3(block), 0, s, h, prm, steps, out);
+  return hipGetLastError();
+}
+
+template <typename R>
 hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
                      Quad<R> *spins) {
   const int64_t n = (int64_t)mp.nsites * h.M;
@@ -252,6 +263,8 @@ hipError_t launch_energy_terms(hipStream_t s, const HamDev<R> &h, int nseg, int 
   template hipError_t launch_llg<R>(hipStream_t, const Tune &, int, int, bool,                \
                                     const HamDev<R> &, const LLGDev<R> &, const Quad<R> *,    \
                                     Quad<R> *, Quad<R> *, const Quad<R> *, Quad<R> *);        \
+  template hipError_t launch_draw<R>(hipStream_t, const HamDev<R> &, const LLGDev<R> &, int,   \
+                                     Quad<R> *);                                              \
   template hipError_t launch_mc<R>(hipStream_t, const Tune &, const HamDev<R> &,              \
                                    const MCParams &, Quad<R> *);                              \
   template hipError_t launch_mc_resident<R>(hipStream_t, const HamDev<R> &, const MCParams &,  \

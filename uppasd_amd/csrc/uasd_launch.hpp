@@ -35,7 +35,25 @@ struct Tune {
   int tile = 0;
   int pipe = 0;  // tile kernel: 1 = resident workgroups loop over several tiles
   int pair = 0;  // MC colour pass: 1 = two adjacent ensembles per thread (M even)
+  int chosen = 0;  // 1: set by the caller or found by the autotuner, 0: default_tune applies
 };
+
+// Launch shape of a gathering kernel that nobody has tuned: n items (sites x
+// ensembles of a launch), w neighbours.  A small launch is a chain of loads on
+// a chip that is mostly idle: workgroups of one wavefront spread it over the
+// most CUs and their caches, and with many neighbours eight gathers in flight
+// halve the number of rounds.  LLG step at 58 neighbours, (4, 256) -> (8, 64):
+// 16,000 sites FP64 24.4 -> 16.9 us, 65,536 sites 26.3 -> 24.2 us; 14
+// neighbours -> (4, 64): 16,000 sites 13.5 -> 12.2 us, 65,536 sites equal.  MC
+// sweep of 15,840 sites at 58 neighbours 338 -> 180 us.  From 2^18 items on
+// the shapes are within a few per cent of each other.
+inline Tune default_tune(const Tune &t, int64_t n, int w) {
+  if (t.chosen || n > (int64_t)1 << 18) return t;
+  Tune d = t;
+  d.block = 64;
+  d.gather = w >= 16 ? 8 : 4;
+  return d;
+}
 
 inline bool tune_valid(const Tune &t) {
   return (t.gather == 2 || t.gather == 4 || t.gather == 8 || t.gather == 16) &&
@@ -67,6 +85,11 @@ template <typename R>
 hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fused,
                       const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p,
                       Quad<R> *b2, const Quad<R> *beff, Quad<R> *out);
+
+// Deviates of `steps` steps from prm.step on into as many quad arrays of out.
+template <typename R>
+hipError_t launch_draw(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
+                       Quad<R> *out);
 
 template <typename R>
 hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
