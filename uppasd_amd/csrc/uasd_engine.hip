@@ -65,6 +65,28 @@ struct DevBuf {
   T *as() const { return static_cast<T *>(p); }
 };
 
+// Owned pinned host memory, which kernels read and write in place.
+struct PinBuf {
+  void *p = nullptr;
+  size_t bytes = 0;
+  PinBuf() = default;
+  PinBuf(const PinBuf &) = delete;
+  PinBuf &operator=(const PinBuf &) = delete;
+  ~PinBuf() {
+    if (p) (void)hipHostFree(p);  // teardown: no caller to report to
+  }
+  hipError_t ensure(size_t n) {
+    if (n <= bytes) return hipSuccess;
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+    bytes = 0;
+    const hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
+    if (e == hipSuccess) bytes = n;
+    else p = nullptr;
+    return e;
+  }
+};
+
 // Hash of a byte string (FNV-1a) for deduplicating rows.
 struct RowKey {
   std::string bytes;
@@ -156,6 +178,8 @@ struct uasd_ctx {
   DevBuf field;   // beff quads for the unfused path
   DevBuf scratch; // emomM quads (w = 1) for host field calls
   DevBuf hostio;  // host arrays on their way in or out (upload_vec, download_vec)
+  PinBuf pinio;   // the same for small arrays
+  PinBuf pinsum;  // final sums of a few (segment, ensemble) pairs
   DevBuf noise;   // injected N(0,1) quads
   DevBuf nsave;   // fused steps: deviates drawn by the predictor for the corrector
   DevBuf llgarr;  // lambda, temp, lande (double, N each)
@@ -221,6 +245,9 @@ struct uasd_ctx {
     hipGraphExec_t exec = nullptr;
   };
   std::map<std::tuple<int, int, int, uint64_t>, Graph> graphs;  // kind, alg/mode, K, seed
+  // steps or sweeps launched one by one under unchanged settings (see
+  // repeats_pay): kind, alg/mode, seed -> gen, count
+  std::map<std::tuple<int, int, uint64_t>, std::pair<uint64_t, int64_t>> repeats;
 
   // colouring
   int ncolors = 0;
@@ -267,6 +294,7 @@ namespace {
 
 void destroy_graphs(uasd_ctx *c);
 int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps);
+int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph);
 int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nsweeps,
                   uint64_t seed);
 
@@ -379,9 +407,8 @@ constexpr size_t kIoPairs = (size_t)1 << 22;
 
 // the w of the quads an upload writes
 struct PackW {
-  const double *host = nullptr;  // an (N,M) Fortran array, or nullptr:
-  int from_state = 0;            // 1: the moment magnitudes of the state's quads
-  double value = 0.0;            // else this constant
+  int from_state = 0;  // 1: the moment magnitudes of the state's quads
+  double value = 0.0;  // else this constant
 };
 
 // In device order, the quad of reference site i, ensemble k.
@@ -429,71 +456,121 @@ PairMap pair_map(const uasd_ctx *c) {
                  uasd::make_fast_div((uint32_t)c->N), c->N};
 }
 
-// Host array a into quad array k of buffer b.  Asynchronous: a (and w.host)
-// must stay as they are until the stream has been waited for.
-int upload_vec(uasd_ctx *c, DevBuf &b, int k, const double *a, PackW w) {
+// The host arrays of one call.  Large ones are copied through the context's
+// device buffer.  Small ones (kPinPairs) go through pinned memory that the
+// kernels read and write in place: a copy command of a few kilobytes costs
+// more than the conversion kernel it would feed.  wait() ends the call's
+// transfers; a call that ends early waits before its caller gets the arrays
+// back.
+struct HostIo {
+  static constexpr size_t kPinPairs = 16384, kPinArrays = 8;
+  uasd_ctx *c;
+  bool open = false;
+  size_t used = 0;  // doubles of c->pinio in use
+  struct Out {
+    double *to;
+    const double *from;
+    size_t n;
+  };
+  std::vector<Out> outs;
+  explicit HostIo(uasd_ctx *cc) : c(cc) {}
+  ~HostIo() {
+    if (open) (void)hipStreamSynchronize(c->stream);  // the call's own error is reported
+  }
+  bool small() const { return (size_t)c->N * c->M <= kPinPairs; }
+  // n doubles of pinned memory that stay untouched until wait()
+  int pinned(size_t n, double **p) {
+    HIP_TRY(c->pinio.ensure(kPinArrays * 3 * (size_t)c->N * c->M * sizeof(double)));
+    if ((used + n) * sizeof(double) > c->pinio.bytes)
+      return fail(UASD_ERR_STATE, "pinned staging exhausted");
+    *p = static_cast<double *>(c->pinio.p) + used;
+    used += n;
+    return UASD_OK;
+  }
+  int wait() {
+    open = false;
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    for (const Out &o : outs) std::memcpy(o.to, o.from, o.n * sizeof(double));
+    outs.clear();
+    used = 0;
+    return UASD_OK;
+  }
+};
+
+int launch_pack(uasd_ctx *c, DevBuf &b, int k, size_t p0, size_t n, const double *a,
+                const double *w, const PackW &pw) {
+  const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+  if (c->prec == UASD_FP64)
+    hipLaunchKernelGGL(k_pack<double>, grid, block, 0, c->stream, pair_map(c), p0, n, a, w,
+                       pw.from_state ? quads<double>(c, c->spins, 0) : nullptr, pw.value,
+                       quads<double>(c, b, k));
+  else
+    hipLaunchKernelGGL(k_pack<float>, grid, block, 0, c->stream, pair_map(c), p0, n, a, w,
+                       pw.from_state ? quads<float>(c, c->spins, 0) : nullptr, pw.value,
+                       quads<float>(c, b, k));
+  HIP_TRY(hipGetLastError());
+  return UASD_OK;
+}
+
+int launch_unpack(uasd_ctx *c, const DevBuf &b, int k, size_t p0, size_t n, bool times_w,
+                  double *out) {
+  const dim3 grid((unsigned)((n + 255) / 256)), block(256);
+  if (c->prec == UASD_FP64)
+    hipLaunchKernelGGL(k_unpack<double>, grid, block, 0, c->stream, pair_map(c), p0, n,
+                       quads<double>(c, b, k), times_w ? 1 : 0, out);
+  else
+    hipLaunchKernelGGL(k_unpack<float>, grid, block, 0, c->stream, pair_map(c), p0, n,
+                       quads<float>(c, b, k), times_w ? 1 : 0, out);
+  HIP_TRY(hipGetLastError());
+  return UASD_OK;
+}
+
+// Host array a into quad array k of buffer b.  Asynchronous: a must stay as it
+// is until io.wait().
+int upload_vec(HostIo &io, DevBuf &b, int k, const double *a, PackW w) {
+  uasd_ctx *c = io.c;
   HIP_TRY(b.ensure(std::max(b.bytes, (size_t)(k + 1) * quad_bytes(c))));
   const size_t total = (size_t)c->N * c->M, step = std::min(total, kIoPairs);
-  HIP_TRY(c->hostio.ensure(4 * step * sizeof(double)));
-  double *sa = c->hostio.as<double>(), *sw = w.host ? sa + 3 * step : nullptr;
+  io.open = true;
+  if (io.small()) {
+    double *sa = nullptr;
+    if (int r = io.pinned(3 * total, &sa)) return r;
+    std::memcpy(sa, a, 3 * total * sizeof(double));
+    return launch_pack(c, b, k, 0, total, sa, nullptr, w);
+  }
+  HIP_TRY(c->hostio.ensure(3 * step * sizeof(double)));
+  double *sa = c->hostio.as<double>();
   for (size_t p0 = 0; p0 < total; p0 += step) {
     const size_t n = std::min(step, total - p0);
     HIP_TRY(hipMemcpyAsync(sa, a + 3 * p0, 3 * n * sizeof(double), hipMemcpyHostToDevice,
                            c->stream));
-    if (sw)
-      HIP_TRY(hipMemcpyAsync(sw, w.host + p0, n * sizeof(double), hipMemcpyHostToDevice,
-                             c->stream));
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    if (c->prec == UASD_FP64)
-      hipLaunchKernelGGL(k_pack<double>, grid, block, 0, c->stream, pair_map(c), p0, n, sa, sw,
-                         w.from_state ? quads<double>(c, c->spins, 0) : nullptr, w.value,
-                         quads<double>(c, b, k));
-    else
-      hipLaunchKernelGGL(k_pack<float>, grid, block, 0, c->stream, pair_map(c), p0, n, sa, sw,
-                         w.from_state ? quads<float>(c, c->spins, 0) : nullptr, w.value,
-                         quads<float>(c, b, k));
-    HIP_TRY(hipGetLastError());
+    if (int r = launch_pack(c, b, k, p0, n, sa, nullptr, w)) return r;
   }
   return UASD_OK;
 }
 
 // Quad array k of buffer b into host array out (times_w: emomM = xyz*w).
-// Asynchronous: out is complete once the stream has been waited for.
-int download_vec(uasd_ctx *c, const DevBuf &b, int k, double *out, bool times_w) {
+// Asynchronous: out is complete after io.wait().
+int download_vec(HostIo &io, const DevBuf &b, int k, double *out, bool times_w) {
+  uasd_ctx *c = io.c;
   const size_t total = (size_t)c->N * c->M, step = std::min(total, kIoPairs);
-  HIP_TRY(c->hostio.ensure(4 * step * sizeof(double)));
+  io.open = true;
+  if (io.small()) {
+    double *so = nullptr;
+    if (int r = io.pinned(3 * total, &so)) return r;
+    io.outs.push_back({out, so, 3 * total});
+    return launch_unpack(c, b, k, 0, total, times_w, so);
+  }
+  HIP_TRY(c->hostio.ensure(3 * step * sizeof(double)));
   double *so = c->hostio.as<double>();
   for (size_t p0 = 0; p0 < total; p0 += step) {
     const size_t n = std::min(step, total - p0);
-    const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-    if (c->prec == UASD_FP64)
-      hipLaunchKernelGGL(k_unpack<double>, grid, block, 0, c->stream, pair_map(c), p0, n,
-                         quads<double>(c, b, k), times_w ? 1 : 0, so);
-    else
-      hipLaunchKernelGGL(k_unpack<float>, grid, block, 0, c->stream, pair_map(c), p0, n,
-                         quads<float>(c, b, k), times_w ? 1 : 0, so);
-    HIP_TRY(hipGetLastError());
+    if (int r = launch_unpack(c, b, k, p0, n, times_w, so)) return r;
     HIP_TRY(hipMemcpyAsync(out + 3 * p0, so, 3 * n * sizeof(double), hipMemcpyDeviceToHost,
                            c->stream));
   }
   return UASD_OK;
 }
-
-// A call's host arrays are in transfer while this is open: wait() ends the
-// call, and a call that ends early waits before its caller gets them back.
-struct HostIo {
-  uasd_ctx *c;
-  bool open = true;
-  explicit HostIo(uasd_ctx *cc) : c(cc) {}
-  ~HostIo() {
-    if (open) (void)hipStreamSynchronize(c->stream);  // the call's own error is reported
-  }
-  int wait() {
-    open = false;
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return UASD_OK;
-  }
-};
 
 // Whether every site's DM neighbours are its exchange neighbours, in the same
 // order and number, at most kFusedW of them (or there is no DM term): the
@@ -699,6 +776,16 @@ uasd::LLGDev<R> llg_view(uasd_ctx *c) {
   return p;
 }
 
+// Steps whose Philox deviates are drawn in one launch ahead of them.  FP64
+// deviates are a third of a predictor's instructions and, while the lattice
+// leaves CUs idle, of its time: midpoint and Depondt steps of 432 to 16,000
+// sites with 14 or 58 neighbours gain 0.3-0.8 us of 11-18.  At 65,536 sites
+// the extra pass over them costs what it saves, and FP32 deviates are too
+// cheap to gain at any size.
+int steps_ahead(const uasd_ctx *c) {
+  return c->prec == UASD_FP64 && (int64_t)c->N * c->M <= 32768 ? 16 : 1;
+}
+
 int ready_for_llg(uasd_ctx *c) {
   if (!c->have_ex) return fail(UASD_ERR_STATE, "exchange not set (uasd_set_exchange)");
   if (!c->have_state) return fail(UASD_ERR_STATE, "moments not set (uasd_set_moments)");
@@ -707,7 +794,7 @@ int ready_for_llg(uasd_ctx *c) {
     return fail(UASD_ERR_STATE, "injected noise selected but no normals uploaded");
   if (c->noise_mode == UASD_NOISE_PHILOX) {
     void *old = c->nsave.p;
-    HIP_TRY(c->nsave.ensure((size_t)c->N * c->M * 4 * c->rsize));
+    HIP_TRY(c->nsave.ensure((size_t)steps_ahead(c) * c->N * c->M * 4 * c->rsize));
     if (c->nsave.p != old) c->gen += 1;  // captured graphs hold the old address
   }
   return rebuild_classes(c);
@@ -723,9 +810,10 @@ bool sde_supported(int alg) {
 // solvers that keep b2eff between the halves
 bool sde_b2eff(int alg) { return alg == UASD_SDE_HEUN || alg == UASD_SDE_DEPONDT; }
 
+// ahead >= 0: the step's deviates lie in quad array `ahead` of c->nsave.
 template <typename R>
 int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
-                 int64_t step_off = -1) {
+                 int64_t step_off = -1, int ahead = -1) {
   uasd::HamDev<R> h = ham_view<R>(c);
   uasd::LLGDev<R> prm = llg_view<R>(c);
   if (step_off >= 0) {
@@ -734,7 +822,10 @@ int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
   }
   // a fused predictor/corrector pair draws the deviates once: the predictor
   // stores them, the corrector of the same step reads them back
-  if (fused && prm.noise_mode == UASD_NOISE_PHILOX) prm.nsave = c->nsave.as<uasd::Quad<R>>();
+  if (fused && prm.noise_mode == UASD_NOISE_PHILOX) {
+    prm.nsave = quads<R>(c, c->nsave, std::max(ahead, 0));
+    prm.nready = ahead >= 0 ? 1 : 0;
+  }
   uasd::Quad<R> *e = quads<R>(c, c->spins, 0), *p = quads<R>(c, c->spins, 1),
                 *b2 = quads<R>(c, c->spins, 2);
   const uasd::Quad<R> *beff = fused ? nullptr : quads<R>(c, c->field);
@@ -751,8 +842,9 @@ int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
     }
   }
   tic(c, half);
-  HIP_TRY(uasd::launch_llg<R>(c->stream, c->tune[0], alg, half, fused, h, prm, e, p, b2, beff,
-                              out));
+  HIP_TRY(uasd::launch_llg<R>(c->stream,
+                              uasd::default_tune(c->tune[0], (int64_t)c->N * c->M, c->W), alg,
+                              half, fused, h, prm, e, p, b2, beff, out));
   return toc(c, half);
 }
 
@@ -770,9 +862,37 @@ int run_field(uasd_ctx *c, bool from_scratch, bool want_energy, bool parts = fal
     en = c->energy.as<double>();
   }
   tic(c, 2);
-  HIP_TRY(uasd::launch_field<R>(c->stream, c->tune[1], h, src, want_beff ? quads<R>(c, c->field) : nullptr, en,
+  HIP_TRY(uasd::launch_field<R>(c->stream,
+                                uasd::default_tune(c->tune[1], (int64_t)c->N * c->M, c->W), h, src,
+                                want_beff ? quads<R>(c, c->field) : nullptr, en,
                                 parts ? quads<R>(c, c->field, 1) : nullptr));
   return toc(c, 2);
+}
+
+// Where a call's final sums are written: a few of them straight into pinned
+// host memory (the call waits for the stream anyway, and saves a copy
+// command), more into the device buffer d.  sums_back waits and brings them to
+// `out`.
+constexpr size_t kPinSums = 512;
+
+int sums_out(uasd_ctx *c, DevBuf &d, size_t n, double **dst) {
+  if (n <= kPinSums) {
+    HIP_TRY(c->pinsum.ensure(kPinSums * sizeof(double)));
+    *dst = static_cast<double *>(c->pinsum.p);
+    return UASD_OK;
+  }
+  HIP_TRY(d.ensure(n * sizeof(double)));
+  *dst = d.as<double>();
+  return UASD_OK;
+}
+
+int sums_back(uasd_ctx *c, const double *src, size_t n, double *out) {
+  const bool pinned = src == c->pinsum.p;
+  if (!pinned)
+    HIP_TRY(hipMemcpyAsync(out, src, n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  if (pinned) std::memcpy(out, src, n * sizeof(double));
+  return UASD_OK;
 }
 
 // FP64 sums per ensemble of emomM (and of the per-q energy terms written by
@@ -782,16 +902,15 @@ int reduce_moments(uasd_ctx *c, bool with_energy, bool from_scratch, std::vector
   const int nv = with_energy ? 4 : 3;
   const int nblocks = std::max(1, std::min(1024, (c->N + 255) / 256));
   HIP_TRY(c->partial.ensure((size_t)c->M * nblocks * nv * sizeof(double)));
-  HIP_TRY(c->redout.ensure((size_t)c->M * nv * sizeof(double)));
+  const size_t nout = (size_t)c->M * nv;
+  double *dst = nullptr;
+  if (int r = sums_out(c, c->redout, nout, &dst)) return r;
   const uasd::Quad<R> *s = from_scratch ? quads<R>(c, c->scratch) : quads<R>(c, c->spins, 0);
   HIP_TRY(uasd::launch_reduce<R>(c->stream, c->N, c->M, s,
                                  with_energy ? c->energy.as<double>() : nullptr, nv,
-                                 c->partial.as<double>(), nblocks, c->redout.as<double>()));
-  out.resize((size_t)c->M * nv);
-  HIP_TRY(hipMemcpyAsync(out.data(), c->redout.p, out.size() * sizeof(double),
-                         hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  return UASD_OK;
+                                 c->partial.as<double>(), nblocks, dst));
+  out.resize(nout);
+  return sums_back(c, dst, nout, out.data());
 }
 
 int build_coloring(uasd_ctx *c) {
@@ -1400,7 +1519,7 @@ int uasd_set_external_field(uasd_ctx *c, const double *field) {
   c->ext_mode = 2;
   if (int r = upload_real(c, c->ext_u, c->ext_u_host)) return r;
   HostIo io(c);
-  if (int r = upload_vec(c, c->ext_full, 0, field, PackW{})) return r;
+  if (int r = upload_vec(io, c->ext_full, 0, field, PackW{})) return r;
   return io.wait();
 }
 
@@ -1453,7 +1572,7 @@ int uasd_set_noise(uasd_ctx *c, int mode, uint64_t seed, const double *normals) 
   if (mode == UASD_NOISE_INJECTED) {
     if (!normals) return fail(UASD_ERR_ARG, "injected noise needs the normals array");
     HostIo io(c);
-    if (int r = upload_vec(c, c->noise, 0, normals, PackW{})) return r;
+    if (int r = upload_vec(io, c->noise, 0, normals, PackW{})) return r;
     if (int r = io.wait()) return r;
   }
   if (mode == UASD_NOISE_PHILOX && (seed != c->seed || c->noise_mode != mode)) c->step = 0;
@@ -1466,7 +1585,16 @@ int uasd_set_moments(uasd_ctx *c, const double *emom, const double *mmom) {
   if (int r = check_ctx(c)) return r;
   if (!emom || !mmom) return fail(UASD_ERR_ARG, "uasd_set_moments: null array");
   HostIo io(c);
-  if (int r = upload_vec(c, c->spins, 0, emom, PackW{mmom})) return r;
+  io.open = true;
+  // the raw arrays pass through the memory of the quad arrays 1 and 2 (32 bytes
+  // a pair in either precision), which are written after them: a call that
+  // every program makes once needs no staging of its own
+  const size_t pairs = (size_t)c->N * c->M;
+  double *sa = reinterpret_cast<double *>(static_cast<char *>(c->spins.p) + quad_bytes(c));
+  HIP_TRY(hipMemcpyAsync(sa, emom, 3 * pairs * sizeof(double), hipMemcpyHostToDevice, c->stream));
+  HIP_TRY(hipMemcpyAsync(sa + 3 * pairs, mmom, pairs * sizeof(double), hipMemcpyHostToDevice,
+                         c->stream));
+  if (int r = launch_pack(c, c->spins, 0, 0, pairs, sa, sa + 3 * pairs, PackW{})) return r;
   HIP_TRY(hipMemcpyAsync(static_cast<char *>(c->spins.p) + quad_bytes(c), c->spins.p,
                          quad_bytes(c), hipMemcpyDeviceToDevice,
                          c->stream));  // emom2 starts as emom
@@ -1484,9 +1612,9 @@ int uasd_get_moments(uasd_ctx *c, double *emom, double *emomM) {
   if (!c->have_state) return fail(UASD_ERR_STATE, "moments not set");
   HostIo io(c);
   if (emom)
-    if (int r = download_vec(c, c->spins, 0, emom, false)) return r;
+    if (int r = download_vec(io, c->spins, 0, emom, false)) return r;
   if (emomM)
-    if (int r = download_vec(c, c->spins, 0, emomM, true)) return r;
+    if (int r = download_vec(io, c->spins, 0, emomM, true)) return r;
   return io.wait();
 }
 
@@ -1496,8 +1624,8 @@ int uasd_get_moments(uasd_ctx *c, double *emom, double *emomM) {
 
 // quad array k of the spins <- the (3,N,M) array a, with w = mmom of the
 // state (quad array 0): the magnitudes stay on the device
-static int upload_vec_keep_w(uasd_ctx *c, int k, const double *a) {
-  return upload_vec(c, c->spins, k, a, PackW{nullptr, 1, 0.0});
+static int upload_vec_keep_w(HostIo &io, int k, const double *a) {
+  return upload_vec(io, io.c->spins, k, a, PackW{1, 0.0});
 }
 
 int uasd_effective_field_host(uasd_ctx *c, const double *emomM, double *beff, double *beff1,
@@ -1507,14 +1635,14 @@ int uasd_effective_field_host(uasd_ctx *c, const double *emomM, double *beff, do
   if (!emomM || !beff) return fail(UASD_ERR_ARG, "null array");
   if (int r = rebuild_classes(c)) return r;
   HostIo io(c);
-  if (int r = upload_vec(c, c->scratch, 0, emomM, PackW{nullptr, 0, 1.0})) return r;
+  if (int r = upload_vec(io, c->scratch, 0, emomM, PackW{0, 1.0})) return r;
   const bool parts = beff1 || beff2;
   int r = c->prec == UASD_FP64 ? run_field<double>(c, true, energy != nullptr, parts)
                                : run_field<float>(c, true, energy != nullptr, parts);
   if (r) return r;
-  if ((r = download_vec(c, c->field, 0, beff, false))) return r;
-  if (beff1 && (r = download_vec(c, c->field, 1, beff1, false))) return r;
-  if (beff2 && (r = download_vec(c, c->field, 2, beff2, false))) return r;
+  if ((r = download_vec(io, c->field, 0, beff, false))) return r;
+  if (beff1 && (r = download_vec(io, c->field, 1, beff1, false))) return r;
+  if (beff2 && (r = download_vec(io, c->field, 2, beff2, false))) return r;
   if (energy) {
     std::vector<double> red;
     r = c->prec == UASD_FP64 ? reduce_moments<double>(c, true, true, red)
@@ -1536,9 +1664,9 @@ int uasd_evolve_first_host(uasd_ctx *c, int alg, const double *beff, double *emo
     return fail(UASD_ERR_ARG, "null array");
   if (int r = ready_for_llg(c)) return r;
   HostIo io(c);
-  if (int r = upload_vec(c, c->field, 0, beff, PackW{})) return r;
+  if (int r = upload_vec(io, c->field, 0, beff, PackW{})) return r;
   // heun4p starts from emom2 (heun_proper.f90:309-311), the others from emom
-  if (int r = upload_vec_keep_w(c, 0, alg == UASD_SDE_HEUN ? emom2 : emom)) return r;
+  if (int r = upload_vec_keep_w(io, 0, alg == UASD_SDE_HEUN ? emom2 : emom)) return r;
   int r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 0, false, false)
                                : run_llg_half<float>(c, alg, 0, false, false);
   if (r) return r;
@@ -1546,19 +1674,19 @@ int uasd_evolve_first_host(uasd_ctx *c, int alg, const double *beff, double *emo
     // depondt.f90:182-187: emom2 = m(t), emom = rotated, emomM = emom*mmom, b2eff = bdup
     if ((r = io.wait())) return r;  // emom has been read before it is written
     std::memcpy(emom2, emom, sizeof(double) * 3 * (size_t)c->N * c->M);
-    if ((r = download_vec(c, c->spins, 1, emom, false))) return r;
-    if ((r = download_vec(c, c->spins, 2, b2eff, false))) return r;
+    if ((r = download_vec(io, c->spins, 1, emom, false))) return r;
+    if ((r = download_vec(io, c->spins, 2, b2eff, false))) return r;
   } else if (alg == UASD_SDE_HEUN) {
     // heun_proper.f90:303-365: b2eff = beff, emom = predictor, emomM =
     // emom*mmom, emom2 unchanged
-    if ((r = download_vec(c, c->spins, 1, emom, false))) return r;
-    if ((r = download_vec(c, c->spins, 2, b2eff, false))) return r;
+    if ((r = download_vec(io, c->spins, 1, emom, false))) return r;
+    if ((r = download_vec(io, c->spins, 2, b2eff, false))) return r;
   } else {
     // midpoint.f90:167-175 (and sibt / sispht, sphmidpoint.f90:247-258,
     // 698-710): emom2 = et', emomM = et'*mmom, emom unchanged
-    if ((r = download_vec(c, c->spins, 1, emom2, false))) return r;
+    if ((r = download_vec(io, c->spins, 1, emom2, false))) return r;
   }
-  if ((r = download_vec(c, c->spins, 1, emomM, true))) return r;
+  if ((r = download_vec(io, c->spins, 1, emomM, true))) return r;
   return io.wait();
 }
 
@@ -1571,15 +1699,15 @@ int uasd_evolve_second_host(uasd_ctx *c, int alg, const double *beff, const doub
     return fail(UASD_ERR_ARG, "null array");
   if (int r = ready_for_llg(c)) return r;
   HostIo io(c);
-  if (int r = upload_vec(c, c->field, 0, beff, PackW{})) return r;
+  if (int r = upload_vec(io, c->field, 0, beff, PackW{})) return r;
   if (alg == UASD_SDE_DEPONDT || alg == UASD_SDE_HEUN) {
     // reference on entry: emom = predicted, emom2 = m(t)
-    if (int r = upload_vec_keep_w(c, 1, emom)) return r;
-    if (int r = upload_vec_keep_w(c, 0, emom2)) return r;
-    if (int r = upload_vec(c, c->spins, 2, b2eff, PackW{})) return r;
+    if (int r = upload_vec_keep_w(io, 1, emom)) return r;
+    if (int r = upload_vec_keep_w(io, 0, emom2)) return r;
+    if (int r = upload_vec(io, c->spins, 2, b2eff, PackW{})) return r;
   } else {
-    if (int r = upload_vec_keep_w(c, 0, emom)) return r;
-    if (int r = upload_vec_keep_w(c, 1, emom2)) return r;
+    if (int r = upload_vec_keep_w(io, 0, emom)) return r;
+    if (int r = upload_vec_keep_w(io, 1, emom2)) return r;
   }
   int r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 1, false, false)
                                : run_llg_half<float>(c, alg, 1, false, false);
@@ -1588,7 +1716,7 @@ int uasd_evolve_second_host(uasd_ctx *c, int alg, const double *beff, const doub
     if ((r = io.wait())) return r;  // both have been read before they are written
     std::memcpy(emom, emom2, sizeof(double) * 3 * (size_t)c->N * c->M);
   }
-  if ((r = download_vec(c, c->spins, 1, emom2, false))) return r;
+  if ((r = download_vec(io, c->spins, 1, emom2, false))) return r;
   if ((r = io.wait())) return r;
   c->step += 1;
   return UASD_OK;
@@ -1693,36 +1821,92 @@ int uasd_sd_steps(uasd_ctx *c, int alg, int64_t nsteps) {
 
 namespace {
 
+// One LLG step, both halves; step_off, ahead as in run_llg_half.
+int llg_step(uasd_ctx *c, int alg, int64_t step_off, int ahead) {
+  const bool d = c->prec == UASD_FP64;
+  for (int half = 0; half < 2; ++half) {
+    const int r = d ? run_llg_half<double>(c, alg, half, true, half == 1, step_off, ahead)
+                    : run_llg_half<float>(c, alg, half, true, half == 1, step_off, ahead);
+    if (r) return r;
+  }
+  return UASD_OK;
+}
+
+// Deviates of n steps (from the context's step, or inside a capture from
+// *ctr[0] + step_off) into c->nsave.
+template <typename R>
+int draw_ahead(uasd_ctx *c, int n, int64_t step_off) {
+  uasd::LLGDev<R> prm = llg_view<R>(c);
+  if (step_off >= 0) {
+    prm.step = (uint64_t)step_off;
+    prm.step_dev = c->ctr.as<uint64_t>();
+  }
+  HIP_TRY(uasd::launch_draw<R>(c->stream, ham_view<R>(c), prm, n, quads<R>(c, c->nsave)));
+  return UASD_OK;
+}
+
+// n LLG steps launched one by one; in_graph: inside a capture, counted from
+// the device counter.
+int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
+  const int K = llg_view<double>(c).noise_mode == UASD_NOISE_PHILOX ? steps_ahead(c) : 1;
+  for (int64_t s = 0; s < n; ++s) {
+    const int k = (int)(s % K);
+    const int64_t off = in_graph ? s : -1;
+    if (K > 1 && k == 0) {
+      const int m = (int)std::min<int64_t>(K, n - s);
+      const int r = c->prec == UASD_FP64 ? draw_ahead<double>(c, m, off)
+                                         : draw_ahead<float>(c, m, off);
+      if (r) return r;
+    }
+    if (int r = llg_step(c, alg, off, K > 1 ? k : -1)) return r;
+    if (!in_graph) c->step += 1;
+  }
+  return UASD_OK;
+}
+
+// Whether n more steps (kind 0) or sweeps (kind 1) of a call should be
+// replayed as graphs although none were asked for: the launches are short
+// (items = sites x ensembles of one), the program has already launched `after`
+// of them one by one with nothing changed in between, and nobody is timing the
+// kernels or capturing the stream.  A replayed launch of a small lattice is
+// 0.4-1.6 us shorter than an enqueued one (its arguments already lie in device
+// memory): 432 sites, 14 neighbours, FP64 13.3 -> 10.3 us a step, FP32 11.9 ->
+// 8.6; 16,000 sites 14.3 -> 11.7; 65,536 sites (film) FP32 14.8 -> 13.0, FP64
+// 16.7 -> 15.6; nothing from 2^18 items on.  Capturing costs about a
+// millisecond, hence `after`.
+bool repeats_pay(uasd_ctx *c, int kind, int alg, uint64_t seed, int64_t items, int64_t n,
+                 int64_t after) {
+  if (c->graph_steps > 0 || c->timing || items > 131072) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
+    return false;
+  if (c->repeats.size() > 64) c->repeats.clear();
+  auto &r = c->repeats[std::make_tuple(kind, alg, seed)];
+  if (r.first != c->gen) r = {c->gen, 0};
+  r.second += n;
+  return r.second - n >= after;
+}
+
 int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps) {
   int64_t s = 0;
-  const int K = c->graph_steps;
-  if (K > 0) {
+  auto replay = [&](int K) -> int {
     auto body = [&]() -> int {
-      for (int j = 0; j < K; ++j) {
-        int r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 0, true, false, j)
-                                     : run_llg_half<float>(c, alg, 0, true, false, j);
-        if (r) return r;
-        r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 1, true, true, j)
-                                 : run_llg_half<float>(c, alg, 1, true, true, j);
-        if (r) return r;
-      }
+      if (int r = llg_steps(c, alg, K, true)) return r;
       HIP_TRY(uasd::launch_counter(c->stream, 0, c->ctr.as<uint64_t>(), (uint64_t)K, 1));
       return UASD_OK;
     };
     for (; nsteps - s >= K; s += K)
       if (int r = replay_graph(c, std::make_tuple(0, alg, K, (uint64_t)0), 0, c->step, K, 4, body))
         return r;
+    return UASD_OK;
+  };
+  if (c->graph_steps > 0) {
+    if (int r = replay(c->graph_steps)) return r;
+  } else if (repeats_pay(c, 0, alg, 0, (int64_t)c->N * c->M, nsteps, 512)) {
+    for (int K : {64, 16})
+      if (int r = replay(K)) return r;
   }
-  for (; s < nsteps; ++s) {
-    int r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 0, true, false)
-                                 : run_llg_half<float>(c, alg, 0, true, false);
-    if (r) return r;
-    r = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 1, true, true)
-                             : run_llg_half<float>(c, alg, 1, true, true);
-    if (r) return r;
-    c->step += 1;
-  }
-  return UASD_OK;
+  return llg_steps(c, alg, nsteps - s, false);
 }
 
 }  // namespace
@@ -1738,7 +1922,7 @@ int uasd_effective_field(uasd_ctx *c, double *beff, double *energy) {
               : run_field<float>(c, false, energy != nullptr, false, beff != nullptr);
   if (r) return r;
   HostIo io(c);
-  if (beff && (r = download_vec(c, c->field, 0, beff, false))) return r;
+  if (beff && (r = download_vec(io, c->field, 0, beff, false))) return r;
   if (energy) {
     std::vector<double> red;
     r = c->prec == UASD_FP64 ? reduce_moments<double>(c, true, false, red)
@@ -1936,6 +2120,11 @@ static int mc_resident(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
   return UASD_OK;
 }
 
+// Launch shape of a colour of nsites sites.
+static uasd::Tune mc_tune(const uasd_ctx *c, int nsites) {
+  return uasd::default_tune(c->tune[2], (int64_t)nsites * c->M, c->W);
+}
+
 // nsweeps colour-ordered sweeps; every launch is asynchronous on the stream.
 static int mc_run(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
   const int *sites_dev = mp.sites;
@@ -1954,10 +2143,10 @@ static int mc_run(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
       mp.sstride = c->color_stride[col];
       tic(c, 3);
       if (c->prec == UASD_FP64) {
-        HIP_TRY(uasd::launch_mc<double>(c->stream, c->tune[2], ham_view<double>(c), mp,
+        HIP_TRY(uasd::launch_mc<double>(c->stream, mc_tune(c, mp.nsites), ham_view<double>(c), mp,
                                         quads<double>(c, c->spins, 0)));
       } else {
-        HIP_TRY(uasd::launch_mc<float>(c->stream, c->tune[2], ham_view<float>(c), mp,
+        HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, mp.nsites), ham_view<float>(c), mp,
                                        quads<float>(c, c->spins, 0)));
       }
       if (int r = toc(c, 3)) return r;
@@ -1984,8 +2173,7 @@ namespace {
 int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nsweeps,
                   uint64_t seed) {
   int64_t s = 0;
-  const int K = c->graph_steps;
-  if (K > 0) {
+  auto replay = [&](int K) -> int {
     auto body = [&]() -> int {
       uasd::MCParams g = mp;
       g.sweep_dev = c->ctr.as<uint64_t>() + 1;
@@ -2002,10 +2190,10 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
           g.site0 = c->color_start[col];
           g.sstride = c->color_stride[col];
           if (c->prec == UASD_FP64) {
-            HIP_TRY(uasd::launch_mc<double>(c->stream, c->tune[2], ham_view<double>(c), g,
+            HIP_TRY(uasd::launch_mc<double>(c->stream, mc_tune(c, mp.nsites), ham_view<double>(c), g,
                                             quads<double>(c, c->spins, 0)));
           } else {
-            HIP_TRY(uasd::launch_mc<float>(c->stream, c->tune[2], ham_view<float>(c), g,
+            HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, mp.nsites), ham_view<float>(c), g,
                                            quads<float>(c, c->spins, 0)));
           }
         }
@@ -2017,6 +2205,15 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
       if (int r = replay_graph(c, std::make_tuple(1, (int)mode, K, seed), 1, c->mc_sweep, K, 5,
                                body))
         return r;
+    return UASD_OK;
+  };
+  if (c->graph_steps > 0) {
+    if (int r = replay(c->graph_steps)) return r;
+  } else if (!mc_use_resident(c) &&
+             repeats_pay(c, 1, mode, seed, (int64_t)c->N * c->M / std::max(c->ncolors, 1),
+                         nsweeps, 64)) {
+    for (int K : {16, 4})
+      if (int r = replay(K)) return r;
   }
   return mc_run(c, mp, nsweeps - s);
 }
@@ -2055,7 +2252,7 @@ int uasd_set_tuning(uasd_ctx *c, int kind, int gather, int block) {
   // where the DM bonds are the exchange bonds (context-wide), 0x1000000 two
   // adjacent ensembles per thread (MC only)
   uasd::Tune t{gather, block & 0xffff, (block >> 16) & 1, (block >> 17) & 1, (block >> 18) & 0xf,
-               (block >> 22) & 1, (block >> 24) & 1};
+               (block >> 22) & 1, (block >> 24) & 1, 1};
   if (!uasd::tune_valid(t) || (block >> 25) != 0 || (kind != 0 && t.tile != 0) ||
       (kind != 2 && t.pair != 0))
     return fail(UASD_ERR_ARG, "gather must be 2, 4, 8 or 16 and block 64, 128 or 256");
@@ -2190,6 +2387,7 @@ int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool 
   for (const uasd::Tune &cd : cand) {
     {
       *slot = cd;
+      slot->chosen = 1;
       if (int r = run()) return r;
       HIP_TRY(hipEventRecord(ev.a, c->stream));
       if (int r = run()) return r;
@@ -2224,6 +2422,7 @@ int uasd_autotune_llg(uasd_ctx *c, int alg, int steps, double *best_ms) {
   double cached_ms = 0.0;
   if (tune_lookup(key, cached, cached_ms) && uasd::tune_valid(cached) && cached.pair == 0 &&
       (cached.tile == 0 || tile_fits(c, cached.tile))) {
+    cached.chosen = 1;
     c->tune[0] = c->tune[1] = cached;
     c->tune[1].tile = c->tune[1].pipe = 0;
     if (best_ms) *best_ms = cached_ms;
@@ -2233,18 +2432,8 @@ int uasd_autotune_llg(uasd_ctx *c, int alg, int steps, double *best_ms) {
   StateGuard g(c);
   if (g.err) return g.err;
   double ms_found = 0.0;
-  int r = tune_search(c, &c->tune[0], [&]() -> int {
-    for (int s = 0; s < steps; ++s) {
-      int e = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 0, true, false)
-                                   : run_llg_half<float>(c, alg, 0, true, false);
-      if (e) return e;
-      e = c->prec == UASD_FP64 ? run_llg_half<double>(c, alg, 1, true, true)
-                               : run_llg_half<float>(c, alg, 1, true, true);
-      if (e) return e;
-      c->step += 1;
-    }
-    return UASD_OK;
-  }, &ms_found);
+  int r = tune_search(c, &c->tune[0], [&]() -> int { return llg_steps(c, alg, steps, false); },
+                      &ms_found);
   if (r) return r;
   if (best_ms) *best_ms = ms_found;
   tune_store(key, c->tune[0], ms_found);
@@ -2262,6 +2451,7 @@ int uasd_autotune_mc(uasd_ctx *c, char mode, const double *temps, int sweeps, do
   uasd::Tune cached;
   double cached_ms = 0.0;
   if (tune_lookup(key, cached, cached_ms) && uasd::tune_valid(cached) && cached.tile == 0) {
+    cached.chosen = 1;
     c->tune[2] = cached;
     if (best_ms) *best_ms = cached_ms;
     c->gen += 1;
