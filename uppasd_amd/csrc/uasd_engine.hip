@@ -219,6 +219,8 @@ struct uasd_ctx {
   DevBuf tile_off;
   int tile_off_shape = 0;
   std::vector<int> cls_host;       // site class per device slot
+  bool one_class = false;          // every site is of class class0
+  uasd::SiteClass class0{0, -1, -1, 0};
   int64_t cls_version = 0;         // bumped by every class rebuild
   int64_t ucls_version = -1;       // cls_version the per-basis check below is for
   int ucls = 0, cls_b[8] = {0};
@@ -362,6 +364,13 @@ uasd::HamDev<R> ham_view(const uasd_ctx *c) {
   }
   h.cls = c->cls.as<int>();
   h.classes = c->classes.as<uasd::SiteClass>();
+  // Scalar couplings take a load per neighbour off the texture-address units,
+  // which bound a full chip (film of 262,144 sites, Depondt FP64 25.2 -> 20.6
+  // us a step; 170,368 sites with 14 neighbours 25.6 -> 23.3), but each batch
+  // waits for them on top of its gathers, which a chip that is mostly waiting
+  // anyway feels (16,000 sites with 58 neighbours 16.5 -> 17.4).
+  h.one = !c->one_class ? 0 : (int64_t)c->N * c->M > 131072 ? 2 : 1;
+  h.c0 = c->class0;
   h.ext_mode = c->ext_mode;
   h.order_na = c->order_na;
   h.idx_kb = idx_kb(c);
@@ -622,6 +631,8 @@ int rebuild_classes(uasd_ctx *c, bool may_alloc = true) {
   r = upload_raw(c, c->classes, table);
   if (r) return r;
   c->cls_host = cls;
+  c->one_class = table.size() == 1;
+  c->class0 = table[0];
   c->cls_version += 1;
   c->classes_dirty = false;
   c->gen += 1;

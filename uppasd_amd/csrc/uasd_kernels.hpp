@@ -99,6 +99,12 @@ struct HamDev {
   // site classes
   const int *__restrict__ cls;
   const SiteClass *__restrict__ classes;
+  // one > 0: every site is of class c0 (a crystal whose basis atoms have the
+  // same couplings), which then comes with the launch.  one = 2: the couplings,
+  // the same for all lanes, are also read through the scalar cache (see
+  // ham_view for where that pays).
+  int one;
+  SiteClass c0;
   // external field: 0 none, 1 uniform per ensemble (ext_u[3*ens+c]), 2 per q
   int ext_mode;
   // 1: neighbour lists are read with non-temporal loads (streamed past L2,
@@ -128,6 +134,27 @@ __device__ __forceinline__ int64_t xcd_block() {
   const uint32_t per = gridDim.x / kXCD;
   const uint32_t b = blockIdx.x;
   return (int64_t)(b % kXCD) * per + (b / kXCD);
+}
+
+// Load through the constant address space: the tables it is used for (class
+// rows, couplings, DM vectors) are not written by any kernel, and a
+// wave-uniform address is then read with a scalar load.
+template <typename T>
+__device__ __forceinline__ T cload(const T *p) {
+  return *(const __attribute__((address_space(4))) T *)p;
+}
+
+// The same where UNI says that the address is wave-uniform, an ordinary load
+// elsewhere.
+template <bool UNI, typename T>
+__device__ __forceinline__ T tload(const T *p) {
+  if constexpr (UNI) return cload(p);
+  return *p;
+}
+
+template <typename R>
+__device__ __forceinline__ SiteClass site_class(const HamDev<R> &h, int site) {
+  return h.one ? h.c0 : h.classes[h.cls[site]];
 }
 
 // ------------------------------------------------------------------- Philox
@@ -413,7 +440,8 @@ __device__ __forceinline__ I nb_load(const I *p) {
 // (J m_j) e_j instead of J (e_j m_j), one multiply fewer per neighbour and
 // equal to rounding (the MC energy differences, not the fields of the LLG
 // step, which keep the reference's emomM products).
-template <typename R, int G, bool NT, typename I, int U, bool JW = false, typename D = NbDec>
+template <typename R, int G, bool NT, typename I, int U, bool JW = false, typename D = NbDec,
+          bool UNI = false>
 __device__ __forceinline__ void exchange_run(const HamDev<R> &h, const I *__restrict__ nb,
                                              const Quad<R> *__restrict__ src, int site, int e0,
                                              int row, int len, R (&f)[U][3]) {
@@ -432,7 +460,7 @@ __device__ __forceinline__ void exchange_run(const HamDev<R> &h, const I *__rest
     for (int u = 0; u < G; ++u) {
 #pragma unroll
       for (int k = 0; k < U; ++k) v[u][k] = src[(size_t)n[u] * M + e0 + k];
-      J[u] = cp[(size_t)(j + u) * rs];
+      J[u] = tload<UNI>(cp + (size_t)(j + u) * rs);
     }
 #pragma unroll
     for (int u = 0; u < G; ++u) {
@@ -463,7 +491,7 @@ __device__ __forceinline__ void exchange_run(const HamDev<R> &h, const I *__rest
       if (j + u < len) {
 #pragma unroll
         for (int k = 0; k < U; ++k) v[u][k] = src[(size_t)n[u] * M + e0 + k];
-        J[u] = cp[(size_t)(j + u) * rs];
+        J[u] = tload<UNI>(cp + (size_t)(j + u) * rs);
       }
     }
 #pragma unroll
@@ -488,12 +516,15 @@ __device__ __forceinline__ void exchange_run(const HamDev<R> &h, const I *__rest
 }
 
 // When every row holds W neighbours the loop runs to the launch argument W,
-// the same for every lane: its control and the batch tail are scalar.
+// the same for every lane: its control and the batch tail are scalar.  With
+// one site class the couplings are too.
 template <typename R, int G, bool NT, typename I, int U, bool JW = false>
 __device__ __forceinline__ void exchange_fields(const HamDev<R> &h, const I *__restrict__ nb,
                                                 const Quad<R> *__restrict__ src, int site, int e0,
                                                 int row, R (&f)[U][3]) {
-  if (h.ex_full)
+  if (h.one == 2)
+    exchange_run<R, G, NT, I, U, JW, NbDec, true>(h, nb, src, site, e0, h.c0.ex_row, h.W, f);
+  else if (h.ex_full)
     exchange_run<R, G, NT, I, U, JW>(h, nb, src, site, e0, row, h.W, f);
   else
     exchange_run<R, G, NT, I, U, JW>(h, nb, src, site, e0, row, h.ex_len[row], f);
@@ -507,7 +538,9 @@ __device__ __forceinline__ void mc_exchange_fields(const HamDev<R> &h, const I *
                                                    const Quad<R> *__restrict__ src, int site,
                                                    int e0, int row, R (&f)[U][3]) {
   if (std::is_same<I, int16_t>::value && h.order_na == 1) {
-    if (h.ex_full)
+    if (h.one == 2)
+      exchange_run<R, G, NT, I, U, true, NbDec1, true>(h, nb, src, site, e0, h.c0.ex_row, h.W, f);
+    else if (h.ex_full)
       exchange_run<R, G, NT, I, U, true, NbDec1>(h, nb, src, site, e0, row, h.W, f);
     else
       exchange_run<R, G, NT, I, U, true, NbDec1>(h, nb, src, site, e0, row, h.ex_len[row], f);
@@ -528,7 +561,7 @@ __device__ __forceinline__ void exchange_sum(const HamDev<R> &h, const I *__rest
 }
 
 // DM sum of site_field: field += m_j x D_ij (hamiltonianactions.f90:565-578).
-template <typename R, int G, typename I, typename D = NbDec>
+template <typename R, int G, typename I, typename D = NbDec, bool UNI = false>
 __device__ __forceinline__ void dm_sum(const HamDev<R> &h, const I *__restrict__ nb,
                                        const Quad<R> *__restrict__ src, int site, int ens,
                                        int row, R &s0, R &s1, R &s2) {
@@ -549,7 +582,8 @@ __device__ __forceinline__ void dm_sum(const HamDev<R> &h, const I *__restrict__
     for (int u = 0; u < G; ++u) {
       if (j + u < len) {
         const size_t r = (size_t)(j + u) * rs + row;
-        const R D0 = h.dvx[r], D1 = h.dvy[r], D2 = h.dvz[r];
+        const R D0 = tload<UNI>(h.dvx + r), D1 = tload<UNI>(h.dvy + r),
+                D2 = tload<UNI>(h.dvz + r);
         const R m0 = v[u].x * v[u].w, m1 = v[u].y * v[u].w, m2 = v[u].z * v[u].w;
         s0 = s0 + D2 * m1 - D1 * m2;
         s1 = s1 + D0 * m2 - D2 * m0;
@@ -566,7 +600,7 @@ __device__ __forceinline__ void dm_sum(const HamDev<R> &h, const I *__restrict__
 // adds them, so the field is bit-identical to the two separate sums.
 constexpr int kFusedW = 8;
 
-template <typename R, int G, bool NT, typename I>
+template <typename R, int G, bool NT, typename I, bool UNI = false>
 __device__ __forceinline__ void exdm_run(const HamDev<R> &h, const I *__restrict__ nb,
                                          const Quad<R> *__restrict__ src, int site, int ens,
                                          int exrow, int dmrow, int len, R &s0, R &s1, R &s2) {
@@ -587,7 +621,7 @@ __device__ __forceinline__ void exdm_run(const HamDev<R> &h, const I *__restrict
     for (int u = 0; u < G; ++u) {
       if (j0 + u < len) {
         v[u] = src[(size_t)n[u] * M + ens];
-        J[u] = cp[(size_t)(j0 + u) * rs];
+        J[u] = tload<UNI>(cp + (size_t)(j0 + u) * rs);
       }
     }
 #pragma unroll
@@ -608,7 +642,7 @@ __device__ __forceinline__ void exdm_run(const HamDev<R> &h, const I *__restrict
   for (int j = 0; j < kFusedW; ++j) {
     if (j < len) {
       const size_t r = (size_t)j * drs + dmrow;
-      const R D0 = h.dvx[r], D1 = h.dvy[r], D2 = h.dvz[r];
+      const R D0 = tload<UNI>(h.dvx + r), D1 = tload<UNI>(h.dvy + r), D2 = tload<UNI>(h.dvz + r);
       s0 = s0 + D2 * c1[j] - D1 * c2[j];
       s1 = s1 + D0 * c2[j] - D2 * c0[j];
       s2 = s2 + D1 * c0[j] - D0 * c1[j];
@@ -621,7 +655,10 @@ template <typename R, int G, bool NT, typename I>
 __device__ __forceinline__ void exdm_sum(const HamDev<R> &h, const I *__restrict__ nb,
                                          const Quad<R> *__restrict__ src, int site, int ens,
                                          int exrow, int dmrow, R &s0, R &s1, R &s2) {
-  if (h.ex_full)
+  if (h.one == 2)
+    exdm_run<R, G, NT, I, true>(h, nb, src, site, ens, h.c0.ex_row, h.Wd > 0 ? h.c0.dm_row : -1,
+                                h.W, s0, s1, s2);
+  else if (h.ex_full)
     exdm_run<R, G, NT, I>(h, nb, src, site, ens, exrow, dmrow, h.W, s0, s1, s2);
   else
     exdm_run<R, G, NT, I>(h, nb, src, site, ens, exrow, dmrow, h.ex_len[exrow], s0, s1, s2);
@@ -634,7 +671,7 @@ __device__ __forceinline__ void site_field(const HamDev<R> &h, const Quad<R> *__
                                            R &qf1, R &qf2, R &x0, R &x1, R &x2) {
   s0 = s1 = s2 = (R)0;
   qf0 = qf1 = qf2 = (R)0;
-  const SiteClass sc = h.classes[h.cls[site]];
+  const SiteClass sc = site_class(h, site);
   const int M = h.M;
   if (h.dm_shared) {
     const int dr = h.Wd > 0 ? sc.dm_row : -1;
@@ -735,7 +772,7 @@ __device__ __forceinline__ void anisotropy(const HamDev<R> &h, const SiteClass &
 template <typename R, int G, int U>
 __device__ __forceinline__ void site_field_u(const HamDev<R> &h, const Quad<R> *__restrict__ src,
                                              int site, int e0, R (&sf)[U][3], R (&qf)[U][3]) {
-  const SiteClass sc = h.classes[h.cls[site]];
+  const SiteClass sc = site_class(h, site);
   const int M = h.M, row = sc.ex_row;
 #pragma unroll
   for (int k = 0; k < U; ++k) sf[k][0] = sf[k][1] = sf[k][2] = qf[k][0] = qf[k][1] = qf[k][2] = (R)0;
@@ -1326,14 +1363,6 @@ __device__ __forceinline__ int dev_slot(const HamDev<R> &h, int i) {
   return h.order_na == 1 ? i : (i % h.order_na) * h.order_nc + i / h.order_na;
 }
 
-// Load through the constant address space: the tables it is used for (class
-// rows, couplings, DM vectors) are not written by any kernel, and a
-// wave-uniform address is then read with a scalar load.
-template <typename T>
-__device__ __forceinline__ T cload(const T *p) {
-  return *(const __attribute__((address_space(4))) T *)p;
-}
-
 // Values per component plane of the LDS tile: the launch takes the smallest
 // that holds NA*HV.  Each is 8 more than a multiple of 64, so the three
 // component reads of a neighbour never pair into one two-address LDS read
@@ -1830,7 +1859,7 @@ __device__ __forceinline__ void mc_delta_e(const HamDev<R> &h, const Quad<R> *__
                                            int site, int e0, const Quad<R> (&me)[U],
                                            const R (&tr)[U][3], const R (&x)[U][3],
                                            R (&de)[U]) {
-  const SiteClass sc = h.classes[h.cls[site]];
+  const SiteClass sc = site_class(h, site);
   R f[U][3];
 #pragma unroll
   for (int k = 0; k < U; ++k) f[k][0] = f[k][1] = f[k][2] = (R)0;
@@ -2409,7 +2438,7 @@ __global__ void __launch_bounds__(256)
   double a[4] = {0.0, 0.0, 0.0, 0.0};
   for (int site = ch.x + (int)threadIdx.x; site < ch.y; site += blockDim.x) {
     const size_t q = (size_t)site * M + ens;
-    const SiteClass sc = h.classes[h.cls[site]];
+    const SiteClass sc = site_class(h, site);
     R m0, m1, m2;
     moment(src, q, m0, m1, m2);
     R b0 = (R)0, b1 = (R)0, b2 = (R)0;
