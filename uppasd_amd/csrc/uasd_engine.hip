@@ -434,16 +434,19 @@ struct PairMap {
 
 // Pairs [p0, p0 + n) of a staged array a (and w) into their quads.  wsrc and
 // dst may be the same array: each thread reads and writes its own quad.
+// dst2, where given, gets the same quads.
 template <typename R>
 __global__ void __launch_bounds__(256)
     k_pack(PairMap m, size_t p0, size_t n, const double *__restrict__ a,
            const double *__restrict__ w, const uasd::Quad<R> *wsrc, double wconst,
-           uasd::Quad<R> *dst) {
+           uasd::Quad<R> *dst, uasd::Quad<R> *dst2) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= n) return;
   const size_t q = m.quad(p0 + t);
-  dst[q] = uasd::Quad<R>{(R)a[3 * t], (R)a[3 * t + 1], (R)a[3 * t + 2],
-                         w ? (R)w[t] : wsrc ? wsrc[q].w : (R)wconst};
+  const uasd::Quad<R> v{(R)a[3 * t], (R)a[3 * t + 1], (R)a[3 * t + 2],
+                        w ? (R)w[t] : wsrc ? wsrc[q].w : (R)wconst};
+  dst[q] = v;
+  if (dst2) dst2[q] = v;
 }
 
 // The reverse: xyz, or xyz*w (emomM), of pairs [p0, p0 + n) in FP64.
@@ -507,16 +510,16 @@ struct HostIo {
 };
 
 int launch_pack(uasd_ctx *c, DevBuf &b, int k, size_t p0, size_t n, const double *a,
-                const double *w, const PackW &pw) {
+                const double *w, const PackW &pw, bool twice = false) {
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
   if (c->prec == UASD_FP64)
     hipLaunchKernelGGL(k_pack<double>, grid, block, 0, c->stream, pair_map(c), p0, n, a, w,
                        pw.from_state ? quads<double>(c, c->spins, 0) : nullptr, pw.value,
-                       quads<double>(c, b, k));
+                       quads<double>(c, b, k), twice ? quads<double>(c, b, k + 1) : nullptr);
   else
     hipLaunchKernelGGL(k_pack<float>, grid, block, 0, c->stream, pair_map(c), p0, n, a, w,
                        pw.from_state ? quads<float>(c, c->spins, 0) : nullptr, pw.value,
-                       quads<float>(c, b, k));
+                       quads<float>(c, b, k), twice ? quads<float>(c, b, k + 1) : nullptr);
   HIP_TRY(hipGetLastError());
   return UASD_OK;
 }
@@ -1280,7 +1283,8 @@ int uasd_ctx_create(uasd_ctx **out, int natom, int mensemble, int precision) {
   if (int r = scratch_init(c->device)) return r;
   HIP_TRY(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
   c->stream = c->own_stream;
-  HIP_TRY(c->spins.ensure(3 * quad_bytes(c.get())));
+  // (b2 has room for the raw doubles of uasd_set_moments in either precision)
+  HIP_TRY(c->spins.ensure(2 * quad_bytes(c.get()) + (size_t)c->N * c->M * 4 * sizeof(double)));
   HIP_TRY(hipMemsetAsync(c->spins.p, 0, 3 * quad_bytes(c.get()), c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   // the whole lattice as one segment until uasd_set_segments says otherwise
@@ -1597,18 +1601,16 @@ int uasd_set_moments(uasd_ctx *c, const double *emom, const double *mmom) {
   if (!emom || !mmom) return fail(UASD_ERR_ARG, "uasd_set_moments: null array");
   HostIo io(c);
   io.open = true;
-  // the raw arrays pass through the memory of the quad arrays 1 and 2 (32 bytes
-  // a pair in either precision), which are written after them: a call that
-  // every program makes once needs no staging of its own
+  // the raw arrays (32 bytes a pair) pass through the memory of b2eff, which
+  // lasts no longer than a step: a call that every program makes once needs no
+  // staging of its own
   const size_t pairs = (size_t)c->N * c->M;
-  double *sa = reinterpret_cast<double *>(static_cast<char *>(c->spins.p) + quad_bytes(c));
+  double *sa = reinterpret_cast<double *>(static_cast<char *>(c->spins.p) + 2 * quad_bytes(c));
   HIP_TRY(hipMemcpyAsync(sa, emom, 3 * pairs * sizeof(double), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(hipMemcpyAsync(sa + 3 * pairs, mmom, pairs * sizeof(double), hipMemcpyHostToDevice,
                          c->stream));
-  if (int r = launch_pack(c, c->spins, 0, 0, pairs, sa, sa + 3 * pairs, PackW{})) return r;
-  HIP_TRY(hipMemcpyAsync(static_cast<char *>(c->spins.p) + quad_bytes(c), c->spins.p,
-                         quad_bytes(c), hipMemcpyDeviceToDevice,
-                         c->stream));  // emom2 starts as emom
+  // emom2 starts as emom
+  if (int r = launch_pack(c, c->spins, 0, 0, pairs, sa, sa + 3 * pairs, PackW{}, true)) return r;
   if (int r = io.wait()) return r;
   c->have_state = true;
   const size_t nm = (size_t)c->N * c->M;
