@@ -99,12 +99,6 @@ struct HamDev {
   // site classes
   const int *__restrict__ cls;
   const SiteClass *__restrict__ classes;
-  // one > 0: every site is of class c0 (a crystal whose basis atoms have the
-  // same couplings), which then comes with the launch.  one = 2: the couplings,
-  // the same for all lanes, are also read through the scalar cache (see
-  // ham_view for where that pays).
-  int one;
-  SiteClass c0;
   // external field: 0 none, 1 uniform per ensemble (ext_u[3*ens+c]), 2 per q
   int ext_mode;
   // 1: neighbour lists are read with non-temporal loads (streamed past L2,
@@ -119,6 +113,12 @@ struct HamDev {
   // reference site, so they do not depend on the order.
   int order_na, order_nc;
   int idx_kb;  // low bits of an int16 list entry holding the basis shift
+  // one > 0: every site is of class c0 (a crystal whose basis atoms have the
+  // same couplings), which then comes with the launch.  one = 2: the couplings,
+  // the same for all lanes, are also read through the scalar cache (see
+  // ham_view for where that pays).
+  int one;
+  SiteClass c0;
 };
 
 template <typename R>
@@ -343,8 +343,8 @@ __device__ __forceinline__ void moment(const Quad<R> *__restrict__ s, size_t q, 
   c = v.z * v.w;
 }
 
-template <typename R>
-__device__ __forceinline__ void uniaxial(const HamDev<R> &h, int row, R m0, R m1, R m2, R &f0,
+template <typename H, typename R>
+__device__ __forceinline__ void uniaxial(const H &h, int row, R m0, R m1, R m2, R &f0,
                                          R &f1, R &f2) {
   R ea0 = h.an_ex[row], ea1 = h.an_ey[row], ea2 = h.an_ez[row];
   R k1 = h.an_k1[row], k2 = h.an_k2[row];
@@ -356,8 +356,8 @@ __device__ __forceinline__ void uniaxial(const HamDev<R> &h, int row, R m0, R m1
   f2 = f2 - tt3 * ea2;
 }
 
-template <typename R>
-__device__ __forceinline__ void cubic(const HamDev<R> &h, int row, R m0, R m1, R m2, R &f0, R &f1,
+template <typename H, typename R>
+__device__ __forceinline__ void cubic(const H &h, int row, R m0, R m1, R m2, R &f0, R &f1,
                                       R &f2) {
   R k1 = h.an_k1[row], k2 = h.an_k2[row];
   R s0 = m0 * m0, s1 = m1 * m1, s2 = m2 * m2;
@@ -850,12 +850,12 @@ struct LLGDev {
   // Philox deviates of a fused step: stored by the predictor, read back by
   // the corrector (the same values it would draw), or nullptr
   Quad<R> *nsave;
-  int nready;  // 1: nsave already holds them (k_draw), the predictor reads them too
   LamConst<R> lc0;       // lam_const(lam0, dt, bn)
   // uniform lam, temperature and moment: the noise amplitudes, computed on
   // the host by the same functions (sig_uniform = 1)
   int sig_uniform;
   R sigk0, sigp0, sigh0;  // midpoint_sigma, depondt_sigma, heun_sigma
+  int nready;  // 1: nsave already holds the deviates (k_draw), the predictor reads them too
   __device__ __forceinline__ LamConst<R> lamc(int s) const {
     return lam ? lam_const<R>(lam[s], dt, bn) : lc0;
   }
@@ -1115,7 +1115,8 @@ struct SiteIn {
 };
 
 // hsite: the site's reference index (the noise counter), q its quad index.
-template <typename R, int ALG, int HALF>
+// AHEAD: the deviates may lie in nsave already (k_draw).
+template <typename R, int ALG, int HALF, bool AHEAD = false>
 __device__ __forceinline__ SiteIn<R> llg_fetch(const LLGDev<R> &prm, int hsite, int ens,
                                                int64_t q, const Quad<R> *e, const Quad<R> *p,
                                                const Quad<R> *b2) {
@@ -1123,7 +1124,7 @@ __device__ __forceinline__ SiteIn<R> llg_fetch(const LLGDev<R> &prm, int hsite, 
   in.eq = e[q];
   if (HALF == 1) in.pq = p[q];
   if ((ALG == 5 || ALG == 4) && HALF == 1) in.bq = b2[q];
-  if ((HALF == 1 || prm.nready) && prm.nsave) {
+  if ((HALF == 1 || (AHEAD && prm.nready)) && prm.nsave) {
     const Quad<R> v = prm.nsave[q];
     in.n0 = v.x;
     in.n1 = v.y;
@@ -1264,7 +1265,8 @@ __device__ __forceinline__ void llg_update(const HamDev<R> &h, const LLGDev<R> &
                                            int ens, int64_t q, R b0, R b1, R b2v,
                                            const Quad<R> *e, Quad<R> *p, Quad<R> *b2,
                                            Quad<R> *out) {
-  const SiteIn<R> in = llg_fetch<R, ALG, HALF>(prm, (int)host_site(h, site), ens, q, e, p, b2);
+  const SiteIn<R> in =
+      llg_fetch<R, ALG, HALF, true>(prm, (int)host_site(h, site), ens, q, e, p, b2);
   llg_apply<R, ALG, HALF>(prm, site, q, b0, b1, b2v, in, p, b2, out);
 }
 
@@ -1351,16 +1353,42 @@ struct TileDev {
   int cls_b[8];
 };
 
+// What the tile kernel needs of the Hamiltonian: the list kernels' fields stay
+// out of its scalar registers, of which it has too few.
+template <typename R>
+struct TileHam {
+  int M, ex_rows, Wd, dm_rows, dm_shared, ext_mode, order_na, order_nc;
+  const int *__restrict__ ex_len;
+  const R *__restrict__ cpl;
+  const int *__restrict__ cls;
+  const SiteClass *__restrict__ classes;
+  const int *__restrict__ dm_len;
+  const R *__restrict__ dvx, *__restrict__ dvy, *__restrict__ dvz;
+  const int *__restrict__ an_type;
+  const R *__restrict__ an_ex, *__restrict__ an_ey, *__restrict__ an_ez;
+  const R *__restrict__ an_k1, *__restrict__ an_k2, *__restrict__ an_sb;
+  const R *__restrict__ ext_u;
+  const Quad<R> *__restrict__ ext_q;
+};
+
+// Offset of the LLGDev argument of k_llg_tile, which follows its TileHam.
+template <typename R>
+constexpr size_t kTilePrmOffset = (sizeof(TileHam<R>) + alignof(LLGDev<R>) - 1) /
+                                  alignof(LLGDev<R>) * alignof(LLGDev<R>);
+
+template <typename R>
+inline TileHam<R> tile_ham(const HamDev<R> &h) {
+  return TileHam<R>{h.M,      h.ex_rows, h.Wd,      h.dm_rows, h.dm_shared, h.ext_mode, h.order_na,
+                    h.order_nc, h.ex_len, h.cpl,    h.cls,     h.classes,   h.dm_len,   h.dvx,
+                    h.dvy,    h.dvz,     h.an_type, h.an_ex,   h.an_ey,     h.an_ez,    h.an_k1,
+                    h.an_k2,  h.an_sb,   h.ext_u,   h.ext_q};
+}
+
 // n / d for 0 <= n < 2^22 and rd = 1/d rounded to FP32: (n + 1/2) rd is
 // within 2^-23 (n + 1/2)/d < 1/(2d) of (n + 1/2)/d, whose fractional part
 // lies in [1/(2d), 1 - 1/(2d)], so the truncation is the exact quotient.
 __device__ __forceinline__ int fdiv(int n, float rd) {
   return (int)(((float)n + 0.5f) * rd);
-}
-
-template <typename R>
-__device__ __forceinline__ int dev_slot(const HamDev<R> &h, int i) {
-  return h.order_na == 1 ? i : (i % h.order_na) * h.order_nc + i / h.order_na;
 }
 
 // Values per component plane of the LDS tile: the launch takes the smallest
@@ -1377,7 +1405,7 @@ constexpr int kTilePlanes[kNumTilePlanes] = {1160, 2312, 3080, 3848};
 // FULL: DM, anisotropy and Zeeman terms may be present; without them the
 // kernel holds fewer launch arguments live (exchange-only Hamiltonians).
 template <typename R, int PL, bool UCLS, bool FULL>
-__device__ __forceinline__ void tile_field(const HamDev<R> &h, const TileDev &t, const R *sm,
+__device__ __forceinline__ void tile_field(const TileHam<R> &h, const TileDev &t, const R *sm,
                                            int hbase, int b, int site, int ens, int64_t q, R &b0,
                                            R &b1, R &b2v) {
   SiteClass sc;
@@ -1541,7 +1569,7 @@ __device__ __forceinline__ void tile_origin(const TileDev &t, int tile, int &X0,
 // multiplicity).  Both terms are scaled by M, so that the sum is the quad
 // index of the slot's ensemble 0 (N*M < 2^31).
 template <typename R>
-__device__ __forceinline__ void halo_table(const HamDev<R> &h, const TileDev &t, int X0, int Y0,
+__device__ __forceinline__ void halo_table(const TileHam<R> &h, const TileDev &t, int X0, int Y0,
                                            int Z0, int ncell, int M, int *tab) {
   const int nr = t.NA * t.HY * t.HZ, hyz = t.HY * t.HZ;
   // wrapped coordinates by the reciprocal divisions (exact: every dividend
@@ -1630,7 +1658,7 @@ __device__ __forceinline__ void halo_rest(const TileDev &t, const int *tab, cons
 // which every unit term folds away at compile time.
 template <typename R, int ALG, int HALF, int PL, bool FULL, bool ENS>
 __global__ void __launch_bounds__(1024)
-    k_llg_tile(HamDev<R> h, LLGDev<R> prm, TileDev t, const Quad<R> *e, Quad<R> *p,
+    k_llg_tile(TileHam<R> h, LLGDev<R> prm, TileDev t, const Quad<R> *e, Quad<R> *p,
                Quad<R> *b2, Quad<R> *out) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   R *sm = reinterpret_cast<R *>(lds_raw);
@@ -1691,8 +1719,17 @@ __global__ void __launch_bounds__(1024)
         tile_field<R, PL, true, FULL>(h, t, sm, hcell, b, site, ens, q, b0, b1, b2v);
       else
         tile_field<R, PL, false, FULL>(h, t, sm, hcell, b, site, ens, q, b0, b1, b2v);
-      const SiteIn<R> in = llg_fetch<R, ALG, HALF>(prm, b + t.NA * cell, ens, q, e, p, b2);
-      llg_apply<R, ALG, HALF>(prm, site, q, b0, b1, b2v, in, p, b2, out);
+      // The solver's parameters are read here, from the argument segment.  As
+      // an ordinary argument the compiler loads all of them at the kernel's
+      // entry and, short of scalar registers, parks them in vector lanes (150
+      // v_readlane, some of them in the exchange loop; 46 this way): headline
+      // step 53.2 -> 51.3 us.
+      typedef const __attribute__((address_space(4))) unsigned char *KArg;
+      KArg ka = (KArg)__builtin_amdgcn_kernarg_segment_ptr() + kTilePrmOffset<R>;
+      asm volatile("" : "+s"(ka));  // not before this point, not hoisted out of the loop
+      const LLGDev<R> &pr = *(const LLGDev<R> *)ka;
+      const SiteIn<R> in = llg_fetch<R, ALG, HALF>(pr, b + t.NA * cell, ens, q, e, p, b2);
+      llg_apply<R, ALG, HALF>(pr, site, q, b0, b1, b2v, in, p, b2, out);
     }
     if (next < 0) break;
     __syncthreads();  // every read of this unit's halo is done

@@ -62,7 +62,7 @@ hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, con
     if (gerr != hipSuccess) return gerr;                                                        \
     const int nwg = (nunits + t.per - 1) / t.per;                                               \
     const dim3 grid((nwg + kXCD - 1) / kXCD * kXCD), block(threads);                            \
-    hipLaunchKernelGGL((k_llg_tile<R, ALG, H, PL, F, E>), grid, block, lds, s, h, prm, t, e, p, b2, \
+    hipLaunchKernelGGL((k_llg_tile<R, ALG, H, PL, F, E>), grid, block, lds, s, tile_ham(h), prm, t, e, p, b2, \
                        out);                                                                    \
     return hipGetLastError();                                                                   \
   }
