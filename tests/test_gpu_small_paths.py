@@ -1,0 +1,123 @@
+"""Paths that a run takes by size or by repetition give the same bits as the
+general ones: deviates drawn ahead, replayed steps and sweeps, a class that
+comes with the launch, couplings through the scalar cache.
+
+Where the path is chosen by size, the reference run joins the system to another
+one that moves the whole lattice to the general path (more sites, or a second
+class of sites): no bond connects the two and random numbers are keyed by the
+site's index, so the first system's trajectory does not change.  Every
+comparison is exact: the arithmetic of a site is the same on both paths."""
+import numpy as np
+import pytest
+
+import uppasd_amd as U
+from uppasd_amd import batch as Bt
+from uppasd_amd import configs as CF
+
+pytestmark = pytest.mark.gpu
+
+
+def _chain(n, J=3.0, mom=1.5):
+    i = np.arange(n)
+    nl = np.stack([(i + 1) % n + 1, (i - 1) % n + 1], axis=1).astype(np.int32)
+    return dict(nlist=nl, nlistsize=np.full(n, 2, np.int32), ncoup=np.full((n, 2), J),
+                mmom=np.full(n, mom))
+
+
+def _run(systems, M, precision, steps, alg, temp=300.0):
+    j = Bt.join(systems)
+    n, N = systems[0]["nlistsize"].shape[0], j.natom
+    eng = Bt.engine_for(j, M, precision)
+    e = CF.random_unit(N, np.random.default_rng(1), M)
+    e[:, :n] = CF.random_unit(n, np.random.default_rng(2), M)
+    eng.set_moments(e, np.broadcast_to(j.mmom, (M, N)))
+    eng.set_llg(0.1, temp, 1e-16)
+    eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+    for k in steps:
+        eng.sd_steps(alg, k)
+    return eng.get_moments()[0][:, :n]
+
+
+@pytest.mark.parametrize("alg", [1, 4, 5, 6, 7])
+@pytest.mark.parametrize("n,M", [(3, 1), (1001, 3), (32768, 1)])
+def test_deviates_drawn_ahead(n, M, alg):
+    """Up to 32,768 FP64 items: 16 steps' deviates in one launch; calls of 1,
+    16, 17 and 5 steps.  The joined run has 33,000 sites more."""
+    steps = (1, 16, 17, 5)
+    a = _run([_chain(n)], M, "fp64", steps, alg)
+    b = _run([_chain(n), _chain(33000)], M, "fp64", steps, alg)
+    assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_repeated_steps_replayed(precision):
+    """After 2048 steps under unchanged settings the rest of a small run is
+    replayed; changed settings start the count again.  Kernel timing keeps the
+    reference run on single launches."""
+    out = []
+    for timed in (False, True):
+        s = CF.bcc_shells((5, 5, 4), [1.34, 0.77], moment=2.2)
+        N = s["lattice"].natom
+        eng = U.Engine(N, 2, precision)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(3), 2), s["mmom"])
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 5)
+        got = []
+        for block in range(26):
+            if timed:
+                eng.set_kernel_timing(True)
+            eng.sd_steps(5, 100)
+            if block == 23:
+                eng.set_llg(0.1, 150.0, 1e-16)
+            got.append(eng.measure(with_energy=True))
+            if block >= 20:
+                got.append((eng.get_moments()[0],))
+        out.append(got)
+    for a, b in zip(*out):
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("mode", ["M", "H"])
+def test_repeated_sweeps_replayed(mode):
+    """The same for sweeps, after 512 of them; 12,000 FP64 sites are more than
+    a resident launch takes."""
+    out, n = [], 12000
+    for timed in (False, True):
+        eng = U.Engine(n, 1)
+        s = _chain(n)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(n, np.random.default_rng(3), 1), s["mmom"])
+        got = []
+        for block in range(24):
+            if timed:
+                eng.set_kernel_timing(True)
+            eng.mc_sweeps(mode, 400.0, 25, 11)
+            got.append(eng.measure(with_energy=True))
+        got.append((eng.get_moments()[0],))
+        out.append(got)
+    for a, b in zip(*out):
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("system,alg", [("bcc", 1), ("film", 5)])
+@pytest.mark.parametrize("size", ["small", "large"])
+def test_one_site_class(system, alg, size, precision):
+    """A crystal of one class, below and above 131,072 sites (from there on its
+    couplings come through the scalar cache), against the same crystal beside a
+    four-site chain of another class."""
+    if system == "bcc":
+        s = CF.bcc_shells((41, 40, 43) if size == "large" else (5, 4, 7), [1.34, 0.77], moment=2.2)
+        other = _chain(4)
+    else:
+        s = CF.triangular_dmi((381, 357, 1) if size == "large" else (9, 7, 1))
+        other = dict(_chain(4), dmlist=np.ones((4, 1), np.int32),
+                     dmlistsize=np.zeros(4, np.int32), dm_vect=np.zeros((4, 1, 3)),
+                     taniso=np.zeros(4, np.int32), eaniso=np.tile([0.0, 0.0, 1.0], (4, 1)),
+                     kaniso=np.zeros((4, 2)), sb=np.zeros(4))
+        other["nlist"] = other["nlist"][:, :2]
+    s = dict(s, mmom=np.full(s["lattice"].natom, 1.5))
+    a = _run([s], 1, precision, (3,), alg)
+    b = _run([s, other], 1, precision, (3,), alg)
+    assert np.array_equal(a, b)

@@ -1179,8 +1179,7 @@ int make_tile(uasd_ctx *c, int k, uasd::TileDev &t) {
 // uasd_energy_terms_noalloc, so that entry point sums in the same order as
 // uasd_energy_terms.  Small chunks fill the chip: calc_energy's terms of
 // 221,184 sites with 58 neighbours took 202 us in 54 chunks of 4096 sites (54
-// workgroups cannot fill 256 CUs); 864 chunks of 256 took 166 us off a pass of
-// field, energy terms and moment sums (1012 -> 846 us, host copies included).
+// workgroups cannot fill 256 CUs) and take 45 us in 864 chunks of 256.
 constexpr int kSegChunkMax = 4096;
 
 int seg_chunk_size(int nseg, const int *off, int M) {
@@ -1861,7 +1860,10 @@ int draw_ahead(uasd_ctx *c, int n, int64_t step_off) {
 // n LLG steps launched one by one; in_graph: inside a capture, counted from
 // the device counter.
 int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
-  const int K = llg_view<double>(c).noise_mode == UASD_NOISE_PHILOX ? steps_ahead(c) : 1;
+  int K = llg_view<double>(c).noise_mode == UASD_NOISE_PHILOX ? steps_ahead(c) : 1;
+  int tile = 0;  // the tile kernels draw their own deviates
+  if (int r = uasd_llg_tile(c, &tile)) return r;
+  if (tile) K = 1;
   for (int64_t s = 0; s < n; ++s) {
     const int k = (int)(s % K);
     const int64_t off = in_graph ? s : -1;
@@ -1885,8 +1887,9 @@ int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
 // 0.4-1.6 us shorter than an enqueued one (its arguments already lie in device
 // memory): 432 sites, 14 neighbours, FP64 13.3 -> 10.3 us a step, FP32 11.9 ->
 // 8.6; 16,000 sites 14.3 -> 11.7; 65,536 sites (film) FP32 14.8 -> 13.0, FP64
-// 16.7 -> 15.6; nothing from 2^18 items on.  Capturing costs about a
-// millisecond, hence `after`.
+// 16.7 -> 15.6; nothing from 2^18 items on.  Capturing costs 25 us a launch
+// (4 ms for 80 steps), which 2048 steps or 512 sweeps would have repaid, hence
+// `after`.
 bool repeats_pay(uasd_ctx *c, int kind, int alg, uint64_t seed, int64_t items, int64_t n,
                  int64_t after) {
   if (c->graph_steps > 0 || c->timing || items > 131072) return false;
@@ -1915,7 +1918,7 @@ int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps) {
   };
   if (c->graph_steps > 0) {
     if (int r = replay(c->graph_steps)) return r;
-  } else if (repeats_pay(c, 0, alg, 0, (int64_t)c->N * c->M, nsteps, 512)) {
+  } else if (repeats_pay(c, 0, alg, 0, (int64_t)c->N * c->M, nsteps, 2048)) {
     for (int K : {64, 16})
       if (int r = replay(K)) return r;
   }
@@ -2203,10 +2206,10 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
           g.site0 = c->color_start[col];
           g.sstride = c->color_stride[col];
           if (c->prec == UASD_FP64) {
-            HIP_TRY(uasd::launch_mc<double>(c->stream, mc_tune(c, mp.nsites), ham_view<double>(c), g,
+            HIP_TRY(uasd::launch_mc<double>(c->stream, mc_tune(c, g.nsites), ham_view<double>(c), g,
                                             quads<double>(c, c->spins, 0)));
           } else {
-            HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, mp.nsites), ham_view<float>(c), g,
+            HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, g.nsites), ham_view<float>(c), g,
                                            quads<float>(c, c->spins, 0)));
           }
         }
@@ -2224,7 +2227,7 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
     if (int r = replay(c->graph_steps)) return r;
   } else if (!mc_use_resident(c) &&
              repeats_pay(c, 1, mode, seed, (int64_t)c->N * c->M / std::max(c->ncolors, 1),
-                         nsweeps, 64)) {
+                         nsweeps, 512)) {
     for (int K : {16, 4})
       if (int r = replay(K)) return r;
   }
@@ -2380,8 +2383,6 @@ int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool 
   HIP_TRY(hipEventCreate(&ev.b));
   const int gathers[] = {2, 4, 8, 16};
   const int blocks[] = {64, 128, 256};
-  uasd::Tune best = *slot;
-  float best_t = 1e30f;
   std::vector<uasd::Tune> cand;
   const int nidx = c->use16 || c->use16_dm ? 2 : 1;
   for (int ix = 0; ix < nidx; ++ix)
@@ -2397,21 +2398,38 @@ int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool 
       if (tile_fits(c, k))
         for (int pipe = 0; pipe < 2; ++pipe) cand.push_back(uasd::Tune{4, 256, 0, 0, k, pipe});
   }
-  for (const uasd::Tune &cd : cand) {
-    {
-      *slot = cd;
-      slot->chosen = 1;
+  // one timed run each, then the fastest few again over several runs: a single
+  // run of a small lattice (tens of us) ranks shapes within its own scatter
+  auto timed = [&](const uasd::Tune &cd, int reps, float &ms) -> int {
+    *slot = cd;
+    slot->chosen = 1;
+    if (int r = run()) return r;
+    HIP_TRY(hipEventRecord(ev.a, c->stream));
+    for (int k = 0; k < reps; ++k)
       if (int r = run()) return r;
-      HIP_TRY(hipEventRecord(ev.a, c->stream));
-      if (int r = run()) return r;
-      HIP_TRY(hipEventRecord(ev.b, c->stream));
-      HIP_TRY(hipEventSynchronize(ev.b));
-      float ms = 0.f;
-      HIP_TRY(hipEventElapsedTime(&ms, ev.a, ev.b));
-      if (ms < best_t) {
-        best_t = ms;
-        best = *slot;
-      }
+    HIP_TRY(hipEventRecord(ev.b, c->stream));
+    HIP_TRY(hipEventSynchronize(ev.b));
+    HIP_TRY(hipEventElapsedTime(&ms, ev.a, ev.b));
+    ms /= (float)reps;
+    return UASD_OK;
+  };
+  std::vector<std::pair<float, int>> rank;
+  for (size_t i = 0; i < cand.size(); ++i) {
+    float ms = 0.f;
+    if (int r = timed(cand[i], 1, ms)) return r;
+    rank.emplace_back(ms, (int)i);
+  }
+  std::sort(rank.begin(), rank.end());
+  constexpr int kFinal = 5, kReps = 6;
+  uasd::Tune best = cand[rank[0].second];
+  best.chosen = 1;
+  float best_t = 1e30f;
+  for (int k = 0; k < kFinal && k < (int)rank.size(); ++k) {
+    float ms = 0.f;
+    if (int r = timed(cand[rank[k].second], kReps, ms)) return r;
+    if (ms < best_t) {
+      best_t = ms;
+      best = *slot;
     }
   }
   *slot = best;
