@@ -145,7 +145,10 @@ int uasd_sd_steps(uasd_ctx *ctx, int sdealgh, int64_t nsteps);
  * launches to capture): with steps_per_graph = K > 0, uasd_sd_steps and
  * uasd_mc_sweeps replay a hipGraph of K steps (K sweeps) for every full run of
  * K, and launch the rest one by one; the numbers are the same either way.
- * The Philox counters then advance on the device.  0 (the default) disables. */
+ * The Philox counters then advance on the device.  0 (the default) leaves it
+ * to the library, which replays the steps or sweeps of small systems once
+ * enough of them have run under unchanged settings (not while kernels are
+ * timed or the stream is being captured). */
 int uasd_set_graph_steps(uasd_ctx *ctx, int steps_per_graph);
 /* Field of the resident moments into a host array (NULL skips the copy). */
 int uasd_effective_field(uasd_ctx *ctx, double *beff, double *energy);
@@ -206,7 +209,8 @@ int uasd_get_coloring(uasd_ctx *ctx, int *ncolors, int *color_of_site);
  * timing off.  Events between kernels cost time of their own, so a sampled
  * run keeps the stream close to an untimed one. */
 int uasd_set_kernel_timing(uasd_ctx *ctx, int enable);
-/* kind: 0 predictor, 1 corrector, 2 field, 3 MC colour pass, 4 LLG graph
+/* kind: 0 predictor, 1 corrector, 2 field, 3 MC colour pass (small systems:
+ * one resident launch of all sweeps of a call), 4 LLG graph
  * replay (K steps), 5 MC graph replay (K sweeps), 6 a whole uasd_sd_steps or
  * uasd_mc_sweeps call */
 int uasd_get_kernel_timing(uasd_ctx *ctx, int kind, int64_t *launches, double *total_ms);

@@ -250,7 +250,7 @@ class Engine:
         return k.value
 
     def set_graph_steps(self, k: int):
-        """Replay hipGraphs of k LLG steps / MC sweeps (0 = launch one by one)."""
+        """Replay hipGraphs of k LLG steps / MC sweeps (0 = left to the library)."""
         B.check(B.lib().uasd_set_graph_steps(self._h, int(k)), "uasd_set_graph_steps")
 
     # --------------------------------------------------------------- batches
