@@ -1,6 +1,6 @@
 """Paths that a run takes by size or by repetition give the same bits as the
 general ones: deviates drawn ahead, replayed steps and sweeps, a class that
-comes with the launch, couplings through the scalar cache.
+comes with the launch, couplings through the scalar cache, resident steps.
 
 Where the path is chosen by size, the reference run joins the system to another
 one that moves the whole lattice to the general path (more sites, or a second
@@ -56,7 +56,7 @@ def test_repeated_steps_replayed(precision):
     reference run on single launches."""
     out = []
     for timed in (False, True):
-        s = CF.bcc_shells((5, 5, 4), [1.34, 0.77], moment=2.2)
+        s = CF.bcc_shells((7, 7, 7), [1.34, 0.77], moment=2.2)    # 686: not resident
         N = s["lattice"].natom
         eng = U.Engine(N, 2, precision)
         eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
@@ -121,3 +121,69 @@ def test_one_site_class(system, alg, size, precision):
     a = _run([s], 1, precision, (3,), alg)
     b = _run([s, other], 1, precision, (3,), alg)
     assert np.array_equal(a, b)
+
+
+def _film(L):
+    s = CF.triangular_dmi(L)
+    N, rng = s["lattice"].natom, np.random.default_rng(3)
+    s["taniso"] = rng.choice([0, 1, 2, 7], size=N).astype(np.int32)   # every anisotropy on the path
+    s["eaniso"], s["kaniso"] = CF.random_unit(N, rng)[0], rng.normal(size=(N, 2))
+    s["sb"] = rng.normal(size=N)
+    return s
+
+
+RESIDENT = {
+    "sites1": lambda: _chain(1, J=0.0),
+    "sites511": lambda: _chain(511),
+    "sites512": lambda: _chain(512),
+    "shells5": lambda: CF.bcc_shells((5, 6, 7), CF.bcc5_couplings(), moment=2.2),
+    "film": lambda: _film((13, 11, 1)),
+}
+
+
+@pytest.mark.parametrize("noise", ["philox", "injected", "none"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("name", list(RESIDENT))
+def test_resident_steps_equal_launched_ones(name, precision, noise):
+    """Systems of up to 512 sites, stepped by one workgroup each, alone, twice
+    over and beside a chain of 66,000 sites (more than the resident path looks
+    through, so that run launches every half step), with a per-site external
+    field and calls of 1, 70 and 3 steps."""
+    small, M = RESIDENT[name](), 2
+    n = small["nlistsize"].shape[0]
+    rng = np.random.default_rng(23)
+    e0, ext0, nrm0 = CF.random_unit(n, rng, M), rng.normal(size=(M, n, 3)) * 30.0, rng.normal(size=(M, n, 3))
+    out = []
+    for systems in ([small], [small, small], [small, _chain(66000)]):
+        systems = [dict(s) for s in systems]
+        for s in systems if "dmlist" in small else ():
+            k = s["nlistsize"].shape[0]
+            for key, v in (("dmlist", np.ones((k, 1), np.int32)), ("dmlistsize", np.zeros(k, np.int32)),
+                           ("dm_vect", np.zeros((k, 1, 3))), ("taniso", np.zeros(k, np.int32)),
+                           ("eaniso", np.tile([0.0, 0.0, 1.0], (k, 1))), ("kaniso", np.zeros((k, 2))),
+                           ("sb", np.zeros(k))):
+                s.setdefault(key, v)
+        j = Bt.join(systems)
+        N = j.natom
+        eng = Bt.engine_for(j, M, precision)
+
+        def pad(a, fill):
+            full = np.broadcast_to(np.asarray(fill, dtype=np.float64), (M, N, 3)).copy()
+            full[:, :n] = a
+            return full
+        eng.set_moments(pad(e0, [0.0, 0.0, 1.0]), np.broadcast_to(j.mmom, (M, N)))
+        eng.set_external_field(pad(ext0, [0.0, 0.0, 5.0]))
+        eng.set_llg(0.1, 200.0, 1e-16)
+        if noise == "injected":
+            eng.set_noise(U.UASD_NOISE_INJECTED, 0, pad(nrm0, 0.0))
+        else:
+            eng.set_noise(U.UASD_NOISE_PHILOX if noise == "philox" else U.UASD_NOISE_NONE, 9)
+        got = []
+        for alg in (1, 5, 4):
+            for k in (1, 70, 3):
+                eng.sd_steps(alg, k)
+            got.append(eng.get_moments()[0][:, :n])
+        out.append(got)
+    for k in range(3):
+        assert np.array_equal(out[0][k], out[2][k]), (name, k)
+        assert np.array_equal(out[1][k], out[2][k]), (name, k)

@@ -268,7 +268,7 @@ struct uasd_ctx {
     uasd::ResDev dev{};
     int64_t cls_version = -1;
     int64_t col_version = -1;
-  } res;
+  } res, lres;  // for MC sweeps (colour order), for LLG steps (device order)
   int64_t col_version = 0;  // bumped by every colouring rebuild
 
   // Per-kernel timing: an event pair is recorded around each launch without
@@ -788,6 +788,96 @@ uasd::LLGDev<R> llg_view(uasd_ctx *c) {
     p.sigh0 = uasd::heun_sigma<R>(p.lc0.Dh, m, c->temp0, c->temprescale, c->dt);
   }
   return p;
+}
+
+// Contiguous ranges of device slots that no bond crosses, as first slots.
+std::vector<int> independent_ranges(const uasd_ctx *c) {
+  const int N = c->N;
+  std::vector<int> reach(N);  // furthest slot bonded to slot i or to one before it
+  auto add = [&](const std::vector<int> &row, const std::vector<int> &len,
+                 const std::vector<int> &nb, int W) {
+    if (W == 0 || row.empty()) return;
+    for (int j = 0; j < W; ++j)
+      for (int i = 0; i < N; ++i)
+        if (j < len[row[i]]) {
+          const int n = nb[(size_t)j * N + i];
+          reach[std::min(i, n)] = std::max(reach[std::min(i, n)], std::max(i, n));
+        }
+  };
+  for (int i = 0; i < N; ++i) reach[i] = i;
+  add(c->ex_row_of_site, c->ex_len_host, c->nbr_host, c->W);
+  add(c->dm_row_of_site, c->dm_len_host, c->dnbr_host, c->Wd);
+  std::vector<int> off(1, 0);
+  for (int i = 0, far = 0; i < N; ++i) {
+    far = std::max(far, reach[i]);
+    if (far == i) off.push_back(i + 1);
+  }
+  return off;
+}
+
+// Builds c->lres, the systems of the lattice for resident LLG steps, where
+// they are small enough for them.  Lattices over kLlgResLattice sites are not
+// looked through: their batches fill the chip with the other kernels.
+constexpr int kLlgResSites = uasd::kResThreads, kLlgResLattice = 65536;
+
+int build_llg_resident(uasd_ctx *c) {
+  auto &r = c->lres;
+  if (r.cls_version == c->cls_version) return UASD_OK;
+  r.ok = false;
+  r.cls_version = c->cls_version;
+  const int N = c->N, W = c->W, Wd = c->Wd;
+  if (N > kLlgResLattice) return UASD_OK;
+  const std::vector<int> off = independent_ranges(c);
+  const int ncomp = (int)off.size() - 1;
+  int nmax = 0;
+  for (int k = 0; k < ncomp; ++k) nmax = std::max(nmax, off[k + 1] - off[k]);
+  if (nmax > kLlgResSites || uasd::res_lds_llg(c->rsize, nmax) > (size_t)c->lds_max)
+    return UASD_OK;
+  std::vector<uint16_t> nb((size_t)(W + Wd) * N);
+  for (int k = 0; k < ncomp; ++k)
+    for (int i = off[k]; i < off[k + 1]; ++i) {
+      for (int j = 0; j < W; ++j)
+        nb[(size_t)j * N + i] = (uint16_t)(c->nbr_host[(size_t)j * N + i] - off[k]);
+      for (int j = 0; j < Wd; ++j)
+        nb[(size_t)(W + j) * N + i] = (uint16_t)(c->dnbr_host[(size_t)j * N + i] - off[k]);
+    }
+  std::vector<uasd::SiteClass> cls(N);
+  for (int i = 0; i < N; ++i)
+    cls[i] = uasd::SiteClass{c->ex_row_of_site.empty() ? 0 : c->ex_row_of_site[i],
+                             c->dm_row_of_site.empty() ? -1 : c->dm_row_of_site[i],
+                             c->an_row_of_site.empty() ? -1 : c->an_row_of_site[i], 0};
+  std::vector<char> all(cls.size() * sizeof(cls[0]) + off.size() * sizeof(int) +
+                        nb.size() * sizeof(uint16_t));
+  const size_t ooff = cls.size() * sizeof(cls[0]), onb = ooff + off.size() * sizeof(int);
+  std::memcpy(all.data(), cls.data(), ooff);
+  std::memcpy(all.data() + ooff, off.data(), off.size() * sizeof(int));
+  std::memcpy(all.data() + onb, nb.data(), nb.size() * sizeof(uint16_t));
+  if (int e = upload_raw(c, r.buf, all)) return e;
+  const char *base = r.buf.as<char>();
+  r.dev = uasd::ResDev{};
+  r.dev.ncomp = ncomp;
+  r.dev.nmax = nmax;
+  r.dev.off = reinterpret_cast<const int *>(base + ooff);
+  r.dev.cls = reinterpret_cast<const uasd::SiteClass *>(base);
+  r.dev.nbr = reinterpret_cast<const uint16_t *>(base + onb);
+  r.dev.dnbr = r.dev.nbr + (size_t)W * N;
+  r.ncomp = ncomp;
+  r.nmax = nmax;
+  r.ok = true;
+  return UASD_OK;
+}
+
+// Whether a call's LLG steps run in k_llg_resident: systems of at most one
+// site per thread of its workgroup.  Per step, two launches -> resident, FP64
+// (FP32), one ensemble: 128 sites, 14 neighbours 9.7 -> 3.6 us (10.6 -> 3.3),
+// 432 sites 11.3 -> 5.0 (11.3 -> 3.8), Depondt 12.4 -> 5.8, 58 neighbours 22.8
+// -> 11.3 (18.2 -> 7.5), SIB 17.1 -> 12.9; 64 ensembles of 432 sites 13.1 ->
+// 6.5.  With 1024 sites the one CU is as slow as the launches (58 neighbours
+// 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  Not while the kernels
+// are timed one by one or graphs were asked for.
+bool llg_use_resident(const uasd_ctx *c) {
+  return c->lres.ok && c->lres.cls_version == c->cls_version && !c->timing &&
+         c->graph_steps == 0 && (int64_t)c->N * c->M <= 131072;
 }
 
 // Steps whose Philox deviates are drawn in one launch ahead of them.  FP64
@@ -1903,7 +1993,40 @@ bool repeats_pay(uasd_ctx *c, int kind, int alg, uint64_t seed, int64_t items, i
   return r.second - n >= after;
 }
 
+// nsteps steps in resident launches of 4 to 64, as many as deviates of 2^18
+// items cover.
+template <typename R>
+int llg_resident_steps(uasd_ctx *c, int alg, int64_t nsteps) {
+  const bool philox = llg_view<R>(c).noise_mode == UASD_NOISE_PHILOX;
+  const int64_t chunk =
+      std::max<int64_t>(4, std::min<int64_t>(64, 262144 / ((int64_t)c->N * c->M)));
+  if (philox) {
+    const int64_t most = std::min(chunk, nsteps);
+    void *old = c->nsave.p;
+    HIP_TRY(c->nsave.ensure((size_t)most * quad_bytes(c)));
+    if (c->nsave.p != old) c->gen += 1;
+  }
+  for (int64_t s = 0; s < nsteps; s += chunk) {
+    const int n = (int)std::min(chunk, nsteps - s);
+    if (philox)
+      if (int r = draw_ahead<R>(c, n, -1)) return r;
+    uasd::LLGDev<R> prm = llg_view<R>(c);
+    if (philox) prm.nsave = quads<R>(c, c->nsave);
+    HIP_TRY(uasd::launch_llg_resident<R>(c->stream, alg, ham_view<R>(c), prm, c->lres.dev, n,
+                                         (size_t)c->lds_max, quads<R>(c, c->spins, 0)));
+    c->step += (uint64_t)n;
+  }
+  return UASD_OK;
+}
+
 int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;  // a caller's own capture:
+  (void)hipStreamIsCapturing(c->stream, &cap);              // no tables, no growing buffers
+  if (cap == hipStreamCaptureStatusNone)
+    if (int r = build_llg_resident(c)) return r;
+  if (cap == hipStreamCaptureStatusNone && llg_use_resident(c))
+    return c->prec == UASD_FP64 ? llg_resident_steps<double>(c, alg, nsteps)
+                                : llg_resident_steps<float>(c, alg, nsteps);
   int64_t s = 0;
   auto replay = [&](int K) -> int {
     auto body = [&]() -> int {
@@ -1949,31 +2072,6 @@ int uasd_effective_field(uasd_ctx *c, double *beff, double *energy) {
     *energy = e * uasd::kMub / uasd::kMry;
   }
   return io.wait();
-}
-
-// Contiguous ranges of device slots that no bond crosses, as first slots.
-static std::vector<int> independent_ranges(const uasd_ctx *c) {
-  const int N = c->N;
-  std::vector<int> reach(N);  // furthest slot bonded to slot i or to one before it
-  auto add = [&](const std::vector<int> &row, const std::vector<int> &len,
-                 const std::vector<int> &nb, int W) {
-    if (W == 0 || row.empty()) return;
-    for (int j = 0; j < W; ++j)
-      for (int i = 0; i < N; ++i)
-        if (j < len[row[i]]) {
-          const int n = nb[(size_t)j * N + i];
-          reach[std::min(i, n)] = std::max(reach[std::min(i, n)], std::max(i, n));
-        }
-  };
-  for (int i = 0; i < N; ++i) reach[i] = i;
-  add(c->ex_row_of_site, c->ex_len_host, c->nbr_host, c->W);
-  add(c->dm_row_of_site, c->dm_len_host, c->dnbr_host, c->Wd);
-  std::vector<int> off(1, 0);
-  for (int i = 0, far = 0; i < N; ++i) {
-    far = std::max(far, reach[i]);
-    if (far == i) off.push_back(i + 1);
-  }
-  return off;
 }
 
 // Builds c->res for the current lists, classes and colouring.

@@ -2295,6 +2295,110 @@ __global__ void __launch_bounds__(kResThreads, !HB && sizeof(R) == 4 ? 4 : 2)
   for (int p = tid; p < n; p += T) s[(size_t)rd.site[off + p] * M + ens] = sp[p];
 }
 
+// ------------------------------------------------ resident LLG of small systems
+// The same for the LLG step: one workgroup per (independent system, ensemble)
+// with e, the predicted moments, b2eff and the lists in LDS, all steps of a
+// call in one launch, two barriers a step instead of two launches.  Philox
+// deviates come from k_draw (nsave, quad array k for the k-th step of the
+// launch): drawn here they would keep the one CU busy for longer than the step
+// itself.  A site's arithmetic is that of k_llg.  Positions are device slots
+// counted from the system's first.
+//
+// What bounds it: instruction issue of one CU, hence the limit on the sites of
+// a system (llg_use_resident).
+template <typename R, int ALG, bool LNB>
+__global__ void __launch_bounds__(kResThreads)
+    k_llg_resident(HamDev<R> h, LLGDev<R> prm, ResDev rd, int nsteps, Quad<R> *s) {
+  constexpr int G = 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds_res[];
+  Quad<R> *el = reinterpret_cast<Quad<R> *>(lds_res);
+  Quad<R> *pl = el + rd.nmax, *bl = pl + rd.nmax;
+  uint16_t *lnb = reinterpret_cast<uint16_t *>(bl + rd.nmax);
+  const int M = h.M, W = h.W, Wd = h.Wd, N = h.N;
+  const int comp = blockIdx.x / M, ens = blockIdx.x - comp * M;
+  const int off = rd.off[comp], n = rd.off[comp + 1] - off;
+  const int tid = threadIdx.x, T = blockDim.x;
+  for (int p = tid; p < n; p += T) el[p] = s[(size_t)(off + p) * M + ens];
+  if (LNB) {
+    for (int j = 0; j < W; ++j)
+      for (int p = tid; p < n; p += T) lnb[j * n + p] = rd.nbr[(size_t)j * N + off + p];
+    for (int j = 0; j < Wd; ++j)
+      for (int p = tid; p < n; p += T) lnb[(W + j) * n + p] = rd.dnbr[(size_t)j * N + off + p];
+  }
+  HamDev<R> lh = h;  // the lists as the gathers see them: one ensemble, stride lh.N
+  lh.M = 1;
+  lh.N = LNB ? n : N;
+  const uint16_t *nb = LNB ? lnb : rd.nbr + off;
+  const uint16_t *dnb = LNB ? lnb + W * n : rd.dnbr + off;
+  __syncthreads();
+  // the field of the moments src at position p
+  auto field = [&](const Quad<R> *src, int p, R &b0, R &b1, R &b2v) {
+    const SiteClass sc = h.one ? h.c0 : rd.cls[off + p];
+    const int len = h.ex_full ? W : h.ex_len[sc.ex_row];
+    R f[1][3] = {{(R)0, (R)0, (R)0}}, qf[3] = {(R)0, (R)0, (R)0}, x[3] = {(R)0, (R)0, (R)0};
+    exchange_run<R, G, false, uint16_t, 1, false, NbDecId>(lh, nb + p, src, p, 0, sc.ex_row, len,
+                                                           f);
+    if (Wd > 0 && sc.dm_row >= 0)
+      dm_sum<R, G, uint16_t, NbDecId>(lh, dnb + p, src, p, 0, sc.dm_row, f[0][0], f[0][1],
+                                      f[0][2]);
+    anisotropy(h, sc, src, (size_t)p, f[0], qf);
+    if (h.ext_mode == 1) {
+      x[0] = h.ext_u[3 * ens];
+      x[1] = h.ext_u[3 * ens + 1];
+      x[2] = h.ext_u[3 * ens + 2];
+    } else if (h.ext_mode == 2) {
+      const Quad<R> v = h.ext_q[(size_t)(off + p) * M + ens];
+      x[0] = v.x;
+      x[1] = v.y;
+      x[2] = v.z;
+    }
+    b0 = (R)0 + f[0][0] + (qf[0] + x[0] + (R)0);
+    b1 = (R)0 + f[0][1] + (qf[1] + x[1] + (R)0);
+    b2v = (R)0 + f[0][2] + (qf[2] + x[2] + (R)0);
+  };
+  const size_t total = (size_t)N * M;
+  for (int k = 0; k < nsteps; ++k) {
+    const Quad<R> *drawn = prm.nsave ? prm.nsave + (size_t)k * total : nullptr;
+    auto deviates = [&](int p, SiteIn<R> &in) {
+      const size_t q = (size_t)(off + p) * M + ens;
+      if (drawn) {
+        const Quad<R> v = drawn[q];
+        in.n0 = v.x;
+        in.n1 = v.y;
+        in.n2 = v.z;
+      } else if (prm.noise_mode == 2) {
+        const Quad<R> v = prm.noise[q];
+        in.n0 = v.x;
+        in.n1 = v.y;
+        in.n2 = v.z;
+      } else {
+        in.n0 = in.n1 = in.n2 = (R)0;
+      }
+    };
+    for (int p = tid; p < n; p += T) {
+      SiteIn<R> in;
+      deviates(p, in);
+      in.eq = el[p];
+      R b0, b1, b2v;
+      field(el, p, b0, b1, b2v);
+      llg_apply<R, ALG, 0>(prm, off + p, p, b0, b1, b2v, in, pl, bl, pl);
+    }
+    __syncthreads();
+    for (int p = tid; p < n; p += T) {
+      SiteIn<R> in;
+      deviates(p, in);
+      in.eq = el[p];
+      in.pq = pl[p];
+      if (ALG == 5 || ALG == 4) in.bq = bl[p];
+      R b0, b1, b2v;
+      field(pl, p, b0, b1, b2v);
+      llg_apply<R, ALG, 1>(prm, off + p, p, b0, b1, b2v, in, pl, bl, el);
+    }
+    __syncthreads();
+  }
+  for (int p = tid; p < n; p += T) s[(size_t)(off + p) * M + ens] = el[p];
+}
+
 // ---------------------------------------------------------- FP64 reductions
 // The measurement sums are short: what bounds them is how many workgroups they
 // fill the chip with and the length of their serial chains, not memory.  A

@@ -127,6 +127,40 @@ hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCP
   });
 }
 
+template <typename R, int ALG, bool LNB>
+static hipError_t llg_resident_one(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm,
+                                   const ResDev &rd, int nsteps, size_t bytes, int threads,
+                                   Quad<R> *spins) {
+  const hipError_t err = hipFuncSetAttribute((const void *)&k_llg_resident<R, ALG, LNB>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)bytes);
+  if (err != hipSuccess) return err;
+  hipLaunchKernelGGL((k_llg_resident<R, ALG, LNB>), dim3((unsigned)(rd.ncomp * h.M)),
+                     dim3(threads), bytes, s, h, prm, rd, nsteps, spins);
+  return hipGetLastError();
+}
+
+template <typename R>
+hipError_t launch_llg_resident(hipStream_t s, int alg, const HamDev<R> &h, const LLGDev<R> &prm,
+                               const ResDev &rd, int nsteps, size_t lds, Quad<R> *spins) {
+  const size_t base = res_lds_llg(sizeof(R), rd.nmax), lists = 2 * (size_t)rd.nmax * (h.W + h.Wd);
+  if (base > lds || nsteps <= 0) return hipErrorInvalidValue;
+  const bool lnb = base + lists <= lds;
+  const size_t bytes = base + (lnb ? lists : 0);
+  const int threads = std::min(kResThreads, (rd.nmax + 63) / 64 * 64);
+#define UASD_RES_CASE(A)                                                                       \
+  if (alg == A)                                                                                \
+    return lnb ? llg_resident_one<R, A, true>(s, h, prm, rd, nsteps, bytes, threads, spins)    \
+               : llg_resident_one<R, A, false>(s, h, prm, rd, nsteps, bytes, threads, spins);
+  UASD_RES_CASE(1)
+  UASD_RES_CASE(4)
+  UASD_RES_CASE(5)
+  UASD_RES_CASE(6)
+  UASD_RES_CASE(7)
+#undef UASD_RES_CASE
+  return hipErrorInvalidValue;
+}
+
 template <typename R, bool HB, bool TRL, bool LNB>
 static hipError_t mc_resident_one(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
                                   const ResDev &rd, int nsweeps, size_t bytes, int threads,
@@ -267,6 +301,9 @@ hipError_t launch_energy_terms(hipStream_t s, const HamDev<R> &h, int nseg, int 
                                      Quad<R> *);                                              \
   template hipError_t launch_mc<R>(hipStream_t, const Tune &, const HamDev<R> &,              \
                                    const MCParams &, Quad<R> *);                              \
+  template hipError_t launch_llg_resident<R>(hipStream_t, int, const HamDev<R> &,             \
+                                             const LLGDev<R> &, const ResDev &, int, size_t,  \
+                                             Quad<R> *);                                      \
   template hipError_t launch_mc_resident<R>(hipStream_t, const HamDev<R> &, const MCParams &,  \
                                             const ResDev &, int, size_t, Quad<R> *, Quad<R> *); \
   template hipError_t launch_llg_tile<R>(hipStream_t, TileDev, int, int, int,              \

@@ -86,6 +86,15 @@ hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fuse
                       const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p,
                       Quad<R> *b2, const Quad<R> *beff, Quad<R> *out);
 
+// nsteps LLG steps of every system with k_llg_resident; Philox deviates in
+// prm.nsave, lds = LDS bytes a workgroup may use.
+template <typename R>
+hipError_t launch_llg_resident(hipStream_t s, int alg, const HamDev<R> &h, const LLGDev<R> &prm,
+                               const ResDev &rd, int nsteps, size_t lds, Quad<R> *spins);
+
+// LDS of k_llg_resident without its lists: e, p and b2 quads.
+inline size_t res_lds_llg(size_t rsize, int nmax) { return 12 * rsize * (size_t)nmax; }
+
 // Deviates of `steps` steps from prm.step on into as many quad arrays of out.
 template <typename R>
 hipError_t launch_draw(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
