@@ -146,8 +146,8 @@ RESIDENT = {
 @pytest.mark.parametrize("name", list(RESIDENT))
 def test_resident_steps_equal_launched_ones(name, precision, noise):
     """Systems of up to 512 sites, stepped by one workgroup each, alone, twice
-    over and beside a chain of 66,000 sites (more than the resident path looks
-    through, so that run launches every half step), with a per-site external
+    over and beside a chain of 66,000 sites (more than the resident path takes, so
+    that run launches every half step), with a per-site external
     field and calls of 1, 70 and 3 steps."""
     small, M = RESIDENT[name](), 2
     n = small["nlistsize"].shape[0]

@@ -818,7 +818,7 @@ std::vector<int> independent_ranges(const uasd_ctx *c) {
 // Builds c->lres, the systems of the lattice for resident LLG steps, where
 // they are small enough for them.  Lattices over kLlgResLattice sites are not
 // looked through: their batches fill the chip with the other kernels.
-constexpr int kLlgResSites = uasd::kResThreads, kLlgResLattice = 65536;
+constexpr int kLlgResSites = uasd::kResThreads, kLlgResLattice = 16384;
 
 int build_llg_resident(uasd_ctx *c) {
   auto &r = c->lres;
@@ -827,6 +827,18 @@ int build_llg_resident(uasd_ctx *c) {
   r.cls_version = c->cls_version;
   const int N = c->N, W = c->W, Wd = c->Wd;
   if (N > kLlgResLattice) return UASD_OK;
+  // a bond that spans more sites than a system may have ends the search, in a
+  // periodic crystal with its first site's
+  auto spans = [&](const std::vector<int> &row, const std::vector<int> &len,
+                   const std::vector<int> &list) {
+    for (int i = 0; i < N && !row.empty(); ++i)
+      for (int j = 0; row[i] >= 0 && j < len[row[i]]; ++j)
+        if (std::abs(list[(size_t)j * N + i] - i) >= kLlgResSites) return true;
+    return false;
+  };
+  if (spans(c->ex_row_of_site, c->ex_len_host, c->nbr_host) ||
+      (Wd > 0 && spans(c->dm_row_of_site, c->dm_len_host, c->dnbr_host)))
+    return UASD_OK;
   const std::vector<int> off = independent_ranges(c);
   const int ncomp = (int)off.size() - 1;
   int nmax = 0;
