@@ -111,3 +111,14 @@ def test_resident_sweeps_equal_launched_ones(name, mode, precision):
         out.append(eng.get_moments()[0][:, :n])
     assert np.array_equal(out[0], out[1]), name
     assert np.array_equal(out[2], out[1]), name
+
+
+@pytest.mark.parametrize("mode", ["M", "H"])
+def test_resident_fp32_trials_beyond_lds(mode):
+    """8192 FP32 sites of 16 colours: the spins alone fill the LDS, the trial
+    moves and the lists stay in global memory."""
+    SYSTEMS["sites8192"] = lambda: _crystal((16, 16, 16), CF.bcc5_couplings())
+    try:
+        test_resident_sweeps_equal_launched_ones("sites8192", mode, "fp32")
+    finally:
+        del SYSTEMS["sites8192"]
