@@ -1,0 +1,70 @@
+"""Contexts on several threads: different contexts may be used at the same
+time, whatever launch limits their kernels share.
+
+The dynamic LDS limit of a kernel belongs to the process, so a context whose
+systems need little LDS must not take it from one whose systems need much."""
+import threading
+
+import numpy as np
+import pytest
+
+import uppasd_amd as U
+from uppasd_amd import configs as CF
+
+pytestmark = pytest.mark.gpu
+
+
+def _in_threads(jobs):
+    """Runs every job in a thread of its own, all at once; results in order."""
+    out, errs = [None] * len(jobs), []
+    start = threading.Barrier(len(jobs))
+
+    def go(k):
+        try:
+            start.wait()
+            out[k] = jobs[k]()
+        except Exception as ex:   # reported by the test's own thread
+            errs.append(ex)
+    ts = [threading.Thread(target=go, args=(k,)) for k in range(len(jobs))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not errs, errs
+    return out
+
+
+def _engine(L, shells):
+    s = CF.bcc_shells(L, shells, moment=2.2)
+    N = s["lattice"].natom
+    eng = U.Engine(N, 1)
+    eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+    eng.set_moments(CF.random_unit(N, np.random.default_rng(N), 1), s["mmom"][None])
+    eng.set_llg(0.1, 300.0, 1e-16)
+    eng.set_noise(U.UASD_NOISE_PHILOX, 5)
+    return eng
+
+
+def _sweeps(L):
+    eng = _engine(L, [1.34, 0.77])
+    for _ in range(150):
+        eng.mc_sweeps("M", 400.0, 1, 3)
+    return eng.get_moments()[0]
+
+
+def _steps(L):
+    eng = _engine(L, CF.bcc5_couplings())
+    for _ in range(150):
+        eng.sd_steps(1, 2)
+    return eng.get_moments()[0]
+
+
+@pytest.mark.parametrize("run,sizes", [
+    (_sweeps, ((10, 10, 10), (3, 3, 3), (6, 5, 4), (12, 9, 10))),   # 2 to 133 KB of LDS
+    (_steps, ((6, 6, 6), (3, 3, 3), (5, 5, 5), (4, 4, 4))),         # 11 to 91 KB
+])
+def test_contexts_of_different_lds_needs_in_threads(run, sizes):
+    want = [run(L) for L in sizes]
+    got = _in_threads([lambda L=L: run(L) for L in sizes])
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)

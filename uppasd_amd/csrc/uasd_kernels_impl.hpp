@@ -131,9 +131,8 @@ template <typename R, int ALG, bool LNB>
 static hipError_t llg_resident_one(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm,
                                    const ResDev &rd, int nsteps, size_t bytes, int threads,
                                    Quad<R> *spins) {
-  const hipError_t err = hipFuncSetAttribute((const void *)&k_llg_resident<R, ALG, LNB>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)bytes);
+  static LdsLimit limit;
+  const hipError_t err = limit.raise((const void *)&k_llg_resident<R, ALG, LNB>, bytes);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL((k_llg_resident<R, ALG, LNB>), dim3((unsigned)(rd.ncomp * h.M)),
                      dim3(threads), bytes, s, h, prm, rd, nsteps, spins);
@@ -165,10 +164,8 @@ template <typename R, bool HB, bool TRL, bool LNB>
 static hipError_t mc_resident_one(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
                                   const ResDev &rd, int nsweeps, size_t bytes, int threads,
                                   Quad<R> *spins, Quad<R> *trials) {
-  const void *kern = (const void *)&k_mc_resident<R, HB, TRL, LNB>;
-  // dynamic LDS above 64 KiB must be requested
-  const hipError_t err =
-      hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  static LdsLimit limit;
+  const hipError_t err = limit.raise((const void *)&k_mc_resident<R, HB, TRL, LNB>, bytes);
   if (err != hipSuccess) return err;
   hipLaunchKernelGGL((k_mc_resident<R, HB, TRL, LNB>), dim3((unsigned)(rd.ncomp * h.M)),
                      dim3(threads), bytes, s, h, mp, rd, nsweeps, spins, trials);

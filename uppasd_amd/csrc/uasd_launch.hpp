@@ -3,6 +3,9 @@
 // translation unit (uasd_kernels_f64.hip / uasd_kernels_f32.hip) so the FP64
 // unit can be compiled without multiply-add contraction.
 #pragma once
+#include <map>
+#include <mutex>
+
 #include "uasd_kernels.hpp"
 
 namespace uasd {
@@ -15,6 +18,26 @@ inline unsigned grid_for(int64_t n, int block) {
 }
 
 constexpr int kBlock = 256;  // largest workgroup the kernels are built for
+
+// The dynamic LDS one kernel may be launched with (above 64 KiB it must be
+// asked for).  That limit belongs to the process's kernel, which contexts on
+// other threads launch too: it is only ever raised, one thread at a time, so
+// no thread lowers it between another one's raise and launch.
+struct LdsLimit {
+  std::mutex mu;
+  std::map<int, size_t> bytes;  // per device
+  hipError_t raise(const void *kern, size_t n) {
+    int dev = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    std::lock_guard<std::mutex> lock(mu);
+    size_t &have = bytes[dev];
+    if (n <= have) return hipSuccess;
+    err = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)n);
+    if (err == hipSuccess) have = n;
+    return err;
+  }
+};
 
 // Launch shape of the gathering kernels (chosen by the autotuner):
 //   gather  neighbours whose loads are issued together: 2, 4, 8 or 16
