@@ -68,3 +68,27 @@ def test_contexts_of_different_lds_needs_in_threads(run, sizes):
     got = _in_threads([lambda L=L: run(L) for L in sizes])
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+def test_tile_shapes_in_threads():
+    """Two lattices of one tile kernel with different halos and threads (their
+    workgroups per CU differ), resident workgroups looping over units."""
+    def run(L, shape):
+        s = CF.bcc_shells(L, CF.bcc5_couplings(), moment=2.2)
+        N = s["lattice"].natom
+        eng = U.Engine(N, 1, site_order=2)
+        eng.set_lattice_dims(2, *L)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(N), 1), s["mmom"][None])
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 5)
+        eng.set_tuning(eng.TUNE_LLG, 4, 256 | (shape << 18) | 0x400000)
+        assert eng.llg_tile() == shape
+        for _ in range(60):
+            eng.sd_steps(1, 1)
+        return eng.get_moments()[0]
+    sizes = [((16, 16, 16), 8), ((18, 17, 16), 9), ((16, 16, 16), 9), ((18, 17, 16), 8)]
+    want = [run(*a) for a in sizes]
+    got = _in_threads([lambda a=a: run(*a) for a in sizes])
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)

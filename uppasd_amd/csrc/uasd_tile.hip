@@ -26,44 +26,45 @@ hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, con
   if (t.rs < 1) return hipErrorInvalidValue;  // at least one halo row per round
   const size_t lds = tile_lds_bytes(sizeof(R), plane, t.HX + t.NA * t.HY * t.HZ);
   // one unit per workgroup, or (pipe) as many workgroups as are resident at
-  // once (occupancy x CUs, cached per kernel and shape), each looping over a
-  // run of consecutive units
-  auto tiles_per_wg = [&](const void *kern, size_t &c_lds, int &c_thr, int &c_slots) -> hipError_t {
+  // once (occupancy x CUs, kept per kernel for its last shape), each looping
+  // over a run of consecutive units
+  struct Slots {
+    std::mutex mu;  // contexts on other threads launch the same kernel
+    int dev = -1, threads = 0, n = 0;
+    size_t lds = 0;
+  };
+  auto units_per_wg = [&](const void *kern, Slots &c) -> hipError_t {
     t.per = 1;
     if (!pipe) return hipSuccess;
-    if (c_lds != lds || c_thr != threads) {
-      int dev = 0, ncu = 0, occ = 0;
-      hipError_t err = hipGetDevice(&dev);
-      if (err == hipSuccess)
-        err = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    int dev = 0, ncu = 0, occ = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    std::lock_guard<std::mutex> lock(c.mu);
+    if (c.dev != dev || c.lds != lds || c.threads != threads) {
+      err = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
       if (err == hipSuccess)
         err = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kern, threads, lds);
       if (err != hipSuccess) return err;
-      c_lds = lds;
-      c_thr = threads;
-      c_slots = std::max(1, occ) * std::max(1, ncu);
+      c.dev = dev;
+      c.lds = lds;
+      c.threads = threads;
+      c.n = std::max(1, occ) * std::max(1, ncu);
     }
-    t.per = (nunits + c_slots - 1) / c_slots;
+    t.per = (nunits + c.n - 1) / c.n;
     return hipSuccess;
   };
 #define UASD_TILE_CASE(H, PL, F, E)                                                             \
   if (half == H && plane == PL && full == F && ens == E) {                                      \
-    static size_t lds_set = 0; /* dynamic LDS above 64 KiB must be requested */                 \
-    if (lds > lds_set) {                                                                        \
-      hipError_t err = hipFuncSetAttribute((const void *)&k_llg_tile<R, ALG, H, PL, F, E>,      \
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-      if (err != hipSuccess) return err;                                                        \
-      lds_set = lds;                                                                            \
-    }                                                                                           \
-    static size_t c_lds = 0;                                                                    \
-    static int c_thr = 0, c_slots = 0;                                                          \
-    hipError_t gerr = tiles_per_wg((const void *)&k_llg_tile<R, ALG, H, PL, F, E>, c_lds, c_thr, \
-                                   c_slots);                                                    \
-    if (gerr != hipSuccess) return gerr;                                                        \
+    const void *kern = (const void *)&k_llg_tile<R, ALG, H, PL, F, E>;                          \
+    static LdsLimit limit;                                                                      \
+    static Slots slots;                                                                         \
+    hipError_t err = limit.raise(kern, lds);                                                    \
+    if (err == hipSuccess) err = units_per_wg(kern, slots);                                     \
+    if (err != hipSuccess) return err;                                                          \
     const int nwg = (nunits + t.per - 1) / t.per;                                               \
     const dim3 grid((nwg + kXCD - 1) / kXCD * kXCD), block(threads);                            \
-    hipLaunchKernelGGL((k_llg_tile<R, ALG, H, PL, F, E>), grid, block, lds, s, tile_ham(h), prm, t, e, p, b2, \
-                       out);                                                                    \
+    hipLaunchKernelGGL((k_llg_tile<R, ALG, H, PL, F, E>), grid, block, lds, s, tile_ham(h), prm, \
+                       t, e, p, b2, out);                                                       \
     return hipGetLastError();                                                                   \
   }
 #define UASD_TILE_FULL(H, PL)                                                                   \
