@@ -818,7 +818,7 @@ std::vector<int> independent_ranges(const uasd_ctx *c) {
 // Builds c->lres, the systems of the lattice for resident LLG steps, where
 // they are small enough for them.  Lattices over kLlgResLattice sites are not
 // looked through: their batches fill the chip with the other kernels.
-constexpr int kLlgResSites = uasd::kResThreads, kLlgResLattice = 16384;
+constexpr int kLlgResSites = uasd::kResThreads, kLlgResLattice = 16384, kLlgResItems = 131072;
 
 int build_llg_resident(uasd_ctx *c) {
   auto &r = c->lres;
@@ -889,7 +889,7 @@ int build_llg_resident(uasd_ctx *c) {
 // are timed one by one or graphs were asked for.
 bool llg_use_resident(const uasd_ctx *c) {
   return c->lres.ok && c->lres.cls_version == c->cls_version && !c->timing &&
-         c->graph_steps == 0 && (int64_t)c->N * c->M <= 131072;
+         c->graph_steps == 0 && (int64_t)c->N * c->M <= kLlgResItems;
 }
 
 // Steps whose Philox deviates are drawn in one launch ahead of them.  FP64
@@ -902,6 +902,20 @@ int steps_ahead(const uasd_ctx *c) {
   return c->prec == UASD_FP64 && (int64_t)c->N * c->M <= 32768 ? 16 : 1;
 }
 
+// Steps of a resident launch: as many as deviates of 2^18 items cover, 4 to 64.
+int64_t resident_steps(const uasd_ctx *c) {
+  return std::max<int64_t>(4, std::min<int64_t>(64, 262144 / ((int64_t)c->N * c->M)));
+}
+
+// Steps whose deviates c->nsave holds: the most that any path of this context
+// draws at once, from its sizes alone.  The buffer then never moves, so steps
+// that a caller captured into a graph of its own keep a valid address whatever
+// runs between its replays.
+int64_t nsave_steps(const uasd_ctx *c) {
+  const bool res = c->N <= kLlgResLattice && (int64_t)c->N * c->M <= kLlgResItems;
+  return std::max<int64_t>(steps_ahead(c), res ? resident_steps(c) : 1);
+}
+
 int ready_for_llg(uasd_ctx *c) {
   if (!c->have_ex) return fail(UASD_ERR_STATE, "exchange not set (uasd_set_exchange)");
   if (!c->have_state) return fail(UASD_ERR_STATE, "moments not set (uasd_set_moments)");
@@ -910,7 +924,7 @@ int ready_for_llg(uasd_ctx *c) {
     return fail(UASD_ERR_STATE, "injected noise selected but no normals uploaded");
   if (c->noise_mode == UASD_NOISE_PHILOX) {
     void *old = c->nsave.p;
-    HIP_TRY(c->nsave.ensure((size_t)steps_ahead(c) * c->N * c->M * 4 * c->rsize));
+    HIP_TRY(c->nsave.ensure((size_t)nsave_steps(c) * quad_bytes(c)));
     if (c->nsave.p != old) c->gen += 1;  // captured graphs hold the old address
   }
   return rebuild_classes(c);
@@ -2005,19 +2019,11 @@ bool repeats_pay(uasd_ctx *c, int kind, int alg, uint64_t seed, int64_t items, i
   return r.second - n >= after;
 }
 
-// nsteps steps in resident launches of 4 to 64, as many as deviates of 2^18
-// items cover.
+// nsteps steps in resident launches.
 template <typename R>
 int llg_resident_steps(uasd_ctx *c, int alg, int64_t nsteps) {
   const bool philox = llg_view<R>(c).noise_mode == UASD_NOISE_PHILOX;
-  const int64_t chunk =
-      std::max<int64_t>(4, std::min<int64_t>(64, 262144 / ((int64_t)c->N * c->M)));
-  if (philox) {
-    const int64_t most = std::min(chunk, nsteps);
-    void *old = c->nsave.p;
-    HIP_TRY(c->nsave.ensure((size_t)most * quad_bytes(c)));
-    if (c->nsave.p != old) c->gen += 1;
-  }
+  const int64_t chunk = resident_steps(c);
   for (int64_t s = 0; s < nsteps; s += chunk) {
     const int n = (int)std::min(chunk, nsteps - s);
     if (philox)
