@@ -56,6 +56,22 @@ enum {
   UASD_SDE_SPHMID = 7   /* sispht/sisphf, sphmidpoint.f90:485-923 */
 };
 
+/* Launches counted by uasd_launch_counts: half steps of the list kernels and
+ * of the tile kernel, resident launches (all the steps or sweeps of small
+ * systems that fit one launch), deviates drawn ahead, colour passes, and
+ * replayed graphs of steps and of sweeps. */
+enum {
+  UASD_LAUNCH_LLG_LIST = 0,
+  UASD_LAUNCH_LLG_TILE = 1,
+  UASD_LAUNCH_LLG_RESIDENT = 2,
+  UASD_LAUNCH_DRAW = 3,
+  UASD_LAUNCH_MC_COLOUR = 4,
+  UASD_LAUNCH_MC_RESIDENT = 5,
+  UASD_LAUNCH_LLG_GRAPH = 6,
+  UASD_LAUNCH_MC_GRAPH = 7,
+  UASD_NUM_LAUNCH_KINDS = 8
+};
+
 typedef struct uasd_ctx uasd_ctx;
 
 const char *uasd_last_error(void);
@@ -226,6 +242,12 @@ int uasd_index_bytes(uasd_ctx *ctx, int *exchange, int *dm);
  * context: no stencil, LDS, thread count). */
 int uasd_llg_tile(uasd_ctx *ctx, int *tile);
 
+/* Launches of the resident entry points since the context was created, by the
+ * path that was taken (no reference counterpart): counts holds
+ * UASD_NUM_LAUNCH_KINDS values.  Which path a call takes is a matter of sizes,
+ * repetition and tuning; results do not depend on it. */
+int uasd_launch_counts(uasd_ctx *ctx, int64_t *counts);
+
 /* ---- launch shapes of the gathering kernels (no reference counterpart:
  * the reference's OpenMP loops have no launch shape) ----
  * kind: 0 fused LLG step, 1 field, 2 MC colour pass.  gather = neighbours
@@ -245,7 +267,10 @@ int uasd_llg_tile(uasd_ctx *ctx, int *tile);
  * most 8), which the list kernels otherwise gather once for both sums;
  * plus 0x1000000 (kind 2 only) for two adjacent ensembles of a site per
  * thread, sharing its neighbour entries and couplings (M even; one per
- * thread otherwise).  Results do not depend on any of them. */
+ * thread otherwise).  A shape that was asked for is launched: small systems,
+ * whose steps (kind 0) or sweeps (kind 2) run in resident launches otherwise,
+ * then take the kernels that have a shape.  Results do not depend on any of
+ * them. */
 int uasd_set_tuning(uasd_ctx *ctx, int kind, int gather, int block);
 int uasd_get_tuning(uasd_ctx *ctx, int kind, int *gather, int *block);
 /* Autotuner: times every shape on the context's own lattice and state

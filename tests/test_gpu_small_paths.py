@@ -187,3 +187,42 @@ def test_resident_steps_equal_launched_ones(name, precision, noise):
     for k in range(3):
         assert np.array_equal(out[0][k], out[2][k]), (name, k)
         assert np.array_equal(out[1][k], out[2][k]), (name, k)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("shape", ["list", "tile", "colour"])
+def test_asked_for_shapes_are_launched(shape, precision):
+    """A launch shape that was set is the one that runs, also on systems small
+    enough for resident launches, which run where none was set; with the same
+    results."""
+    s = CF.triangular_dmi(20)                                # 400 sites, DM + K + B
+    N, M, alg, steps = s["lattice"].natom, 2, 5, 6
+    temps = [300.0, 900.0]
+    out = []
+    for asked in (False, True):
+        eng = U.Engine(N, M, precision)
+        eng.set_lattice_dims(1, *s["lattice"].n)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_dm(s["dmlist"], s["dmlistsize"], s["dm_vect"])
+        eng.set_anisotropy(s["taniso"], s["eaniso"], s["kaniso"], s["sb"])
+        eng.set_external_field(s["ext"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(6), M),
+                        np.broadcast_to(s["mmom"], (M, N)))
+        eng.set_llg(0.1, 200.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 3)
+        if asked and shape == "colour":
+            eng.set_tuning(eng.TUNE_MC, 8, 128 | 0x1000000)
+        elif asked:
+            eng.set_tuning(eng.TUNE_LLG, 4, 256 | ((5 << 18) if shape == "tile" else 0))
+        if shape == "colour":
+            eng.mc_sweeps("M", temps, steps, 9)
+            want = {"mc_colour": steps * eng.coloring()[0]} if asked else {"mc_resident": 1}
+        else:
+            eng.sd_steps(alg, steps)
+            want = {"llg_" + shape: 2 * steps} if asked else {"llg_resident": 1}
+        n = {k: v for k, v in eng.launch_counts().items() if v and k != "draw"}
+        assert n == want
+        if asked and shape != "colour":
+            assert eng.llg_tile() == (5 if shape == "tile" else 0)
+        out.append(eng.get_moments()[0])
+    assert np.array_equal(out[0], out[1])

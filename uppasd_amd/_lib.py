@@ -37,7 +37,7 @@ EXPORTS = (
     "uasd_accumulate", "uasd_get_accumulators", "uasd_reset_accumulators", "uasd_set_graph_steps",
     "uasd_index_bytes", "uasd_llg_tile", "uasd_set_site_order", "uasd_set_lattice_dims",
     "uasd_has_stencil",
-    "uasd_build_pair_list", "uasd_set_tune_cache",
+    "uasd_build_pair_list", "uasd_set_tune_cache", "uasd_launch_counts",
 )
 
 
@@ -97,6 +97,7 @@ def lib() -> C.CDLL:
         L.uasd_set_graph_steps.argtypes = [vp, C.c_int]
         L.uasd_index_bytes.argtypes = [vp, ip, ip]
         L.uasd_llg_tile.argtypes = [vp, ip]
+        L.uasd_launch_counts.argtypes = [vp, C.POINTER(C.c_int64)]
         L.uasd_set_site_order.argtypes = [vp, C.c_int]
         L.uasd_set_lattice_dims.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.c_int]
         L.uasd_has_stencil.argtypes = [vp, ip, vp]

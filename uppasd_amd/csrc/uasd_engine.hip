@@ -271,6 +271,9 @@ struct uasd_ctx {
   } res, lres;  // for MC sweeps (colour order), for LLG steps (device order)
   int64_t col_version = 0;  // bumped by every colouring rebuild
 
+  // launches by path (uasd_launch_counts)
+  int64_t launches[UASD_NUM_LAUNCH_KINDS] = {};
+
   // Per-kernel timing: an event pair is recorded around each launch without
   // a host wait; pairs are resolved when the totals are read.
   bool timing = false;
@@ -745,6 +748,11 @@ int region_toc(uasd_ctx *c) {
   return UASD_OK;
 }
 
+// One launch of `kind` that runs now (not one recorded into a graph).
+void count(uasd_ctx *c, int kind) {
+  if (!c->capturing) c->launches[kind] += 1;
+}
+
 int resolve_timing(uasd_ctx *c) {
   for (auto &p : c->pending) {
     HIP_TRY(hipEventSynchronize(p.b));
@@ -886,10 +894,11 @@ int build_llg_resident(uasd_ctx *c) {
 // -> 11.3 (18.2 -> 7.5), SIB 17.1 -> 12.9; 64 ensembles of 432 sites 13.1 ->
 // 6.5.  With 1024 sites the one CU is as slow as the launches (58 neighbours
 // 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  Not while the kernels
-// are timed one by one or graphs were asked for.
+// are timed one by one, graphs were asked for or a launch shape was: a shape
+// is one of the kernels that the resident launch would take the place of.
 bool llg_use_resident(const uasd_ctx *c) {
   return c->lres.ok && c->lres.cls_version == c->cls_version && !c->timing &&
-         c->graph_steps == 0 && (int64_t)c->N * c->M <= kLlgResItems;
+         c->graph_steps == 0 && !c->tune[0].chosen && (int64_t)c->N * c->M <= kLlgResItems;
 }
 
 // Steps whose Philox deviates are drawn in one launch ahead of them.  FP64
@@ -968,6 +977,7 @@ int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
       tic(c, half);
       HIP_TRY(uasd::launch_llg_tile<R>(c->stream, t, c->tune[0].pipe, alg, half, h, prm, e, p, b2,
                                        out));
+      count(c, UASD_LAUNCH_LLG_TILE);
       return toc(c, half);
     }
   }
@@ -975,6 +985,7 @@ int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
   HIP_TRY(uasd::launch_llg<R>(c->stream,
                               uasd::default_tune(c->tune[0], (int64_t)c->N * c->M, c->W), alg,
                               half, fused, h, prm, e, p, b2, beff, out));
+  count(c, UASD_LAUNCH_LLG_LIST);
   return toc(c, half);
 }
 
@@ -1916,6 +1927,7 @@ int replay_graph(uasd_ctx *c, const std::tuple<int, int, int, uint64_t> &key, in
   }
   tic(c, timer);
   HIP_TRY(hipGraphLaunch(it->second.exec, c->stream));
+  count(c, idx == 0 ? UASD_LAUNCH_LLG_GRAPH : UASD_LAUNCH_MC_GRAPH);
   if (int r = toc(c, timer)) return r;
   host_ctr += (uint64_t)K;
   c->ctr_val[idx] = host_ctr;
@@ -1970,6 +1982,7 @@ int draw_ahead(uasd_ctx *c, int n, int64_t step_off) {
     prm.step_dev = c->ctr.as<uint64_t>();
   }
   HIP_TRY(uasd::launch_draw<R>(c->stream, ham_view<R>(c), prm, n, quads<R>(c, c->nsave)));
+  count(c, UASD_LAUNCH_DRAW);
   return UASD_OK;
 }
 
@@ -2032,6 +2045,7 @@ int llg_resident_steps(uasd_ctx *c, int alg, int64_t nsteps) {
     if (philox) prm.nsave = quads<R>(c, c->nsave);
     HIP_TRY(uasd::launch_llg_resident<R>(c->stream, alg, ham_view<R>(c), prm, c->lres.dev, n,
                                          (size_t)c->lds_max, quads<R>(c, c->spins, 0)));
+    count(c, UASD_LAUNCH_LLG_RESIDENT);
     c->step += (uint64_t)n;
   }
   return UASD_OK;
@@ -2225,8 +2239,9 @@ static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed
 //    (1024 ensembles of 2000 sites, 9 colours) 158 -> 113 us a sweep, at 262k
 //    (alloy pairs of 1024 sites, 256 ensembles, 2 colours) 29 -> 21 us; at
 //    600k (64 alloys, 32 ensembles) 54 -> 61 us, slower.
+// Not where a launch shape was asked for: it is one of the colour pass.
 static bool mc_use_resident(const uasd_ctx *c) {
-  return c->res.ok && c->res.nmax <= uasd::kResThreads * c->ncolors &&
+  return c->res.ok && !c->tune[2].chosen && c->res.nmax <= uasd::kResThreads * c->ncolors &&
          (int64_t)c->N * c->M <= (int64_t)c->ncolors << 18;
 }
 
@@ -2246,6 +2261,7 @@ static int mc_resident(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
       HIP_TRY(uasd::launch_mc_resident<float>(c->stream, ham_view<float>(c), mp, c->res.dev, n,
                                               (size_t)c->lds_max, quads<float>(c, c->spins, 0),
                                                quads<float>(c, c->spins, 1)));
+    count(c, UASD_LAUNCH_MC_RESIDENT);
     if (int r = toc(c, 3)) return r;
     mp.sweep += (uint64_t)n;
   }
@@ -2281,6 +2297,7 @@ static int mc_run(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
         HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, mp.nsites), ham_view<float>(c), mp,
                                        quads<float>(c, c->spins, 0)));
       }
+      count(c, UASD_LAUNCH_MC_COLOUR);
       if (int r = toc(c, 3)) return r;
     }
     c->mc_sweep += 1;
@@ -2371,6 +2388,13 @@ int uasd_llg_tile(uasd_ctx *c, int *tile) {
     build_stencil(c);
     if (tile_fits(c, c->tune[0].tile)) *tile = c->tune[0].tile;
   }
+  return UASD_OK;
+}
+
+int uasd_launch_counts(uasd_ctx *c, int64_t *counts) {
+  if (int r = check_ctx(c)) return r;
+  if (!counts) return fail(UASD_ERR_ARG, "counts must not be NULL");
+  std::copy(c->launches, c->launches + UASD_NUM_LAUNCH_KINDS, counts);
   return UASD_OK;
 }
 

@@ -249,6 +249,15 @@ class Engine:
         B.check(B.lib().uasd_llg_tile(self._h, C.byref(k)), "uasd_llg_tile")
         return k.value
 
+    LAUNCH_KINDS = ("llg_list", "llg_tile", "llg_resident", "draw", "mc_colour", "mc_resident",
+                    "llg_graph", "mc_graph")
+
+    def launch_counts(self):
+        """Launches by path since the engine was made, as a dict over LAUNCH_KINDS."""
+        n = (C.c_int64 * len(self.LAUNCH_KINDS))()
+        B.check(B.lib().uasd_launch_counts(self._h, n), "uasd_launch_counts")
+        return dict(zip(self.LAUNCH_KINDS, n))
+
     def set_graph_steps(self, k: int):
         """Replay hipGraphs of k LLG steps / MC sweeps (0 = left to the library)."""
         B.check(B.lib().uasd_set_graph_steps(self._h, int(k)), "uasd_set_graph_steps")
