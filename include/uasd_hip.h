@@ -239,7 +239,8 @@ int uasd_index_bytes(uasd_ctx *ctx, int *exchange, int *dm);
 /* The kernel the fused LLG step launches under the current tuning (no
  * reference counterpart): *tile = the LDS-tiled stencil shape k (1..15), or 0
  * for the list-gather kernels (also when a requested shape does not fit the
- * context: no stencil, LDS, thread count). */
+ * context: no stencil, LDS, thread count) and where the step runs in resident
+ * launches. */
 int uasd_llg_tile(uasd_ctx *ctx, int *tile);
 
 /* Launches of the resident entry points since the context was created, by the
@@ -273,7 +274,8 @@ int uasd_launch_counts(uasd_ctx *ctx, int64_t *counts);
  * them. */
 int uasd_set_tuning(uasd_ctx *ctx, int kind, int gather, int block);
 int uasd_get_tuning(uasd_ctx *ctx, int kind, int *gather, int *block);
-/* Autotuner: times every shape on the context's own lattice and state
+/* Autotuner: times every shape (and the resident launch, where the systems are
+ * small enough for it) on the context's own lattice and state
  * (steps LLG steps / sweeps MC sweeps per candidate), keeps the fastest and
  * restores the spins and step counters, so a run is unchanged by tuning.
  * best_ms (may be NULL) receives the fastest candidate's time. */

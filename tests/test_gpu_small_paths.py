@@ -226,3 +226,52 @@ def test_asked_for_shapes_are_launched(shape, precision):
             assert eng.llg_tile() == (5 if shape == "tile" else 0)
         out.append(eng.get_moments()[0])
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("kind", ["llg", "mc"])
+def test_autotuner_times_what_runs(kind, tmp_path):
+    """On small systems the autotuner times the shapes with the kernels they
+    belong to and the resident launch beside them; what it keeps is what the
+    next call runs, in this context and in one that takes the kept result."""
+    s = CF.bcc_shells((6, 6, 6), CF.bcc5_couplings(), moment=2.2)
+    N, path = s["lattice"].natom, tmp_path / "tune.txt"
+
+    def make():
+        eng = U.Engine(N, 1)
+        eng.set_lattice_dims(2, 6, 6, 6)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(8), 1), s["mmom"][None])
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 3)
+        return eng
+
+    def tune(eng):
+        return eng.autotune_llg(1, steps=4) if kind == "llg" else eng.autotune_mc("M", 400.0, 2)
+
+    def run(eng):
+        before = eng.launch_counts()
+        eng.sd_steps(1, 4) if kind == "llg" else eng.mc_sweeps("M", 400.0, 2, 9)
+        after = eng.launch_counts()
+        return {k for k in after if after[k] > before[k] and k != "draw"}, eng.get_moments()[0]
+
+    ref = run(make())
+    try:
+        U.set_tune_cache(True, str(path))
+        a = make()
+        ms = tune(a)
+        n = a.launch_counts()
+        launched = n["llg_list"] + n["llg_tile"] if kind == "llg" else n["mc_colour"]
+        assert launched > 0 and n[kind + "_resident"] > 0 and ms > 0.0    # both were timed
+        line, = path.read_text().splitlines()
+        won = line.split()[0].endswith("/res1")
+        assert won or line.split()[0].endswith("/res0")
+        b = make()
+        assert tune(b) == ms and sum(b.launch_counts().values()) == 0     # taken over, not timed
+        for eng in (a, b):
+            path_of, e = run(eng)
+            assert (path_of == {kind + "_resident"}) == won
+            assert won or path_of <= {"llg_list", "llg_tile", "mc_colour"}
+            assert np.array_equal(e, ref[1])
+            assert kind == "mc" or not (won and eng.llg_tile())
+    finally:
+        U.set_tune_cache(False)

@@ -896,9 +896,13 @@ int build_llg_resident(uasd_ctx *c) {
 // 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  Not while the kernels
 // are timed one by one, graphs were asked for or a launch shape was: a shape
 // is one of the kernels that the resident launch would take the place of.
+bool llg_can_be_resident(const uasd_ctx *c) {
+  return c->lres.ok && c->lres.cls_version == c->cls_version && c->graph_steps == 0 &&
+         (int64_t)c->N * c->M <= kLlgResItems;
+}
+
 bool llg_use_resident(const uasd_ctx *c) {
-  return c->lres.ok && c->lres.cls_version == c->cls_version && !c->timing &&
-         c->graph_steps == 0 && !c->tune[0].chosen && (int64_t)c->N * c->M <= kLlgResItems;
+  return llg_can_be_resident(c) && !c->timing && c->tune[0].chosen != uasd::kShapeAsked;
 }
 
 // Steps whose Philox deviates are drawn in one launch ahead of them.  FP64
@@ -1972,6 +1976,13 @@ int llg_step(uasd_ctx *c, int alg, int64_t step_off, int ahead) {
   return UASD_OK;
 }
 
+// The tile shape the launched half steps take, 0 for the list kernels.
+int launched_tile(uasd_ctx *c) {
+  if (c->tune[0].tile == 0) return 0;
+  build_stencil(c);
+  return tile_fits(c, c->tune[0].tile) ? c->tune[0].tile : 0;
+}
+
 // Deviates of n steps (from the context's step, or inside a capture from
 // *ctr[0] + step_off) into c->nsave.
 template <typename R>
@@ -1990,9 +2001,7 @@ int draw_ahead(uasd_ctx *c, int n, int64_t step_off) {
 // the device counter.
 int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
   int K = llg_view<double>(c).noise_mode == UASD_NOISE_PHILOX ? steps_ahead(c) : 1;
-  int tile = 0;  // the tile kernels draw their own deviates
-  if (int r = uasd_llg_tile(c, &tile)) return r;
-  if (tile) K = 1;
+  if (launched_tile(c)) K = 1;  // the tile kernels draw their own deviates
   for (int64_t s = 0; s < n; ++s) {
     const int k = (int)(s % K);
     const int64_t off = in_graph ? s : -1;
@@ -2240,9 +2249,13 @@ static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed
 //    (alloy pairs of 1024 sites, 256 ensembles, 2 colours) 29 -> 21 us; at
 //    600k (64 alloys, 32 ensembles) 54 -> 61 us, slower.
 // Not where a launch shape was asked for: it is one of the colour pass.
-static bool mc_use_resident(const uasd_ctx *c) {
-  return c->res.ok && !c->tune[2].chosen && c->res.nmax <= uasd::kResThreads * c->ncolors &&
+static bool mc_can_be_resident(const uasd_ctx *c) {
+  return c->res.ok && c->res.nmax <= uasd::kResThreads * c->ncolors &&
          (int64_t)c->N * c->M <= (int64_t)c->ncolors << 18;
+}
+
+static bool mc_use_resident(const uasd_ctx *c) {
+  return mc_can_be_resident(c) && c->tune[2].chosen != uasd::kShapeAsked;
 }
 
 // nsweeps sweeps in resident launches of at most kResSweeps, from mp.sweep on.
@@ -2383,11 +2396,7 @@ int uasd_index_bytes(uasd_ctx *c, int *exchange, int *dm) {
 int uasd_llg_tile(uasd_ctx *c, int *tile) {
   if (int r = check_ctx(c)) return r;
   if (!tile) return fail(UASD_ERR_ARG, "tile must not be NULL");
-  *tile = 0;
-  if (c->tune[0].tile > 0) {
-    build_stencil(c);
-    if (tile_fits(c, c->tune[0].tile)) *tile = c->tune[0].tile;
-  }
+  *tile = llg_use_resident(c) ? 0 : launched_tile(c);
   return UASD_OK;
 }
 
@@ -2408,7 +2417,7 @@ int uasd_set_tuning(uasd_ctx *c, int kind, int gather, int block) {
   // where the DM bonds are the exchange bonds (context-wide), 0x1000000 two
   // adjacent ensembles per thread (MC only)
   uasd::Tune t{gather, block & 0xffff, (block >> 16) & 1, (block >> 17) & 1, (block >> 18) & 0xf,
-               (block >> 22) & 1, (block >> 24) & 1, 1};
+               (block >> 22) & 1, (block >> 24) & 1, uasd::kShapeAsked};
   if (!uasd::tune_valid(t) || (block >> 25) != 0 || (kind != 0 && t.tile != 0) ||
       (kind != 2 && t.pair != 0))
     return fail(UASD_ERR_ARG, "gather must be 2, 4, 8 or 16 and block 64, 128 or 256");
@@ -2466,8 +2475,6 @@ struct EventPair {
   }
 };
 
-// Times `run` (asynchronous launches on c->stream) for every candidate shape,
-// once untimed and once timed, and leaves the fastest in *slot.
 // ------------------------------------------------------ autotuner cache
 // Winners of uasd_autotune_* per workload, kept for the process once
 // uasd_set_tune_cache has switched the cache on, and read from / appended to
@@ -2515,9 +2522,39 @@ void tune_store(const std::string &key, const uasd::Tune &t, double ms) {
   }
 }
 
+// Key of a context whose steps or sweeps could be resident: its entry also
+// says whether that was faster than every shape, which other contexts of the
+// same sizes (other bonds) must not take over.
+std::string resident_key(const std::string &key, bool won) { return key + (won ? "/res1" : "/res0"); }
+
+// The kept result of this workload into slot, as tune_search leaves it.
+bool tune_cached(const std::string &key, bool resident, uasd::Tune *slot, double &ms) {
+  uasd::Tune t;
+  bool won = resident;
+  if (!resident) {
+    if (!tune_lookup(key, t, ms)) return false;
+  } else if (!tune_lookup(resident_key(key, true), t, ms)) {
+    won = false;
+    if (!tune_lookup(resident_key(key, false), t, ms)) return false;
+  }
+  if (!uasd::tune_valid(t)) return false;
+  t.chosen = won ? uasd::kShapeResident : uasd::kShapeAsked;
+  *slot = t;
+  return true;
+}
+
+void tune_keep(const std::string &key, bool resident, const uasd::Tune &t, double ms) {
+  tune_store(resident ? resident_key(key, t.chosen == uasd::kShapeResident) : key, t, ms);
+}
+
+// Times `run` (asynchronous launches on c->stream) for every shape and leaves the fastest in *slot, marked as asked
+// for.  pair: also two ensembles per thread (the MC colour pass, M even);
+// resident: also the resident launch, which run() makes while the slot is
+// marked kShapeResident; where that is the fastest, the slot keeps the fastest
+// shape beside that mark.
 template <typename Run>
-// pair: also time two ensembles per thread (the MC colour pass, M even)
-int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool pair = false) {
+int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool pair,
+                bool resident) {
   EventPair ev;
   HIP_TRY(hipEventCreate(&ev.a));
   HIP_TRY(hipEventCreate(&ev.b));
@@ -2542,7 +2579,6 @@ int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool 
   // run of a small lattice (tens of us) ranks shapes within its own scatter
   auto timed = [&](const uasd::Tune &cd, int reps, float &ms) -> int {
     *slot = cd;
-    slot->chosen = 1;
     if (int r = run()) return r;
     HIP_TRY(hipEventRecord(ev.a, c->stream));
     for (int k = 0; k < reps; ++k)
@@ -2556,13 +2592,13 @@ int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool 
   std::vector<std::pair<float, int>> rank;
   for (size_t i = 0; i < cand.size(); ++i) {
     float ms = 0.f;
+    cand[i].chosen = uasd::kShapeAsked;
     if (int r = timed(cand[i], 1, ms)) return r;
     rank.emplace_back(ms, (int)i);
   }
   std::sort(rank.begin(), rank.end());
   constexpr int kFinal = 5, kReps = 6;
   uasd::Tune best = cand[rank[0].second];
-  best.chosen = 1;
   float best_t = 1e30f;
   for (int k = 0; k < kFinal && k < (int)rank.size(); ++k) {
     float ms = 0.f;
@@ -2570,6 +2606,16 @@ int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool 
     if (ms < best_t) {
       best_t = ms;
       best = *slot;
+    }
+  }
+  if (resident) {
+    uasd::Tune res = best;
+    res.chosen = uasd::kShapeResident;
+    float ms = 0.f;
+    if (int r = timed(res, kReps, ms)) return r;
+    if (ms < best_t) {
+      best_t = ms;
+      best = res;
     }
   }
   *slot = best;
@@ -2588,12 +2634,13 @@ int uasd_autotune_llg(uasd_ctx *c, int alg, int steps, double *best_ms) {
   if (steps <= 0) return fail(UASD_ERR_ARG, "steps must be > 0");
   if (int r = ready_for_llg(c)) return r;
   build_stencil(c);
+  if (int r = build_llg_resident(c)) return r;
   const std::string key = tune_key(c, "llg", alg);
+  const bool resident = llg_can_be_resident(c);
   uasd::Tune cached;
   double cached_ms = 0.0;
-  if (tune_lookup(key, cached, cached_ms) && uasd::tune_valid(cached) && cached.pair == 0 &&
+  if (tune_cached(key, resident, &cached, cached_ms) && cached.pair == 0 &&
       (cached.tile == 0 || tile_fits(c, cached.tile))) {
-    cached.chosen = 1;
     c->tune[0] = c->tune[1] = cached;
     c->tune[1].tile = c->tune[1].pipe = 0;
     if (best_ms) *best_ms = cached_ms;
@@ -2603,11 +2650,14 @@ int uasd_autotune_llg(uasd_ctx *c, int alg, int steps, double *best_ms) {
   StateGuard g(c);
   if (g.err) return g.err;
   double ms_found = 0.0;
-  int r = tune_search(c, &c->tune[0], [&]() -> int { return llg_steps(c, alg, steps, false); },
-                      &ms_found);
+  int r = tune_search(c, &c->tune[0], [&]() -> int {
+    if (!llg_use_resident(c)) return llg_steps(c, alg, steps, false);
+    return c->prec == UASD_FP64 ? llg_resident_steps<double>(c, alg, steps)
+                                : llg_resident_steps<float>(c, alg, steps);
+  }, &ms_found, false, resident);
   if (r) return r;
   if (best_ms) *best_ms = ms_found;
-  tune_store(key, c->tune[0], ms_found);
+  tune_keep(key, resident, c->tune[0], ms_found);
   c->tune[1] = c->tune[0];  // the field kernel gathers the same way
   c->gen += 1;
   return g.restore();
@@ -2619,10 +2669,10 @@ int uasd_autotune_mc(uasd_ctx *c, char mode, const double *temps, int sweeps, do
   uasd::MCParams mp;
   if (int r = mc_prepare(c, mode, temps, 0x7u, mp)) return r;
   const std::string key = tune_key(c, "mc", (int)mode);
+  const bool resident = mc_can_be_resident(c);
   uasd::Tune cached;
   double cached_ms = 0.0;
-  if (tune_lookup(key, cached, cached_ms) && uasd::tune_valid(cached) && cached.tile == 0) {
-    cached.chosen = 1;
+  if (tune_cached(key, resident, &cached, cached_ms) && cached.tile == 0) {
     c->tune[2] = cached;
     if (best_ms) *best_ms = cached_ms;
     c->gen += 1;
@@ -2632,10 +2682,10 @@ int uasd_autotune_mc(uasd_ctx *c, char mode, const double *temps, int sweeps, do
   if (g.err) return g.err;
   double ms_found = 0.0;
   int r = tune_search(c, &c->tune[2], [&]() -> int { return mc_run(c, mp, sweeps); }, &ms_found,
-                      true);
+                      true, resident);
   if (r) return r;
   if (best_ms) *best_ms = ms_found;
-  tune_store(key, c->tune[2], ms_found);
+  tune_keep(key, resident, c->tune[2], ms_found);
   c->gen += 1;
   return g.restore();
 }

@@ -58,8 +58,12 @@ struct Tune {
   int tile = 0;
   int pipe = 0;  // tile kernel: 1 = resident workgroups loop over several tiles
   int pair = 0;  // MC colour pass: 1 = two adjacent ensembles per thread (M even)
-  int chosen = 0;  // 1: set by the caller or found by the autotuner, 0: default_tune applies
+  // 0: nobody has tuned, default_tune applies; kShapeAsked: set by the caller,
+  // or the autotuner's fastest; kShapeResident: the autotuner's fastest shape,
+  // for where resident launches, which were faster still, do not apply
+  int chosen = 0;
 };
+constexpr int kShapeAsked = 1, kShapeResident = 2;
 
 // Launch shape of a gathering kernel that nobody has tuned: n items (sites x
 // ensembles of a launch), w neighbours.  A small launch is a chain of loads on
