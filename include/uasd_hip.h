@@ -273,6 +273,9 @@ int uasd_launch_counts(uasd_ctx *ctx, int64_t *counts);
  * then take the kernels that have a shape.  Results do not depend on any of
  * them. */
 int uasd_set_tuning(uasd_ctx *ctx, int kind, int gather, int block);
+/* The shape the launches of a kind take: as set, as tuned, or, where neither
+ * was done, the library's own choice by size (for the colour pass that of a
+ * colour of average size). */
 int uasd_get_tuning(uasd_ctx *ctx, int kind, int *gather, int *block);
 /* Autotuner: times every shape (and the resident launch, where the systems are
  * small enough for it) on the context's own lattice and state

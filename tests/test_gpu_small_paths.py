@@ -275,3 +275,20 @@ def test_autotuner_times_what_runs(kind, tmp_path):
             assert kind == "mc" or not (won and eng.llg_tile())
     finally:
         U.set_tune_cache(False)
+
+
+@pytest.mark.parametrize("L,shells,want", [
+    ((7, 7, 7), [1.34, 0.77], (4, 64)),              # small, 14 neighbours
+    ((7, 7, 7), CF.bcc5_couplings(), (8, 64)),       # small, 58
+    ((64, 64, 32), [1.34, 0.77], (4, 64)),           # 2^18 items: the last small size
+    ((64, 64, 33), [1.34, 0.77], (4, 256)),
+])
+def test_tuning_reports_what_is_launched(L, shells, want):
+    s = CF.bcc_shells(L, shells, moment=2.2)
+    eng = U.Engine(s["lattice"].natom, 1)
+    eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+    assert eng.tuning(eng.TUNE_LLG) == eng.tuning(eng.TUNE_FIELD) == want
+    eng.set_tuning(eng.TUNE_LLG, *eng.tuning(eng.TUNE_LLG))
+    assert eng.tuning(eng.TUNE_LLG) == want
+    eng.set_tuning(eng.TUNE_FIELD, 16, 128)
+    assert eng.tuning(eng.TUNE_FIELD) == (16, 128)

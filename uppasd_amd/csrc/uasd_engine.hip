@@ -2429,11 +2429,13 @@ int uasd_set_tuning(uasd_ctx *c, int kind, int gather, int block) {
 int uasd_get_tuning(uasd_ctx *c, int kind, int *gather, int *block) {
   if (int r = check_ctx(c)) return r;
   if (kind < 0 || kind > 2) return fail(UASD_ERR_ARG, "kind must be 0 (LLG), 1 (field) or 2 (MC)");
-  if (gather) *gather = c->tune[kind].gather;
+  // the shape that is launched (colours differ in size: that of an average one)
+  const int64_t items = (int64_t)c->N * c->M / (kind == 2 ? std::max(c->ncolors, 1) : 1);
+  const uasd::Tune t = uasd::default_tune(c->tune[kind], items, c->W);
+  if (gather) *gather = t.gather;
   if (block)
-    *block = c->tune[kind].block | (c->tune[kind].nt << 16) | (c->tune[kind].idx32 << 17) |
-             (c->tune[kind].tile << 18) | (c->tune[kind].pipe << 22) |
-             ((c->tune_no_fuse ? 1 : 0) << 23) | (c->tune[kind].pair << 24);
+    *block = t.block | (t.nt << 16) | (t.idx32 << 17) | (t.tile << 18) | (t.pipe << 22) |
+             ((c->tune_no_fuse ? 1 : 0) << 23) | (t.pair << 24);
   return UASD_OK;
 }
 
