@@ -292,3 +292,31 @@ def test_tuning_reports_what_is_launched(L, shells, want):
     assert eng.tuning(eng.TUNE_LLG) == want
     eng.set_tuning(eng.TUNE_FIELD, 16, 128)
     assert eng.tuning(eng.TUNE_FIELD) == (16, 128)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [250, 2000])
+def test_short_calls_draw_in_the_predictor(n, precision):
+    """Calls of one Philox step, or of too few for a launch of their deviates to
+    be repaid, and such a rest of a longer call, are half steps that draw for
+    themselves; the moments are those of one long call."""
+    s = _chain(n)
+    out = []
+    for calls in ((1, 5, 1, 1, 70, 6), (84,)):
+        eng = U.Engine(n, 1, precision)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(n, np.random.default_rng(3), 1), s["mmom"][None])
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 5)
+        for k in calls:
+            before = eng.launch_counts()
+            eng.sd_steps(5, k)
+            c = {key: v - before[key] for key, v in eng.launch_counts().items()}
+            if n == 250:        # resident from two steps on, in launches of up to 64
+                assert c["llg_list"] == (2 if k == 1 else 0)
+                assert c["draw"] == c["llg_resident"] == (0 if k == 1 else (k + 63) // 64)
+            else:               # groups of 16 steps, a rest of 6 or more
+                assert c["llg_list"] == 2 * k
+                assert c["draw"] == (k // 16 + (k % 16 >= 6) if precision == "fp64" else 0)
+        out.append(eng.get_moments()[0])
+    assert np.array_equal(out[0], out[1])

@@ -910,7 +910,13 @@ bool llg_use_resident(const uasd_ctx *c) {
 // leaves CUs idle, of its time: midpoint and Depondt steps of 432 to 16,000
 // sites with 14 or 58 neighbours gain 0.3-0.8 us of 11-18.  At 65,536 sites
 // the extra pass over them costs what it saves, and FP32 deviates are too
-// cheap to gain at any size.
+// cheap to gain at any size.  The extra launch wants a group of at least
+// kDrawGroup steps to repay it: Depondt with 14 neighbours, us a step drawn in
+// the predictor, in groups of 2, 4, 6, 16: 686 sites 11.7, 12.4, 11.6, 11.3,
+// 11.0; 16,000 sites 11.8, 12.6, 11.8, 11.6, 11.3; 32,500 sites 12.6, 13.5,
+// 12.9, 12.7, 12.4.
+constexpr int kDrawGroup = 6;
+
 int steps_ahead(const uasd_ctx *c) {
   return c->prec == UASD_FP64 && (int64_t)c->N * c->M <= 32768 ? 16 : 1;
 }
@@ -2004,14 +2010,14 @@ int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
   if (launched_tile(c)) K = 1;  // the tile kernels draw their own deviates
   for (int64_t s = 0; s < n; ++s) {
     const int k = (int)(s % K);
+    const int group = (int)std::min<int64_t>(K, n - (s - k));  // steps drawn with this one
     const int64_t off = in_graph ? s : -1;
-    if (K > 1 && k == 0) {
-      const int m = (int)std::min<int64_t>(K, n - s);
-      const int r = c->prec == UASD_FP64 ? draw_ahead<double>(c, m, off)
-                                         : draw_ahead<float>(c, m, off);
+    if (group >= kDrawGroup && k == 0) {
+      const int r = c->prec == UASD_FP64 ? draw_ahead<double>(c, group, off)
+                                         : draw_ahead<float>(c, group, off);
       if (r) return r;
     }
-    if (int r = llg_step(c, alg, off, K > 1 ? k : -1)) return r;
+    if (int r = llg_step(c, alg, off, group >= kDrawGroup ? k : -1)) return r;
     if (!in_graph) c->step += 1;
   }
   return UASD_OK;
@@ -2048,6 +2054,10 @@ int llg_resident_steps(uasd_ctx *c, int alg, int64_t nsteps) {
   const int64_t chunk = resident_steps(c);
   for (int64_t s = 0; s < nsteps; s += chunk) {
     const int n = (int)std::min(chunk, nsteps - s);
+    // a single step: its draw and the resident launch take longer than the
+    // two half steps (432 sites FP64 14.7 against 11.8 us, FP32 12.5 against
+    // 10.4); two steps are faster (10.3, 8.4)
+    if (philox && n == 1) return llg_steps(c, alg, 1, false);
     if (philox)
       if (int r = draw_ahead<R>(c, n, -1)) return r;
     uasd::LLGDev<R> prm = llg_view<R>(c);
