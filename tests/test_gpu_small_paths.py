@@ -320,3 +320,39 @@ def test_short_calls_draw_in_the_predictor(n, precision):
                 assert c["draw"] == (k // 16 + (k % 16 >= 6) if precision == "fp64" else 0)
         out.append(eng.get_moments()[0])
     assert np.array_equal(out[0], out[1])
+
+
+def _rings(n, R):
+    """R rings of n sites (single sites for n = 1)."""
+    i = np.arange(n * R)
+    b, k = i // n * n, i % n
+    nl = np.stack([b + (k + 1) % n, b + (k - 1) % n], axis=1).astype(np.int32) + 1
+    return dict(nlist=nl, nlistsize=np.full(n * R, 2 if n > 1 else 0, np.int32),
+                ncoup=np.full((n * R, 2), 3.0))
+
+
+@pytest.mark.parametrize("kind,precision,n,R,M,resident", [
+    ("llg", "fp64", 1, 2048, 1, True), ("llg", "fp64", 1, 2049, 1, False),
+    ("llg", "fp32", 4, 512, 8, True), ("llg", "fp32", 4, 513, 8, False),
+    ("llg", "fp64", 64, 256, 8, True), ("llg", "fp64", 65, 252, 8, False),
+    ("H", "fp64", 1, 2048, 1, True), ("H", "fp32", 1, 2049, 1, False),
+    ("M", "fp64", 4, 2049, 1, False), ("M", "fp32", 4, 2048, 4, True),
+    ("M", "fp32", 4, 2049, 4, False), ("H", "fp64", 64, 1024, 4, True),
+    ("H", "fp64", 64, 1025, 4, False)])
+def test_batches_of_many_tiny_systems_are_launched(kind, precision, n, R, M, resident):
+    """A system takes a workgroup of at least one wavefront: batches of more
+    wavefronts than the rule allows go half step by half step, colour by colour."""
+    s = _rings(n, R)
+    eng = U.Engine(n * R, M, precision)
+    eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+    eng.set_moments(CF.random_unit(n * R, np.random.default_rng(2), M), np.ones((M, n * R)))
+    if kind == "llg":
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+        eng.sd_steps(5, 8)
+    else:
+        eng.mc_sweeps(kind, np.full(M, 300.0), 3, 9)
+    c = eng.launch_counts()
+    ran = c["llg_resident"] if kind == "llg" else c["mc_resident"]
+    launched = c["llg_list"] if kind == "llg" else c["mc_colour"]
+    assert (ran > 0, launched == 0) == (resident, resident), c

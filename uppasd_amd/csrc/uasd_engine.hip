@@ -893,12 +893,19 @@ int build_llg_resident(uasd_ctx *c) {
 // 432 sites 11.3 -> 5.0 (11.3 -> 3.8), Depondt 12.4 -> 5.8, 58 neighbours 22.8
 // -> 11.3 (18.2 -> 7.5), SIB 17.1 -> 12.9; 64 ensembles of 432 sites 13.1 ->
 // 6.5.  With 1024 sites the one CU is as slow as the launches (58 neighbours
-// 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  Not while the kernels
+// 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  At most 2048 wavefronts in
+// FP64 and 4096 in FP32: Depondt, launches against resident, sites x systems, 64
+// x 2048 (2048 wavefronts) FP64 12.0 -> 10.9 us, FP32 8.0 -> 7.8; 32 x 4096
+// (4096) 12.0 -> 12.7, 8.0 -> 8.3; 4 x 4096 (4096) 6.9 -> 7.8, 6.4 -> 4.4; 16 x
+// 8192 (8192) 12.0 -> 17.8, 8.0 -> 11.4; 1 x 131,072 11.2 -> 167, 7.4 -> 86.
+// Not while the kernels
 // are timed one by one, graphs were asked for or a launch shape was: a shape
 // is one of the kernels that the resident launch would take the place of.
 bool llg_can_be_resident(const uasd_ctx *c) {
   return c->lres.ok && c->lres.cls_version == c->cls_version && c->graph_steps == 0 &&
-         (int64_t)c->N * c->M <= kLlgResItems;
+         (int64_t)c->N * c->M <= kLlgResItems &&
+         uasd::res_waves((int64_t)c->lres.ncomp * c->M, c->lres.nmax) <=
+             (c->prec == UASD_FP32 ? 4096 : 2048);
 }
 
 bool llg_use_resident(const uasd_ctx *c) {
@@ -2258,14 +2265,25 @@ static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed
 //    (1024 ensembles of 2000 sites, 9 colours) 158 -> 113 us a sweep, at 262k
 //    (alloy pairs of 1024 sites, 256 ensembles, 2 colours) 29 -> 21 us; at
 //    600k (64 alloys, 32 ensembles) 54 -> 61 us, slower.
+//  - Wavefronts (res_waves; sites per system, systems): 2048 where less than
+//    half of a phase's lanes have a site (FP64 heat bath 4 x 4096 in 4096
+//    wavefronts 8.2 -> 9.7 us a sweep, Metropolis 10.9 -> 11.5, 16 x 1024 in 1024
+//    8.2 -> 5.3, 11.0 -> 6.2; 2 x 262,144 16.2 -> 457), 4096 otherwise (heat bath
+//    256 x 2048 in 4096 16.7 -> 12.1, 64 x 8192 in 8192 16.7 -> 17.3), 8192 in
+//    FP32 Metropolis with its cheap moves (2 x 8192 7.7 -> 6.7, 64 x 8192 12.2 ->
+//    7.9, 16 x 32,768 in 32,768 12.3 -> 23.7).
 // Not where a launch shape was asked for: it is one of the colour pass.
-static bool mc_can_be_resident(const uasd_ctx *c) {
-  return c->res.ok && c->res.nmax <= uasd::kResThreads * c->ncolors &&
-         (int64_t)c->N * c->M <= (int64_t)c->ncolors << 18;
+static bool mc_can_be_resident(const uasd_ctx *c, bool heat_bath) {
+  if (!c->res.ok || c->res.nmax > uasd::kResThreads * c->ncolors) return false;
+  const int64_t items = (int64_t)c->N * c->M, col = c->ncolors;
+  const int64_t waves = uasd::res_waves((int64_t)c->res.ncomp * c->M, c->res.dev.cmax);
+  const bool full = 2 * items >= 64 * col * waves;  // half of a phase's lanes and more
+  const int64_t most = c->prec == UASD_FP32 && !heat_bath ? 8192 : full ? 4096 : 2048;
+  return items <= col << 18 && waves <= most;
 }
 
-static bool mc_use_resident(const uasd_ctx *c) {
-  return mc_can_be_resident(c) && c->tune[2].chosen != uasd::kShapeAsked;
+static bool mc_use_resident(const uasd_ctx *c, bool heat_bath) {
+  return mc_can_be_resident(c, heat_bath) && c->tune[2].chosen != uasd::kShapeAsked;
 }
 
 // nsweeps sweeps in resident launches of at most kResSweeps, from mp.sweep on.
@@ -2299,7 +2317,7 @@ static uasd::Tune mc_tune(const uasd_ctx *c, int nsites) {
 // nsweeps colour-ordered sweeps; every launch is asynchronous on the stream.
 static int mc_run(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
   const int *sites_dev = mp.sites;
-  if (mc_use_resident(c)) {
+  if (mc_use_resident(c, mp.heat_bath)) {
     mp.sweep = c->mc_sweep;
     if (int r = mc_resident(c, mp, nsweeps)) return r;
     c->mc_sweep += (uint64_t)nsweeps;
@@ -2349,7 +2367,7 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
     auto body = [&]() -> int {
       uasd::MCParams g = mp;
       g.sweep_dev = c->ctr.as<uint64_t>() + 1;
-      const bool resident = mc_use_resident(c);
+      const bool resident = mc_use_resident(c, mp.heat_bath);
       if (resident) {
         g.sweep = 0;
         if (int r = mc_resident(c, g, K)) return r;
@@ -2381,7 +2399,7 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
   };
   if (c->graph_steps > 0) {
     if (int r = replay(c->graph_steps)) return r;
-  } else if (!mc_use_resident(c) &&
+  } else if (!mc_use_resident(c, mp.heat_bath) &&
              repeats_pay(c, 1, mode, seed, (int64_t)c->N * c->M / std::max(c->ncolors, 1),
                          nsweeps, 512)) {
     for (int K : {16, 4})
@@ -2681,7 +2699,7 @@ int uasd_autotune_mc(uasd_ctx *c, char mode, const double *temps, int sweeps, do
   uasd::MCParams mp;
   if (int r = mc_prepare(c, mode, temps, 0x7u, mp)) return r;
   const std::string key = tune_key(c, "mc", (int)mode);
-  const bool resident = mc_can_be_resident(c);
+  const bool resident = mc_can_be_resident(c, mp.heat_bath);
   uasd::Tune cached;
   double cached_ms = 0.0;
   if (tune_cached(key, resident, &cached, cached_ms) && cached.tile == 0) {

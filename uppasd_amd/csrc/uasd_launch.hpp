@@ -3,6 +3,7 @@
 // translation unit (uasd_kernels_f64.hip / uasd_kernels_f32.hip) so the FP64
 // unit can be compiled without multiply-add contraction.
 #pragma once
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -112,6 +113,14 @@ template <typename R>
 hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fused,
                       const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p,
                       Quad<R> *b2, const Quad<R> *beff, Quad<R> *out);
+
+// Wavefronts of a resident launch: at least one per system, however few sites
+// it has, each of them idle but for the sites it got.  Batches of many tiny
+// systems are faster half step by half step or colour by colour, with full
+// wavefronts, hence a limit (`sites` of a system are worked on at once).
+inline int64_t res_waves(int64_t systems, int sites) {
+  return systems * ((std::min(sites, kResThreads) + 63) / 64);
+}
 
 // nsteps LLG steps of every system with k_llg_resident; Philox deviates in
 // prm.nsave, lds = LDS bytes a workgroup may use.
