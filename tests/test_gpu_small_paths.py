@@ -356,3 +356,30 @@ def test_batches_of_many_tiny_systems_are_launched(kind, precision, n, R, M, res
     ran = c["llg_resident"] if kind == "llg" else c["mc_resident"]
     launched = c["llg_list"] if kind == "llg" else c["mc_colour"]
     assert (ran > 0, launched == 0) == (resident, resident), c
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("kind,L,M", [("M", (8, 8, 8), 257), ("H", (8, 8, 8), 257)])
+def test_more_systems_than_lists_in_lds_allow(kind, L, M, precision):
+    """257 systems whose lists would leave one workgroup a CU (256 CUs): the
+    lists stay in global memory, the moments are those of the launched kernels."""
+    s = CF.bcc_shells(L, CF.bcc5_couplings(), moment=2.2)
+    N, out = s["lattice"].natom, []
+    for asked in (False, True):
+        eng = U.Engine(N, M, precision)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(2), M),
+                        np.broadcast_to(s["mmom"], (M, N)))
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+        if asked:
+            eng.set_tuning(eng.TUNE_LLG, 8, 64)
+            eng.set_tuning(eng.TUNE_MC, 8, 64)
+        if kind == "llg":
+            eng.sd_steps(1, 5)
+        else:
+            eng.mc_sweeps(kind, np.linspace(100.0, 1500.0, M), 3, 9)
+        c = eng.launch_counts()
+        assert (c["llg_resident"] + c["mc_resident"] > 0) != asked
+        out.append(eng.get_moments()[0])
+    assert np.array_equal(out[0], out[1])

@@ -122,6 +122,22 @@ inline int64_t res_waves(int64_t systems, int sites) {
   return systems * ((std::min(sites, kResThreads) + 63) / 64);
 }
 
+// Whether a resident launch keeps its lists in LDS beside `base` bytes of
+// state: where they fit and do not make the workgroups take turns on a CU that
+// would hold several at once without them (`lds` bytes and sixteen wavefronts a
+// CU, 256 CUs).  1000 systems of 1024 sites with 58 neighbours, lists of 119 KB in
+// LDS (one workgroup a CU, four rounds) -> in global memory, us a sweep: FP32
+// Metropolis 327 -> 83, heat bath 370 -> 88, FP64 360 -> 86 (colour by colour
+// 180, 186, 283); 260 systems 97 -> 63, 186 -> 80, 169 -> 79.
+inline bool res_lists_in_lds(int64_t systems, int threads, size_t base, size_t lists, size_t lds) {
+  if (base + lists > lds) return false;
+  auto rounds = [&](size_t bytes) {
+    const int64_t cu = std::min<int64_t>(lds / std::max<size_t>(bytes, 1), 1024 / threads);
+    return (systems + 256 * cu - 1) / (256 * cu);
+  };
+  return rounds(base + lists) <= rounds(base);
+}
+
 // nsteps LLG steps of every system with k_llg_resident; Philox deviates in
 // prm.nsave, lds = LDS bytes a workgroup may use.
 template <typename R>
