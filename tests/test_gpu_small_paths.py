@@ -332,13 +332,14 @@ def _rings(n, R):
 
 
 @pytest.mark.parametrize("kind,precision,n,R,M,resident", [
-    ("llg", "fp64", 1, 2048, 1, True), ("llg", "fp64", 1, 2049, 1, False),
-    ("llg", "fp32", 4, 512, 8, True), ("llg", "fp32", 4, 513, 8, False),
+    ("llg", "fp64", 1, 2069, 1, True), ("llg", "fp64", 1, 2070, 1, False),
+    ("llg", "fp32", 4, 529, 8, True), ("llg", "fp32", 4, 530, 8, False),
     ("llg", "fp64", 64, 256, 8, True), ("llg", "fp64", 65, 252, 8, False),
-    ("H", "fp64", 1, 2048, 1, True), ("H", "fp32", 1, 2049, 1, False),
-    ("M", "fp64", 4, 2049, 1, False), ("M", "fp32", 4, 2048, 4, True),
-    ("M", "fp32", 4, 2049, 4, False), ("H", "fp64", 64, 1024, 4, True),
-    ("H", "fp64", 64, 1025, 4, False)])
+    ("llg", "fp64", 32, 510, 8, False),
+    ("H", "fp64", 2, 3059, 1, True), ("H", "fp32", 2, 3060, 1, False),
+    ("M", "fp64", 4, 1560, 2, True), ("M", "fp64", 4, 1561, 2, False),
+    ("M", "fp32", 4, 2341, 4, True), ("M", "fp32", 4, 2342, 4, False),
+    ("H", "fp64", 256, 512, 4, True), ("H", "fp64", 64, 2048, 4, False)])
 def test_batches_of_many_tiny_systems_are_launched(kind, precision, n, R, M, resident):
     """A system takes a workgroup of at least one wavefront: batches of more
     wavefronts than the rule allows go half step by half step, colour by colour."""
@@ -359,7 +360,8 @@ def test_batches_of_many_tiny_systems_are_launched(kind, precision, n, R, M, res
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
-@pytest.mark.parametrize("kind,L,M", [("M", (8, 8, 8), 257), ("H", (8, 8, 8), 257)])
+@pytest.mark.parametrize("kind,L,M", [("M", (8, 8, 8), 257), ("H", (8, 8, 8), 257),
+                                      ("llg", (6, 7, 6), 257)])
 def test_more_systems_than_lists_in_lds_allow(kind, L, M, precision):
     """257 systems whose lists would leave one workgroup a CU (256 CUs): the
     lists stay in global memory, the moments are those of the launched kernels."""

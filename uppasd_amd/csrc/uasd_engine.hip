@@ -264,6 +264,7 @@ struct uasd_ctx {
   struct Resident {
     bool ok = false;
     int ncomp = 0, nmax = 0;
+    int64_t waves = 0;  // of one ensemble: of a half step; of all colours of a sweep
     DevBuf buf;
     uasd::ResDev dev{};
     int64_t cls_version = -1;
@@ -883,6 +884,9 @@ int build_llg_resident(uasd_ctx *c) {
   r.dev.dnbr = r.dev.nbr + (size_t)W * N;
   r.ncomp = ncomp;
   r.nmax = nmax;
+  r.waves = 0;
+  for (int k = 0; k < ncomp; ++k)
+    r.waves += uasd::res_waves(off[k + 1] - off[k], (nmax + 63) / 64);
   r.ok = true;
   return UASD_OK;
 }
@@ -893,19 +897,21 @@ int build_llg_resident(uasd_ctx *c) {
 // 432 sites 11.3 -> 5.0 (11.3 -> 3.8), Depondt 12.4 -> 5.8, 58 neighbours 22.8
 // -> 11.3 (18.2 -> 7.5), SIB 17.1 -> 12.9; 64 ensembles of 432 sites 13.1 ->
 // 6.5.  With 1024 sites the one CU is as slow as the launches (58 neighbours
-// 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  At most 2048 wavefronts in
-// FP64 and 4096 in FP32: Depondt, launches against resident, sites x systems, 64
-// x 2048 (2048 wavefronts) FP64 12.0 -> 10.9 us, FP32 8.0 -> 7.8; 32 x 4096
-// (4096) 12.0 -> 12.7, 8.0 -> 8.3; 4 x 4096 (4096) 6.9 -> 7.8, 6.4 -> 4.4; 16 x
-// 8192 (8192) 12.0 -> 17.8, 8.0 -> 11.4; 1 x 131,072 11.2 -> 167, 7.4 -> 86.
+// 22.5 -> 22.5, film 13.7 -> 13.9, SIB 17.4 -> 24.0).  Fewer than 2040 idle
+// wavefronts in FP64 and 4000 in FP32: Depondt, launches against resident, sites
+// x systems, idle wavefronts in brackets, 64 x 2048 (205) FP64 12.0 -> 10.9 us,
+// FP32 8.0 -> 7.8; 250 x 520 (252) 21.0 -> 14.0, 15.6 -> 10.3; 100 x 1280 (760)
+// 12.1 -> 10.7, 8.0 -> 8.0; 65 x 2016 (2189) 12.1 -> 13.9, 8.4 -> 8.5; 1 x 2048
+// (2019) 5.6 -> 3.6, 5.7 -> 2.4; 4 x 4096 (3866) 6.9 -> 7.8, 6.4 -> 4.4; 16 x 8192
+// (6349) 12.0 -> 17.8, 8.0 -> 11.4; 1 x 131,072 11.2 -> 167, 7.4 -> 86.
 // Not while the kernels
 // are timed one by one, graphs were asked for or a launch shape was: a shape
 // is one of the kernels that the resident launch would take the place of.
 bool llg_can_be_resident(const uasd_ctx *c) {
   return c->lres.ok && c->lres.cls_version == c->cls_version && c->graph_steps == 0 &&
          (int64_t)c->N * c->M <= kLlgResItems &&
-         uasd::res_waves((int64_t)c->lres.ncomp * c->M, c->lres.nmax) <=
-             (c->prec == UASD_FP32 ? 4096 : 2048);
+         uasd::res_idle_waves(c->lres.waves * c->M, (int64_t)c->N * c->M, 0.9) <
+             (c->prec == UASD_FP32 ? 4000 : 2040);
 }
 
 bool llg_use_resident(const uasd_ctx *c) {
@@ -2204,6 +2210,13 @@ static int build_resident(uasd_ctx *c) {
                        reinterpret_cast<const uint16_t *>(base + onb) + (size_t)W * N};
   r.ncomp = ncomp;
   r.nmax = nmax;
+  r.waves = 0;
+  const int slots = (std::min(cmax, uasd::kResThreads) + 63) / 64;
+  for (int k = 0; k < ncomp; ++k)
+    for (int q = 0; q < ncol; ++q) {
+      const int *pc = ptr.data() + (size_t)k * (ncol + 1) + q;
+      r.waves += uasd::res_waves(pc[1] - pc[0], slots);
+    }
   r.ok = true;
   c->gen += 1;  // captured sweeps hold the old tables
   return UASD_OK;
@@ -2265,21 +2278,20 @@ static int mc_prepare(uasd_ctx *c, char mode, const double *temps, uint64_t seed
 //    (1024 ensembles of 2000 sites, 9 colours) 158 -> 113 us a sweep, at 262k
 //    (alloy pairs of 1024 sites, 256 ensembles, 2 colours) 29 -> 21 us; at
 //    600k (64 alloys, 32 ensembles) 54 -> 61 us, slower.
-//  - Wavefronts (res_waves; sites per system, systems): 2048 where less than
-//    half of a phase's lanes have a site (FP64 heat bath 4 x 4096 in 4096
-//    wavefronts 8.2 -> 9.7 us a sweep, Metropolis 10.9 -> 11.5, 16 x 1024 in 1024
-//    8.2 -> 5.3, 11.0 -> 6.2; 2 x 262,144 16.2 -> 457), 4096 otherwise (heat bath
-//    256 x 2048 in 4096 16.7 -> 12.1, 64 x 8192 in 8192 16.7 -> 17.3), 8192 in
-//    FP32 Metropolis with its cheap moves (2 x 8192 7.7 -> 6.7, 64 x 8192 12.2 ->
-//    7.9, 16 x 32,768 in 32,768 12.3 -> 23.7).
+//  - Fewer than 3000 idle wavefronts a phase (9000 in FP32 Metropolis with its
+//    cheap moves): a phase of resident launches is 1.7 us and 0.8 ns a wavefront
+//    longer, a launched colour 4-5 us and 16 ns per 1000 updates, 1.0 ns a full
+//    wavefront.  Heat bath FP64, launches against resident, sites x systems, idle
+//    wavefronts in brackets: 16 x 1024 (864) 8.2 -> 5.3 us a sweep, 256 x 2048
+//    (none) 16.7 -> 12.1, 64 x 8192 (3072) 16.7 -> 17.3, 4 x 4096 (3936) 8.2 ->
+//    9.7, 2 x 262,144 16.2 -> 457; FP32 Metropolis 64 x 8192 12.2 -> 7.9, 2 x 8192
+//    (8032) 7.7 -> 6.7, 16 x 32,768 (27,648) 12.3 -> 23.7.
 // Not where a launch shape was asked for: it is one of the colour pass.
 static bool mc_can_be_resident(const uasd_ctx *c, bool heat_bath) {
   if (!c->res.ok || c->res.nmax > uasd::kResThreads * c->ncolors) return false;
   const int64_t items = (int64_t)c->N * c->M, col = c->ncolors;
-  const int64_t waves = uasd::res_waves((int64_t)c->res.ncomp * c->M, c->res.dev.cmax);
-  const bool full = 2 * items >= 64 * col * waves;  // half of a phase's lanes and more
-  const int64_t most = c->prec == UASD_FP32 && !heat_bath ? 8192 : full ? 4096 : 2048;
-  return items <= col << 18 && waves <= most;
+  const double idle = uasd::res_idle_waves(c->res.waves * c->M / col, items / col, 1.25);
+  return items <= col << 18 && idle < (c->prec == UASD_FP32 && !heat_bath ? 9000 : 3000);
 }
 
 static bool mc_use_resident(const uasd_ctx *c, bool heat_bath) {

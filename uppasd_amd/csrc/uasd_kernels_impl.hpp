@@ -145,7 +145,7 @@ hipError_t launch_llg_resident(hipStream_t s, int alg, const HamDev<R> &h, const
   const size_t base = res_lds_llg(sizeof(R), rd.nmax), lists = 2 * (size_t)rd.nmax * (h.W + h.Wd);
   if (base > lds || nsteps <= 0) return hipErrorInvalidValue;
   const int threads = std::min(kResThreads, (rd.nmax + 63) / 64 * 64);
-  const bool lnb = res_lists_in_lds((int64_t)rd.ncomp * h.M, threads, base, lists, lds);
+  const bool lnb = res_lists_in_lds((int64_t)rd.ncomp * h.M, threads, 16, base, lists, lds);
   const size_t bytes = base + (lnb ? lists : 0);
 #define UASD_RES_CASE(A)                                                                       \
   if (alg == A)                                                                                \
@@ -188,7 +188,8 @@ hipError_t launch_mc_resident(hipStream_t s, const HamDev<R> &h, const MCParams 
   // the trials of a sweep in LDS where they fit, then the lists
   const bool trl = !mp.heat_bath && sp + tr <= lds;
   const size_t base = sp + (trl ? tr : 0);
-  const bool lnb = res_lists_in_lds((int64_t)rd.ncomp * h.M, threads, base, lists, lds);
+  const int cu_waves = sizeof(R) == 8 && !mp.heat_bath ? 8 : 16;
+  const bool lnb = res_lists_in_lds((int64_t)rd.ncomp * h.M, threads, cu_waves, base, lists, lds);
   const size_t bytes = base - 16 + (lnb ? lists : 0);  // the counters are static
 #define UASD_RES_CASE(HB_, TRL_, LNB_)                                                          \
   if ((mp.heat_bath != 0) == HB_ && trl == TRL_ && lnb == LNB_)                                 \

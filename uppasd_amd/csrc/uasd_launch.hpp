@@ -114,25 +114,35 @@ hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fuse
                       const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p,
                       Quad<R> *b2, const Quad<R> *beff, Quad<R> *out);
 
-// Wavefronts of a resident launch: at least one per system, however few sites
-// it has, each of them idle but for the sites it got.  Batches of many tiny
-// systems are faster half step by half step or colour by colour, with full
-// wavefronts, hence a limit (`sites` of a system are worked on at once).
-inline int64_t res_waves(int64_t systems, int sites) {
-  return systems * ((std::min(sites, kResThreads) + 63) / 64);
+// Wavefronts that one phase of a system (a colour, a half step) of `sites`
+// sites takes in a workgroup of `slots` wavefronts: at least one, and a quarter
+// of the workgroup's, whose slots stay taken.
+inline int res_waves(int sites, int slots) {
+  return std::max({1, (sites + 63) / 64, slots / 4});
+}
+
+// Wavefronts of a phase (res_waves over all systems) less `weight` times the
+// full ones that `items` sites would make: the idle share of a resident launch.
+// A system takes a workgroup of at least one wavefront however few sites it
+// has, so batches of many tiny systems are faster half step by half step or
+// colour by colour; the callers' comments have the limits and their figures.
+inline double res_idle_waves(int64_t waves, int64_t items, double weight) {
+  return (double)waves - weight * (double)items / 64.0;
 }
 
 // Whether a resident launch keeps its lists in LDS beside `base` bytes of
 // state: where they fit and do not make the workgroups take turns on a CU that
-// would hold several at once without them (`lds` bytes and sixteen wavefronts a
-// CU, 256 CUs).  1000 systems of 1024 sites with 58 neighbours, lists of 119 KB in
+// would hold several at once without them (`lds` bytes and `cu_waves` wavefronts
+// a CU, which the kernel's registers allow; 256 CUs).  1000 systems of 1024 sites with 58 neighbours, lists of 119 KB in
 // LDS (one workgroup a CU, four rounds) -> in global memory, us a sweep: FP32
 // Metropolis 327 -> 83, heat bath 370 -> 88, FP64 360 -> 86 (colour by colour
 // 180, 186, 283); 260 systems 97 -> 63, 186 -> 80, 169 -> 79.
-inline bool res_lists_in_lds(int64_t systems, int threads, size_t base, size_t lists, size_t lds) {
+inline bool res_lists_in_lds(int64_t systems, int threads, int cu_waves, size_t base,
+                             size_t lists, size_t lds) {
   if (base + lists > lds) return false;
   auto rounds = [&](size_t bytes) {
-    const int64_t cu = std::min<int64_t>(lds / std::max<size_t>(bytes, 1), 1024 / threads);
+    const int64_t cu =
+        std::min<int64_t>(lds / std::max<size_t>(bytes, 1), std::max(1, 64 * cu_waves / threads));
     return (systems + 256 * cu - 1) / (256 * cu);
   };
   return rounds(base + lists) <= rounds(base);
