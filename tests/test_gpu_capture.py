@@ -77,3 +77,80 @@ def test_captured_steps_between_longer_calls(precision):
         assert np.array_equal(a.get_moments()[0], e), n
         b.sd_steps(5, at - 4)                         # the counter where a's is
         b.set_moments(e, mm)
+
+
+def _chain_engine(n, stream=None):
+    """A ring of n sites: too many for resident launches, few enough for replays."""
+    i = np.arange(n)
+    nl = np.stack([(i + 1) % n + 1, (i - 1) % n + 1], axis=1).astype(np.int32)
+    eng = U.Engine(n, 1)
+    if stream is not None:
+        eng.set_stream(stream)
+    eng.set_exchange(nl, np.full(n, 2, np.int32), np.full((n, 2), 3.0))
+    eng.set_moments(CF.random_unit(n, np.random.default_rng(3), 1), np.ones((1, n)))
+    eng.set_llg(0.1, 300.0, 1e-16)
+    eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+    return eng
+
+
+RUNS = {"llg": (1000, lambda e, k: e.sd_steps(5, 64 * k), 32, "llg_list"),
+        "mc": (12000, lambda e, k: e.mc_sweeps("M", 400.0, 16 * k, 5), 32, "mc_colour")}
+
+
+def _stream(kind):
+    """A caller's stream: its own, or the legacy stream, which cannot be captured."""
+    if kind == "legacy":
+        return 1
+    s = C.c_void_p()
+    assert _hip().hipStreamCreate(C.byref(s)) == 0
+    return s.value
+
+
+@pytest.mark.parametrize("what", list(RUNS))
+@pytest.mark.parametrize("kind", ["own", "blocking", "legacy"])
+def test_repeats_on_any_stream(kind, what):
+    """Steps and sweeps that repeat go on where they would be replayed, on every
+    stream a caller may give, with the same results; the context's own stream
+    and ordinary ones are replayed."""
+    n, run, before, single = RUNS[what]
+    ref = _chain_engine(n)
+    ref.set_kernel_timing(True)                        # single launches throughout
+    eng = _chain_engine(n, None if kind == "own" else _stream(kind))
+    for k in (before, 3, 2):
+        run(ref, k)
+        run(eng, k)
+        assert np.array_equal(eng.get_moments()[0], ref.get_moments()[0]), k
+    replays = eng.launch_counts()[what + "_graph"]
+    assert ref.launch_counts()[what + "_graph"] == 0
+    assert replays == 5 or (kind == "legacy" and replays == 0)
+    print(kind, what, eng.launch_counts())
+
+
+def test_failed_automatic_capture_goes_on_with_launches():
+    """The stream that automatic replays are recorded on is made busy with a
+    capture of the test's own: the call launches as before, and the context
+    does not try again until it is given another stream."""
+    what = "llg"
+    n, run, before, single = RUNS[what]
+    ref = _chain_engine(n)
+    ref.set_kernel_timing(True)
+    eng = _chain_engine(n)
+    hip, own = _hip(), C.c_void_p(eng.stream())
+    eng.set_stream(_stream("blocking"))
+    for e in (ref, eng):
+        run(e, before)
+    eng.get_moments()
+    assert hip.hipStreamBeginCapture(own, 1) == 0
+    run(eng, 1)
+    g = C.c_void_p()
+    assert hip.hipStreamEndCapture(own, C.byref(g)) == 0
+    run(eng, 1)
+    assert eng.launch_counts()[what + "_graph"] == 0
+    for _ in range(2):
+        run(ref, 1)
+    assert np.array_equal(eng.get_moments()[0], ref.get_moments()[0])
+    eng.set_stream(_stream("blocking"))
+    run(eng, 1)
+    run(ref, 1)
+    assert eng.launch_counts()[what + "_graph"] == 1
+    assert np.array_equal(eng.get_moments()[0], ref.get_moments()[0])

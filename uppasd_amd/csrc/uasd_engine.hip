@@ -242,6 +242,7 @@ struct uasd_ctx {
   bool ctr_valid[2] = {false, false};
   uint64_t ctr_val[2] = {0, 0};
   bool capturing = false;
+  bool replays_off = false;   // an automatic replay failed on this stream
   struct Graph {
     hipGraph_t g = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1436,6 +1437,9 @@ int uasd_ctx_create(uasd_ctx **out, int natom, int mensemble, int precision) {
   HIP_TRY(c->spins.ensure(2 * quad_bytes(c.get()) + (size_t)c->N * c->M * 4 * sizeof(double)));
   HIP_TRY(hipMemsetAsync(c->spins.p, 0, 3 * quad_bytes(c.get()), c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
+  // (here, not with the first replay, which may come unasked for: another
+  // thread's capture can forbid allocations)
+  HIP_TRY(c->ctr.ensure(2 * sizeof(uint64_t)));
   // the whole lattice as one segment until uasd_set_segments says otherwise
   if (int r = ensure_segments(c.get())) return r;
   *out = c.release();
@@ -1467,6 +1471,7 @@ int uasd_ctx_set_stream(uasd_ctx *c, void *s) {
   if (int r = check_ctx(c)) return r;
   HIP_TRY(hipStreamSynchronize(c->stream));
   c->stream = s ? static_cast<hipStream_t>(s) : c->own_stream;
+  c->replays_off = false;
   return UASD_OK;
 }
 
@@ -1898,14 +1903,20 @@ void destroy_graphs(uasd_ctx *c) {
 }
 
 // Records what body() enqueues on the context stream and instantiates it.
+// Graphs that nobody asked for are recorded on the context's own stream, which
+// nothing else uses or waits for: a caller's may not be capturable, or other
+// threads' work may be ordered with it.
 template <typename F>
 int capture_graph(uasd_ctx *c, F &&body, uasd_ctx::Graph &out) {
-  HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+  const hipStream_t run = c->stream, rec = c->graph_steps > 0 ? run : c->own_stream;
+  HIP_TRY(hipStreamBeginCapture(rec, hipStreamCaptureModeThreadLocal));
   c->capturing = true;
+  c->stream = rec;
   const int r = body();
+  c->stream = run;
   c->capturing = false;
   hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(c->stream, &g);
+  const hipError_t e = hipStreamEndCapture(rec, &g);
   if (r) {
     if (g) (void)hipGraphDestroy(g);
     return r;
@@ -1933,10 +1944,6 @@ int replay_graph(uasd_ctx *c, const std::tuple<int, int, int, uint64_t> &key, in
   if (c->graphs_gen != c->gen || c->graphs.size() > 16) {
     destroy_graphs(c);
     c->graphs_gen = c->gen;
-  }
-  if (!c->ctr.p) {
-    HIP_TRY(c->ctr.ensure(2 * sizeof(uint64_t)));
-    c->ctr_valid[0] = c->ctr_valid[1] = false;
   }
   auto it = c->graphs.find(key);
   if (it == c->graphs.end()) {
@@ -1983,6 +1990,21 @@ int uasd_sd_steps(uasd_ctx *c, int alg, int64_t nsteps) {
 }  // extern "C"
 
 namespace {
+
+// Whether the context stream is known not to be capturing.
+bool stream_free(uasd_ctx *c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // not known: the next launch's error is its own
+  return false;
+}
+
+// An automatic replay that failed: nothing of it ran, so the call goes on with
+// single launches, and no other replay is tried on this stream.
+void replay_failed(uasd_ctx *c) {
+  (void)hipGetLastError();
+  c->replays_off = true;
+}
 
 // One LLG step, both halves; step_off, ahead as in run_llg_half.
 int llg_step(uasd_ctx *c, int alg, int64_t step_off, int ahead) {
@@ -2049,10 +2071,8 @@ int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
 // `after`.
 bool repeats_pay(uasd_ctx *c, int kind, int alg, uint64_t seed, int64_t items, int64_t n,
                  int64_t after) {
-  if (c->graph_steps > 0 || c->timing || items > 131072) return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(c->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
-    return false;
+  if (c->graph_steps > 0 || c->timing || c->replays_off || items > 131072) return false;
+  if (!stream_free(c)) return false;
   if (c->repeats.size() > 64) c->repeats.clear();
   auto &r = c->repeats[std::make_tuple(kind, alg, seed)];
   if (r.first != c->gen) r = {c->gen, 0};
@@ -2084,11 +2104,10 @@ int llg_resident_steps(uasd_ctx *c, int alg, int64_t nsteps) {
 }
 
 int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps) {
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;  // a caller's own capture:
-  (void)hipStreamIsCapturing(c->stream, &cap);              // no tables, no growing buffers
-  if (cap == hipStreamCaptureStatusNone)
+  const bool open = stream_free(c);  // not in a caller's own capture, which takes no tables
+  if (open)
     if (int r = build_llg_resident(c)) return r;
-  if (cap == hipStreamCaptureStatusNone && llg_use_resident(c))
+  if (open && llg_use_resident(c))
     return c->prec == UASD_FP64 ? llg_resident_steps<double>(c, alg, nsteps)
                                 : llg_resident_steps<float>(c, alg, nsteps);
   int64_t s = 0;
@@ -2107,7 +2126,10 @@ int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps) {
     if (int r = replay(c->graph_steps)) return r;
   } else if (repeats_pay(c, 0, alg, 0, (int64_t)c->N * c->M, nsteps, 2048)) {
     for (int K : {64, 16})
-      if (int r = replay(K)) return r;
+      if (replay(K)) {
+        replay_failed(c);
+        break;
+      }
   }
   return llg_steps(c, alg, nsteps - s, false);
 }
@@ -2415,7 +2437,10 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
              repeats_pay(c, 1, mode, seed, (int64_t)c->N * c->M / std::max(c->ncolors, 1),
                          nsweeps, 512)) {
     for (int K : {16, 4})
-      if (int r = replay(K)) return r;
+      if (replay(K)) {
+        replay_failed(c);
+        break;
+      }
   }
   return mc_run(c, mp, nsweeps - s);
 }
