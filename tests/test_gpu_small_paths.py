@@ -385,3 +385,19 @@ def test_more_systems_than_lists_in_lds_allow(kind, L, M, precision):
         assert (c["llg_resident"] + c["mc_resident"] > 0) != asked
         out.append(eng.get_moments()[0])
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("kind,n,resident", [("M", 1024, True), ("H", 1026, False),
+                                             ("llg", 512, True), ("llg", 513, False)])
+def test_largest_resident_systems(kind, n, resident):
+    """Rings, whose closing bond spans the whole system, at the most sites that
+    resident launches take (512 a colour, 512 a half step) and beyond."""
+    s = _rings(n, 1)
+    eng = U.Engine(n, 1)
+    eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+    eng.set_moments(CF.random_unit(n, np.random.default_rng(2), 1), np.ones((1, n)))
+    eng.set_llg(0.1, 300.0, 1e-16)
+    eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+    eng.sd_steps(5, 8) if kind == "llg" else eng.mc_sweeps(kind, 300.0, 2, 9)
+    c = eng.launch_counts()
+    assert (c["llg_resident" if kind == "llg" else "mc_resident"] == 1) == resident

@@ -800,6 +800,20 @@ uasd::LLGDev<R> llg_view(uasd_ctx *c) {
   return p;
 }
 
+// Whether some bond spans `sites` slots or more, so that its system has more
+// sites than that.  In a periodic crystal that is larger the first site's does.
+bool bond_spans(const uasd_ctx *c, int sites) {
+  auto spans = [&](const std::vector<int> &row, const std::vector<int> &len,
+                   const std::vector<int> &list) {
+    for (int i = 0; i < c->N && !row.empty(); ++i)
+      for (int j = 0; row[i] >= 0 && j < len[row[i]]; ++j)
+        if (std::abs(list[(size_t)j * c->N + i] - i) >= sites) return true;
+    return false;
+  };
+  return spans(c->ex_row_of_site, c->ex_len_host, c->nbr_host) ||
+         (c->Wd > 0 && spans(c->dm_row_of_site, c->dm_len_host, c->dnbr_host));
+}
+
 // Contiguous ranges of device slots that no bond crosses, as first slots.
 std::vector<int> independent_ranges(const uasd_ctx *c) {
   const int N = c->N;
@@ -837,18 +851,7 @@ int build_llg_resident(uasd_ctx *c) {
   r.cls_version = c->cls_version;
   const int N = c->N, W = c->W, Wd = c->Wd;
   if (N > kLlgResLattice) return UASD_OK;
-  // a bond that spans more sites than a system may have ends the search, in a
-  // periodic crystal with its first site's
-  auto spans = [&](const std::vector<int> &row, const std::vector<int> &len,
-                   const std::vector<int> &list) {
-    for (int i = 0; i < N && !row.empty(); ++i)
-      for (int j = 0; row[i] >= 0 && j < len[row[i]]; ++j)
-        if (std::abs(list[(size_t)j * N + i] - i) >= kLlgResSites) return true;
-    return false;
-  };
-  if (spans(c->ex_row_of_site, c->ex_len_host, c->nbr_host) ||
-      (Wd > 0 && spans(c->dm_row_of_site, c->dm_len_host, c->dnbr_host)))
-    return UASD_OK;
+  if (bond_spans(c, kLlgResSites)) return UASD_OK;
   const std::vector<int> off = independent_ranges(c);
   const int ncomp = (int)off.size() - 1;
   int nmax = 0;
@@ -2168,6 +2171,13 @@ static int build_resident(uasd_ctx *c) {
   r.cls_version = c->cls_version;
   r.col_version = c->col_version;
   const int N = c->N, ncol = c->ncolors;
+  // the limits that need no look at the lists, or at a few bonds only, first
+  if ((int64_t)N * c->M > (int64_t)ncol << 18) return UASD_OK;
+  const size_t lds0 = uasd::res_lds_spins(c->rsize, 0);
+  const size_t most = std::min<size_t>(
+      (size_t)uasd::kResThreads * ncol,
+      ((size_t)c->lds_max - lds0) / (uasd::res_lds_spins(c->rsize, 1) - lds0));
+  if (bond_spans(c, (int)most)) return UASD_OK;
   const std::vector<int> off = independent_ranges(c);
   const int ncomp = (int)off.size() - 1;
   int nmax = 0;
