@@ -41,3 +41,26 @@ def test_field_of_host_moments(N, M, na):
     assert np.array_equal(b1, 2.0 * np.roll(eM, -1, axis=1))
     assert np.array_equal(b2, ext)
     assert np.array_equal(beff, b1 + b2)
+
+
+@pytest.mark.parametrize("precision,per_pair", [("fp64", 96), ("fp32", 48)])
+def test_context_holds_three_quads_a_pair(precision, per_pair):
+    """A new context's device memory is its three quad arrays: the staging of
+    the moments on their way in has no room of its own."""
+    import ctypes as C
+    import re
+    N = 1 << 24
+    small = U.Engine(1, 1)                       # the library and its device are up
+    hip = C.CDLL(re.search(r"\S*libamdhip64\.so\S*", open("/proc/self/maps").read()).group(0))
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+    before = free()
+    eng = U.Engine(N, 1, precision)
+    assert before - free() <= per_pair * N + (16 << 20)
+    e = np.random.default_rng(1).normal(size=(1, N, 3)).astype(np.float32).astype(np.float64)
+    eng.set_moments(e, np.ones((1, N)))
+    assert np.array_equal(eng.get_moments()[0], e)
+    small.close()

@@ -419,6 +419,9 @@ int upload_raw(uasd_ctx *c, DevBuf &dst, const std::vector<T> &src) {
 // at 65,536 spins 2.13 -> 1.55 ms, moments of 4.1e6 pairs read back 95 -> 34 ms.
 constexpr size_t kIoPairs = (size_t)1 << 22;
 
+// Host bytes of one pair in uasd_set_moments: its direction and magnitude.
+constexpr size_t kRawMoment = 4 * sizeof(double);
+
 // the w of the quads an upload writes
 struct PackW {
   int from_state = 0;  // 1: the moment magnitudes of the state's quads
@@ -1436,8 +1439,8 @@ int uasd_ctx_create(uasd_ctx **out, int natom, int mensemble, int precision) {
   if (int r = scratch_init(c->device)) return r;
   HIP_TRY(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
   c->stream = c->own_stream;
-  // (b2 has room for the raw doubles of uasd_set_moments in either precision)
-  HIP_TRY(c->spins.ensure(2 * quad_bytes(c.get()) + (size_t)c->N * c->M * 4 * sizeof(double)));
+  // (b2 has room for the raw doubles of one pair at least: uasd_set_moments)
+  HIP_TRY(c->spins.ensure(3 * quad_bytes(c.get()) + kRawMoment - 4 * c->rsize));
   HIP_TRY(hipMemsetAsync(c->spins.p, 0, 3 * quad_bytes(c.get()), c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   // (here, not with the first replay, which may come unasked for: another
@@ -1760,14 +1763,19 @@ int uasd_set_moments(uasd_ctx *c, const double *emom, const double *mmom) {
   io.open = true;
   // the raw arrays (32 bytes a pair) pass through the memory of b2eff, which
   // lasts no longer than a step: a call that every program makes once needs no
-  // staging of its own
+  // staging of its own.  In FP32 that is half of them at a time.
   const size_t pairs = (size_t)c->N * c->M;
+  const size_t step = (quad_bytes(c) + kRawMoment - 4 * c->rsize) / kRawMoment;
   double *sa = reinterpret_cast<double *>(static_cast<char *>(c->spins.p) + 2 * quad_bytes(c));
-  HIP_TRY(hipMemcpyAsync(sa, emom, 3 * pairs * sizeof(double), hipMemcpyHostToDevice, c->stream));
-  HIP_TRY(hipMemcpyAsync(sa + 3 * pairs, mmom, pairs * sizeof(double), hipMemcpyHostToDevice,
-                         c->stream));
-  // emom2 starts as emom
-  if (int r = launch_pack(c, c->spins, 0, 0, pairs, sa, sa + 3 * pairs, PackW{}, true)) return r;
+  for (size_t p0 = 0; p0 < pairs; p0 += step) {
+    const size_t n = std::min(step, pairs - p0);
+    HIP_TRY(hipMemcpyAsync(sa, emom + 3 * p0, 3 * n * sizeof(double), hipMemcpyHostToDevice,
+                           c->stream));
+    HIP_TRY(hipMemcpyAsync(sa + 3 * n, mmom + p0, n * sizeof(double), hipMemcpyHostToDevice,
+                           c->stream));
+    // emom2 starts as emom
+    if (int r = launch_pack(c, c->spins, 0, p0, n, sa, sa + 3 * n, PackW{}, true)) return r;
+  }
   if (int r = io.wait()) return r;
   c->have_state = true;
   const size_t nm = (size_t)c->N * c->M;
