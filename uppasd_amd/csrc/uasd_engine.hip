@@ -419,8 +419,14 @@ int upload_raw(uasd_ctx *c, DevBuf &dst, const std::vector<T> &src) {
 // at 65,536 spins 2.13 -> 1.55 ms, moments of 4.1e6 pairs read back 95 -> 34 ms.
 constexpr size_t kIoPairs = (size_t)1 << 22;
 
-// Host bytes of one pair in uasd_set_moments: its direction and magnitude.
+// Host bytes of one pair in uasd_set_moments, its direction and magnitude, and
+// the bytes of b2eff they pass through: its quads, which in FP32 hold half of
+// the pairs at a time, or all of up to 65,536 (a second pair of copies is 9 us).
 constexpr size_t kRawMoment = 4 * sizeof(double);
+size_t raw_room(const uasd_ctx *c) {
+  const size_t pairs = (size_t)c->N * c->M;
+  return std::max(quad_bytes(c), kRawMoment * std::min<size_t>(pairs, 65536));
+}
 
 // the w of the quads an upload writes
 struct PackW {
@@ -1439,8 +1445,7 @@ int uasd_ctx_create(uasd_ctx **out, int natom, int mensemble, int precision) {
   if (int r = scratch_init(c->device)) return r;
   HIP_TRY(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
   c->stream = c->own_stream;
-  // (b2 has room for the raw doubles of one pair at least: uasd_set_moments)
-  HIP_TRY(c->spins.ensure(3 * quad_bytes(c.get()) + kRawMoment - 4 * c->rsize));
+  HIP_TRY(c->spins.ensure(2 * quad_bytes(c.get()) + raw_room(c.get())));
   HIP_TRY(hipMemsetAsync(c->spins.p, 0, 3 * quad_bytes(c.get()), c->stream));
   HIP_TRY(hipStreamSynchronize(c->stream));
   // (here, not with the first replay, which may come unasked for: another
@@ -1763,9 +1768,8 @@ int uasd_set_moments(uasd_ctx *c, const double *emom, const double *mmom) {
   io.open = true;
   // the raw arrays (32 bytes a pair) pass through the memory of b2eff, which
   // lasts no longer than a step: a call that every program makes once needs no
-  // staging of its own.  In FP32 that is half of them at a time.
-  const size_t pairs = (size_t)c->N * c->M;
-  const size_t step = (quad_bytes(c) + kRawMoment - 4 * c->rsize) / kRawMoment;
+  // staging of its own
+  const size_t pairs = (size_t)c->N * c->M, step = raw_room(c) / kRawMoment;
   double *sa = reinterpret_cast<double *>(static_cast<char *>(c->spins.p) + 2 * quad_bytes(c));
   for (size_t p0 = 0; p0 < pairs; p0 += step) {
     const size_t n = std::min(step, pairs - p0);
