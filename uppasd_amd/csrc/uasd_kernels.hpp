@@ -417,7 +417,7 @@ struct NbDec1 {
   }
 };
 
-// Lists whose entries are the gather index itself (the resident MC kernel).
+// Lists whose entries are the gather index itself (the resident kernels).
 struct NbDecId {
   template <typename R>
   __device__ __forceinline__ NbDecId(const HamDev<R> &, int) {}
@@ -561,7 +561,7 @@ __device__ __forceinline__ void exchange_sum(const HamDev<R> &h, const I *__rest
 }
 
 // DM sum of site_field: field += m_j x D_ij (hamiltonianactions.f90:565-578).
-template <typename R, int G, typename I, typename D = NbDec, bool UNI = false>
+template <typename R, int G, typename I, typename D = NbDec>
 __device__ __forceinline__ void dm_sum(const HamDev<R> &h, const I *__restrict__ nb,
                                        const Quad<R> *__restrict__ src, int site, int ens,
                                        int row, R &s0, R &s1, R &s2) {
@@ -582,8 +582,7 @@ __device__ __forceinline__ void dm_sum(const HamDev<R> &h, const I *__restrict__
     for (int u = 0; u < G; ++u) {
       if (j + u < len) {
         const size_t r = (size_t)(j + u) * rs + row;
-        const R D0 = tload<UNI>(h.dvx + r), D1 = tload<UNI>(h.dvy + r),
-                D2 = tload<UNI>(h.dvz + r);
+        const R D0 = h.dvx[r], D1 = h.dvy[r], D2 = h.dvz[r];
         const R m0 = v[u].x * v[u].w, m1 = v[u].y * v[u].w, m2 = v[u].z * v[u].w;
         s0 = s0 + D2 * m1 - D1 * m2;
         s1 = s1 + D0 * m2 - D2 * m0;
@@ -2103,8 +2102,8 @@ __global__ void __launch_bounds__(256) k_mc_colour(HamDev<R> h, MCParams mp, Qua
 
 // ------------------------------------------------- resident MC of small systems
 // A system is one independent part of the lattice (no bond leaves it) in one
-// ensemble.  A small one is swept by one workgroup with its spins in LDS, all
-// the sweeps of a call in one launch: the colours of a sweep then cost a
+// ensemble.  A small one is swept by one workgroup with its spins in LDS, up to
+// 1024 sweeps of a call in one launch: the colours of a sweep then cost a
 // barrier each instead of a launch each, which is what a small system's sweep
 // consists of (a launch of a few hundred updates takes 6-7 us, the updates
 // themselves a fraction of one).
@@ -2119,8 +2118,10 @@ __global__ void __launch_bounds__(256) k_mc_colour(HamDev<R> h, MCParams mp, Qua
 // whose lanes chose freely would run the arithmetic of all three moves.  Every
 // update is arithmetically the one of k_mc_colour, from the same counters.
 //
-// What bounds it: instruction issue of the one CU for the trials, and for the
-// phases the latency of their chain (class, couplings, LDS gather, exp).
+// What bounds it: latency of the phases' chain (class, couplings, LDS gather,
+// exp) and their barriers.  2000 sites, 14 neighbours, FP64 Metropolis: 26 us a
+// sweep of nine phases, eight wavefronts, which wait in 62 % of their cycles and
+// issue VALU instructions in 19 %, 38 % of a SIMD's with its two wavefronts.
 struct ResDev {
   int ncomp, ncol;                      // systems per ensemble, colours
   int nmax, cmax;                       // sites of the largest system, of the largest phase
@@ -2297,15 +2298,18 @@ __global__ void __launch_bounds__(kResThreads, !HB && sizeof(R) == 4 ? 4 : 2)
 
 // ------------------------------------------------ resident LLG of small systems
 // The same for the LLG step: one workgroup per (independent system, ensemble)
-// with e, the predicted moments, b2eff and the lists in LDS, all steps of a
+// with e, the predicted moments, b2eff and the lists in LDS, 4 to 64 steps of a
 // call in one launch, two barriers a step instead of two launches.  Philox
 // deviates come from k_draw (nsave, quad array k for the k-th step of the
 // launch): drawn here they would keep the one CU busy for longer than the step
 // itself.  A site's arithmetic is that of k_llg.  Positions are device slots
 // counted from the system's first.
 //
-// What bounds it: instruction issue of one CU, hence the limit on the sites of
-// a system (llg_use_resident).
+// What bounds it: one CU, its latencies more than its issue.  432 sites, 14
+// neighbours, Depondt FP64: 5.6 us a step, seven wavefronts, which wait in 45 %
+// of their cycles (LDS gathers, two barriers) and issue VALU instructions in
+// 27 %, 55 % of a SIMD's that holds two of them.  With more than one site a
+// thread both grow with the sites, hence the limit (llg_use_resident).
 template <typename R, int ALG, bool LNB>
 __global__ void __launch_bounds__(kResThreads)
     k_llg_resident(HamDev<R> h, LLGDev<R> prm, ResDev rd, int nsteps, Quad<R> *s) {
