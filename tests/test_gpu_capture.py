@@ -154,3 +154,25 @@ def test_failed_automatic_capture_goes_on_with_launches():
     run(ref, 1)
     assert eng.launch_counts()[what + "_graph"] == 1
     assert np.array_equal(eng.get_moments()[0], ref.get_moments()[0])
+
+
+@pytest.mark.parametrize("asked", [0, 64])
+def test_settings_changed_while_replays_run(asked):
+    """A new temperature right after an asynchronous call ends the graphs that
+    call is still replaying; asked for or not, the moments are those of single
+    launches."""
+    out = []
+    for replayed in (True, False):
+        eng = _chain_engine(30000)
+        if replayed:
+            eng.set_graph_steps(asked)
+        else:
+            eng.set_kernel_timing(True)
+        for k in range(4):
+            eng.set_llg(0.1, 100.0 * (k + 1), 1e-16)
+            eng.sd_steps(5, 2048)
+            eng.sd_steps(5, 640)
+        n = eng.launch_counts()["llg_graph"]
+        assert n == ((4 * 2688 // 64 if asked else 4 * 10) if replayed else 0)
+        out.append(eng.get_moments()[0])
+    assert np.array_equal(out[0], out[1])

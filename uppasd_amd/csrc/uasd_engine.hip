@@ -1961,6 +1961,9 @@ template <typename F>
 int replay_graph(uasd_ctx *c, const std::tuple<int, int, int, uint64_t> &key, int idx,
                  uint64_t &host_ctr, int K, int timer, F &&body) {
   if (c->graphs_gen != c->gen || c->graphs.size() > 16) {
+    // HIP does not say that a graph outlives its last handle while it runs:
+    // the replays of an earlier call, which did not wait for them, end first
+    if (!c->graphs.empty()) HIP_TRY(hipStreamSynchronize(c->stream));
     destroy_graphs(c);
     c->graphs_gen = c->gen;
   }
