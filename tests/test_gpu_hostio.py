@@ -64,3 +64,35 @@ def test_context_holds_three_quads_a_pair(precision, per_pair):
     eng.set_moments(e, np.ones((1, N)))
     assert np.array_equal(eng.get_moments()[0], e)
     small.close()
+
+
+def test_moments_come_back_from_a_full_device():
+    """With too little device memory left for the largest piece of a transfer,
+    smaller pieces take it."""
+    import ctypes as C
+    import re
+    N = (1 << 22) + 5
+    e = np.random.default_rng(1).normal(size=(1, N, 3))
+    warm = U.Engine(N, 1)                              # what the runtime itself allocates
+    warm.set_moments(e, np.ones((1, N)))
+    warm.get_moments()
+    warm.close()
+    eng = U.Engine(N, 1)
+    eng.set_moments(e, np.ones((1, N)))
+    hip = C.CDLL(re.search(r"\S*libamdhip64\.so\S*", open("/proc/self/maps").read()).group(0))
+    held = []
+    try:
+        size = 1 << 35
+        while size >= 1 << 24:                         # leaves 16 to 32 MB of it
+            p = C.c_void_p()
+            if hip.hipMalloc(C.byref(p), C.c_size_t(size)) == 0:
+                held.append(p)
+            else:
+                hip.hipGetLastError()
+                size //= 2
+        hip.hipFree(held.pop())
+        got = eng.get_moments()
+    finally:
+        for p in held:
+            hip.hipFree(p)
+    assert np.array_equal(got[0], e) and np.array_equal(got[1], e)

@@ -417,7 +417,8 @@ int upload_raw(uasd_ctx *c, DevBuf &dst, const std::vector<T> &src) {
 // buffer of at most kIoPairs pairs, in stream order.  Against conversion on a
 // host thread with pageable quads in between: a step of the host-array halves
 // at 65,536 spins 2.13 -> 1.55 ms, moments of 4.1e6 pairs read back 95 -> 34 ms.
-constexpr size_t kIoPairs = (size_t)1 << 22;
+// A device with no room for that takes them in smaller pieces (io_pairs).
+constexpr size_t kIoPairs = (size_t)1 << 22, kIoPairsLeast = (size_t)1 << 16;
 
 // Host bytes of one pair in uasd_set_moments, its direction and magnitude, and
 // the bytes of b2eff they pass through: its quads, which in FP32 hold half of
@@ -555,12 +556,27 @@ int launch_unpack(uasd_ctx *c, const DevBuf &b, int k, size_t p0, size_t n, bool
   return UASD_OK;
 }
 
+// Pairs that pass through c->hostio at a time, allocated with the first call.
+int io_pairs(uasd_ctx *c, size_t *pairs) {
+  constexpr size_t kBytes = 3 * sizeof(double);
+  *pairs = std::min((size_t)c->N * c->M, kIoPairs);
+  while (!c->hostio.p) {
+    const hipError_t e = c->hostio.ensure(*pairs * kBytes);
+    if (e == hipSuccess) break;
+    if (e != hipErrorOutOfMemory || *pairs <= kIoPairsLeast) HIP_TRY(e);
+    (void)hipGetLastError();  // the smaller piece's launches have errors of their own
+    *pairs = std::max(*pairs / 4, kIoPairsLeast);
+  }
+  *pairs = std::min(*pairs, c->hostio.bytes / kBytes);
+  return UASD_OK;
+}
+
 // Host array a into quad array k of buffer b.  Asynchronous: a must stay as it
 // is until io.wait().
 int upload_vec(HostIo &io, DevBuf &b, int k, const double *a, PackW w) {
   uasd_ctx *c = io.c;
   HIP_TRY(b.ensure(std::max(b.bytes, (size_t)(k + 1) * quad_bytes(c))));
-  const size_t total = (size_t)c->N * c->M, step = std::min(total, kIoPairs);
+  const size_t total = (size_t)c->N * c->M;
   io.open = true;
   if (io.small()) {
     double *sa = nullptr;
@@ -568,7 +584,8 @@ int upload_vec(HostIo &io, DevBuf &b, int k, const double *a, PackW w) {
     std::memcpy(sa, a, 3 * total * sizeof(double));
     return launch_pack(c, b, k, 0, total, sa, nullptr, w);
   }
-  HIP_TRY(c->hostio.ensure(3 * step * sizeof(double)));
+  size_t step = 0;
+  if (int r = io_pairs(c, &step)) return r;
   double *sa = c->hostio.as<double>();
   for (size_t p0 = 0; p0 < total; p0 += step) {
     const size_t n = std::min(step, total - p0);
@@ -583,7 +600,7 @@ int upload_vec(HostIo &io, DevBuf &b, int k, const double *a, PackW w) {
 // Asynchronous: out is complete after io.wait().
 int download_vec(HostIo &io, const DevBuf &b, int k, double *out, bool times_w) {
   uasd_ctx *c = io.c;
-  const size_t total = (size_t)c->N * c->M, step = std::min(total, kIoPairs);
+  const size_t total = (size_t)c->N * c->M;
   io.open = true;
   if (io.small()) {
     double *so = nullptr;
@@ -591,7 +608,8 @@ int download_vec(HostIo &io, const DevBuf &b, int k, double *out, bool times_w) 
     io.outs.push_back({out, so, 3 * total});
     return launch_unpack(c, b, k, 0, total, times_w, so);
   }
-  HIP_TRY(c->hostio.ensure(3 * step * sizeof(double)));
+  size_t step = 0;
+  if (int r = io_pairs(c, &step)) return r;
   double *so = c->hostio.as<double>();
   for (size_t p0 = 0; p0 < total; p0 += step) {
     const size_t n = std::min(step, total - p0);
