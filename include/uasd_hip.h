@@ -288,7 +288,7 @@ int uasd_autotune_mc(uasd_ctx *ctx, char mode, const double *temps, int sweeps,
 /* Autotuner cache (no reference counterpart).  enable = 1 keeps every
  * autotuner winner for the process, keyed by the workload (kernel family,
  * solver or mode, precision, sizes, list widths, terms, site order, lattice
- * dimensions), and later uasd_autotune_* calls on the same workload take the
+ * dimensions) and the generation of the kernels, and later uasd_autotune_* calls on the same workload take the
  * kept shape without timing (best_ms is then the kept time).  path (may be
  * NULL) names a text file whose entries are loaded now and to which new
  * winners are appended.  enable = 0 switches the cache off and forgets it

@@ -262,3 +262,39 @@ def test_tune_cache_reuses_winners_and_persists(tmp_path):
         assert np.array_equal(d.get_moments()[0], e_c)
     finally:
         U.set_tune_cache(False)
+
+
+def test_tune_cache_leaves_entries_of_earlier_kernels(tmp_path):
+    """Entries whose keys name no generation of the kernels, or another one,
+    are not taken: the workload is timed."""
+    sysd = CF.bcc_shells(7, [1.34, 0.77])                 # 686 sites
+    N = sysd["lattice"].natom
+    path = tmp_path / "tune.txt"
+
+    def timed():
+        eng = U.Engine(N, 1)
+        eng.set_exchange(sysd["nlist"], sysd["nlistsize"], sysd["ncoup"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(1), 1),
+                        np.broadcast_to(sysd["mmom"], (1, N)))
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 1234)
+        eng.autotune_llg(1, steps=2)
+        return eng.launch_counts()["llg_list"] > 0
+
+    try:
+        U.set_tune_cache(True, str(path))
+        assert timed() and not timed()
+        line = path.read_text()
+        key, rest = line.split(" ", 1)
+        head, gen = key.rsplit("/k", 1)
+        for old in (head, f"{head}/k{int(gen) - 1}"):
+            path.write_text(f"{old} {rest}")
+            U.set_tune_cache(False)
+            U.set_tune_cache(True, str(path))
+            assert timed()
+        path.write_text(line)
+        U.set_tune_cache(False)
+        U.set_tune_cache(True, str(path))
+        assert not timed()
+    finally:
+        U.set_tune_cache(False)

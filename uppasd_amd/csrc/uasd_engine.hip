@@ -2595,22 +2595,27 @@ struct EventPair {
 // its text file when it names one: one line per workload, "key gather block
 // nt idx32 tile pipe best_ms".  The key holds what the launch shapes' speed
 // depends on: the kernel family, solver or mode, precision, sizes, list
-// widths, terms, site order, lattice dimensions, list entry width and noise
-// source (none at a uniform T = 0).
+// widths, terms, site order, lattice dimensions, list entry width, noise
+// source (none at a uniform T = 0) and kTuneKernels.
 std::mutex g_tune_mu;
 bool g_tune_on = false;
 std::string g_tune_path;
 std::map<std::string, std::pair<uasd::Tune, double>> g_tune;
 
+// kTuneKernels is the generation of the kernels that were timed: entries of an
+// earlier one (none in the key: 1) are times and winners of other code, and
+// some of its small systems' were those of a path that ignored the shape.
+constexpr int kTuneKernels = 2;
+
 std::string tune_key(const uasd_ctx *c, const char *kind, int alg) {
   char buf[320];
   std::snprintf(buf, sizeof buf,
                 "v2/gfx950/%s/a%d/%s/N%d/M%d/seg%d/W%d/Wd%d/an%d/ext%d/order%d/lat%d,%d,%d,%d/i16%d%d/"
-                "noise%d",
+                "noise%d/k%d",
                 kind, alg, c->prec == UASD_FP64 ? "fp64" : "fp32", c->N, c->M, c->nseg, c->W,
                 c->Wd, c->an_rows > 0 ? 1 : 0, c->ext_mode, c->order_na, c->lat_na, c->lat_n1,
                 c->lat_n2, c->lat_n3, c->use16 ? 1 : 0, c->use16_dm ? 1 : 0,
-                c->temp_uniform && c->temp0 == 0.0 ? 0 : c->noise_mode);
+                c->temp_uniform && c->temp0 == 0.0 ? 0 : c->noise_mode, kTuneKernels);
   return buf;
 }
 
