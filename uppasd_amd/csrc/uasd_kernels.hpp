@@ -663,6 +663,32 @@ __device__ __forceinline__ void exdm_sum(const HamDev<R> &h, const I *__restrict
     exdm_run<R, G, NT, I>(h, nb, src, site, ens, exrow, dmrow, h.ex_len[exrow], s0, s1, s2);
 }
 
+// The anisotropy field of one moment, added to s (uniaxial, cubic) and qf
+// (type 7's cubic part times sb).
+template <typename R>
+__device__ __forceinline__ void anisotropy(const HamDev<R> &h, const SiteClass &sc,
+                                           const Quad<R> *__restrict__ src, int site, int ens,
+                                           R (&s)[3], R (&qf)[3]) {
+  if (sc.an_row < 0) return;
+  const int t = h.an_type[sc.an_row];
+  if (t != 1 && t != 2 && t != 7) return;
+  R m0, m1, m2;
+  moment(src, (size_t)site * h.M + ens, m0, m1, m2);
+  if (t == 1) {
+    uniaxial(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
+  } else if (t == 2) {
+    cubic(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
+  } else {
+    R t0 = 0, t1 = 0, t2 = 0;
+    uniaxial(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
+    cubic(h, sc.an_row, m0, m1, m2, t0, t1, t2);
+    const R sb = h.an_sb[sc.an_row];
+    qf[0] = qf[0] + t0 * sb;
+    qf[1] = qf[1] + t1 * sb;
+    qf[2] = qf[2] + t2 * sb;
+  }
+}
+
 // G = neighbours whose loads are issued together (a tuning parameter).
 template <typename R, int G>
 __device__ __forceinline__ void site_field(const HamDev<R> &h, const Quad<R> *__restrict__ src,
@@ -702,26 +728,14 @@ __device__ __forceinline__ void site_field(const HamDev<R> &h, const Quad<R> *__
     else
       dm_sum<R, G>(h, h.dnbr + site, src, site, ens, sc.dm_row, s0, s1, s2);
   }
-  if (sc.an_row >= 0) {
-    const int t = h.an_type[sc.an_row];
-    if (t == 1 || t == 2 || t == 7) {
-      R m0, m1, m2;
-      moment(src, (size_t)site * M + ens, m0, m1, m2);
-      if (t == 1) {
-        uniaxial(h, sc.an_row, m0, m1, m2, s0, s1, s2);
-      } else if (t == 2) {
-        cubic(h, sc.an_row, m0, m1, m2, s0, s1, s2);
-      } else {
-        R t0 = 0, t1 = 0, t2 = 0;
-        uniaxial(h, sc.an_row, m0, m1, m2, s0, s1, s2);
-        cubic(h, sc.an_row, m0, m1, m2, t0, t1, t2);
-        const R sb = h.an_sb[sc.an_row];
-        qf0 = qf0 + t0 * sb;
-        qf1 = qf1 + t1 * sb;
-        qf2 = qf2 + t2 * sb;
-      }
-    }
-  }
+  R sf[3] = {s0, s1, s2}, qf[3] = {qf0, qf1, qf2};
+  anisotropy(h, sc, src, site, ens, sf, qf);
+  s0 = sf[0];
+  s1 = sf[1];
+  s2 = sf[2];
+  qf0 = qf[0];
+  qf1 = qf[1];
+  qf2 = qf[2];
   if (h.ext_mode == 1) {
     x0 = h.ext_u[3 * ens];
     x1 = h.ext_u[3 * ens + 1];
@@ -736,32 +750,6 @@ __device__ __forceinline__ void site_field(const HamDev<R> &h, const Quad<R> *__
   }
 }
 
-// The anisotropy field of the moment at quad q, added to s (uniaxial, cubic)
-// and qf (type 7's cubic part times sb) as site_field adds it.
-template <typename R>
-__device__ __forceinline__ void anisotropy(const HamDev<R> &h, const SiteClass &sc,
-                                           const Quad<R> *__restrict__ src, size_t q, R (&s)[3],
-                                           R (&qf)[3]) {
-  if (sc.an_row < 0) return;
-  const int t = h.an_type[sc.an_row];
-  if (t != 1 && t != 2 && t != 7) return;
-  R m0, m1, m2;
-  moment(src, q, m0, m1, m2);
-  if (t == 1) {
-    uniaxial(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
-  } else if (t == 2) {
-    cubic(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
-  } else {
-    R t0 = 0, t1 = 0, t2 = 0;
-    uniaxial(h, sc.an_row, m0, m1, m2, s[0], s[1], s[2]);
-    cubic(h, sc.an_row, m0, m1, m2, t0, t1, t2);
-    const R sb = h.an_sb[sc.an_row];
-    qf[0] = qf[0] + t0 * sb;
-    qf[1] = qf[1] + t1 * sb;
-    qf[2] = qf[2] + t2 * sb;
-  }
-}
-
 // The pair, DM and anisotropy parts of site_field for the U adjacent
 // ensembles e0 .. e0+U-1 of one site: the exchange terms of all U from one
 // read of the neighbour entries and couplings, then each ensemble's DM and
@@ -772,7 +760,7 @@ template <typename R, int G, int U>
 __device__ __forceinline__ void site_field_u(const HamDev<R> &h, const Quad<R> *__restrict__ src,
                                              int site, int e0, R (&sf)[U][3], R (&qf)[U][3]) {
   const SiteClass sc = site_class(h, site);
-  const int M = h.M, row = sc.ex_row;
+  const int row = sc.ex_row;
 #pragma unroll
   for (int k = 0; k < U; ++k) sf[k][0] = sf[k][1] = sf[k][2] = qf[k][0] = qf[k][1] = qf[k][2] = (R)0;
   if (h.nbr16) {
@@ -796,7 +784,7 @@ __device__ __forceinline__ void site_field_u(const HamDev<R> &h, const Quad<R> *
         dm_sum<R, G>(h, h.dnbr + site, src, site, e0 + k, sc.dm_row, sf[k][0], sf[k][1],
                      sf[k][2]);
     }
-    anisotropy(h, sc, src, (size_t)site * M + e0 + k, sf[k], qf[k]);
+    anisotropy(h, sc, src, site, e0 + k, sf[k], qf[k]);
   }
 }
 
@@ -2267,7 +2255,7 @@ __global__ void __launch_bounds__(kResThreads, !HB && sizeof(R) == 4 ? 4 : 2)
           if (Wd > 0 && sc.dm_row >= 0)
             dm_sum<R, G, uint16_t, NbDecId>(lh, dnb + p, sp, p, 0, sc.dm_row, f[0][0], f[0][1],
                                             f[0][2]);
-          anisotropy(h, sc, (const Quad<R> *)sp, (size_t)p, f[0], qf);
+          anisotropy(lh, sc, (const Quad<R> *)sp, p, 0, f[0], qf);
           double u0, u1, u2, u3;
           uniform4(mp.seed, kTagMCU, sweep, host_site(h, rd.site[off + p]), (uint32_t)ens, u0, u1,
                    u2, u3);
@@ -2345,7 +2333,7 @@ __global__ void __launch_bounds__(kResThreads)
     if (Wd > 0 && sc.dm_row >= 0)
       dm_sum<R, G, uint16_t, NbDecId>(lh, dnb + p, src, p, 0, sc.dm_row, f[0][0], f[0][1],
                                       f[0][2]);
-    anisotropy(h, sc, src, (size_t)p, f[0], qf);
+    anisotropy(lh, sc, src, p, 0, f[0], qf);
     if (h.ext_mode == 1) {
       x[0] = h.ext_u[3 * ens];
       x[1] = h.ext_u[3 * ens + 1];
