@@ -57,8 +57,8 @@ enum {
 };
 
 /* Launches counted by uasd_launch_counts: half steps of the list kernels and
- * of the tile kernel, resident launches (all the steps or sweeps of small
- * systems that fit one launch), deviates drawn ahead, colour passes, and
+ * of the tile kernel, resident launches (4 to 64 steps or up to 1024 sweeps of
+ * small systems in one launch), deviates drawn ahead, colour passes, and
  * replayed graphs of steps and of sweeps. */
 enum {
   UASD_LAUNCH_LLG_LIST = 0,
@@ -155,7 +155,8 @@ int uasd_evolve_second_host(uasd_ctx *ctx, int sdealgh, const double *beff,
 
 /* ---- device-resident hot path ---- */
 /* nsteps of the sd_mphase body (sd_driver.f90:668-765): field -> evolve_first
- * -> field -> evolve_second -> moment_update, fused into two kernels/step. */
+ * -> field -> evolve_second -> moment_update, fused into two kernels/step, or
+ * for systems of up to 512 sites into one launch of 4 to 64 steps. */
 int uasd_sd_steps(uasd_ctx *ctx, int sdealgh, int64_t nsteps);
 /* Graph-captured stepping (no reference counterpart: the reference has no
  * launches to capture): with steps_per_graph = K > 0, uasd_sd_steps and
@@ -198,7 +199,8 @@ int uasd_energy_terms(uasd_ctx *ctx, double *ene);
  * that must not call hipMalloc).  Same kernels, same results.  The partial
  * sums live in a fixed device array of 2^19 doubles (4 MiB) per device, held
  * until the process ends: (ceil(n_s / 4096) summed over segments + nseg) *
- * Mensemble * 4 must not exceed 2^19 (UASD_ERR_ARG otherwise).  The site-class
+ * Mensemble * 4 must not exceed 2^19 (UASD_ERR_ARG otherwise; the sums take
+ * chunks of 256 sites where those fit, of up to 4096 where they don't).  The site-class
  * tables must already be on the device: after a Hamiltonian upload that
  * changes them, call uasd_energy_terms (or a field, step or sweep entry point)
  * once first (UASD_ERR_STATE otherwise).  Every call on one device shares the
@@ -223,11 +225,15 @@ int uasd_get_coloring(uasd_ctx *ctx, int *ncolors, int *color_of_site);
  * kind (1: every launch) and around every uasd_sd_steps / uasd_mc_sweeps
  * call; -1 times the calls only, with no events between kernels; 0 switches
  * timing off.  Events between kernels cost time of their own, so a sampled
- * run keeps the stream close to an untimed one. */
+ * run keeps the stream close to an untimed one.  With n > 0 every LLG step is
+ * two half steps (or part of a replay that was asked for): small systems take
+ * no resident launches and nothing else is replayed, so the times are those of
+ * the half-step kernels.  -1 leaves the paths as they are.  Results are the
+ * same. */
 int uasd_set_kernel_timing(uasd_ctx *ctx, int enable);
-/* kind: 0 predictor, 1 corrector, 2 field, 3 MC colour pass (small systems:
- * one resident launch of all sweeps of a call), 4 LLG graph
- * replay (K steps), 5 MC graph replay (K sweeps), 6 a whole uasd_sd_steps or
+/* kind: 0 predictor, 1 corrector, 2 field, 3 MC colour pass (small systems: a
+ * resident launch of up to 1024 sweeps of a call), 4 LLG graph replay (K
+ * steps), 5 MC graph replay (K sweeps), 6 a whole uasd_sd_steps or
  * uasd_mc_sweeps call */
 int uasd_get_kernel_timing(uasd_ctx *ctx, int kind, int64_t *launches, double *total_ms);
 

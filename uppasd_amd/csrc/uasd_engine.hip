@@ -939,9 +939,9 @@ int build_llg_resident(uasd_ctx *c) {
 // 12.1 -> 10.7, 8.0 -> 8.0; 65 x 2016 (2189) 12.1 -> 13.9, 8.4 -> 8.5; 1 x 2048
 // (2019) 5.6 -> 3.6, 5.7 -> 2.4; 4 x 4096 (3866) 6.9 -> 7.8, 6.4 -> 4.4; 16 x 8192
 // (6349) 12.0 -> 17.8, 8.0 -> 11.4; 1 x 131,072 11.2 -> 167, 7.4 -> 86.
-// Not while the kernels
-// are timed one by one, graphs were asked for or a launch shape was: a shape
-// is one of the kernels that the resident launch would take the place of.
+// Not while the kernels are timed one by one, graphs were asked for or a launch
+// shape was: a shape is one of the kernels that the resident launch would take
+// the place of.
 bool llg_can_be_resident(const uasd_ctx *c) {
   return c->lres.ok && c->lres.cls_version == c->cls_version && c->graph_steps == 0 &&
          (int64_t)c->N * c->M <= kLlgResItems &&
@@ -2666,11 +2666,11 @@ void tune_keep(const std::string &key, bool resident, const uasd::Tune &t, doubl
   tune_store(resident ? resident_key(key, t.chosen == uasd::kShapeResident) : key, t, ms);
 }
 
-// Times `run` (asynchronous launches on c->stream) for every shape and leaves the fastest in *slot, marked as asked
-// for.  pair: also two ensembles per thread (the MC colour pass, M even);
-// resident: also the resident launch, which run() makes while the slot is
-// marked kShapeResident; where that is the fastest, the slot keeps the fastest
-// shape beside that mark.
+// Times `run` (asynchronous launches on c->stream) for every shape and leaves
+// the fastest in *slot, marked as asked for.  pair: also two ensembles per
+// thread (the MC colour pass, M even); resident: also the resident launch,
+// which run() makes while the slot is marked kShapeResident; where that is the
+// fastest, the slot keeps the fastest shape beside that mark.
 template <typename Run>
 int tune_search(uasd_ctx *c, uasd::Tune *slot, Run &&run, double *best_ms, bool pair,
                 bool resident) {
@@ -3006,7 +3006,7 @@ int uasd_energy_terms_noalloc(uasd_ctx *c, double *ene) {
     return fail(UASD_ERR_ARG,
                 "uasd_energy_terms_noalloc needs " + std::to_string(need) +
                     " doubles of scratch, more than its fixed " + std::to_string(kScratchDoubles) +
-                    ": (chunks of 4096 sites + segments) * ensembles * 4 must not exceed it; "
+                    ": (chunks of up to 4096 sites + segments) * ensembles * 4 must not exceed it; "
                     "use uasd_energy_terms");
   double *base = scratch_of(c->device);
   if (!base) return fail(UASD_ERR_STATE, "no scratch address for this device");

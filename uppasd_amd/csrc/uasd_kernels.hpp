@@ -1039,9 +1039,9 @@ __device__ __forceinline__ void midpoint_solve(R A0, R A1, R A2, R e0, R e1, R e
 // =================================================================== kernels
 
 // effective_field_full over all (site, ens): beff (quads, w unused; null where
-// only the energy is wanted) and, when en != null, the per-site field-routine energy -m.(0.5*(bs+2bq+2bext)) in FP64;
-// when parts != null also beff1 = bs into parts[q] and beff2 = bq + bext into
-// parts[N*M + q] (hamiltonianactions.f90:240-241).
+// only the energy is wanted) and, when en != null, the per-site field-routine
+// energy -m.(0.5*(bs+2bq+2bext)) in FP64; when parts != null also beff1 = bs into
+// parts[q] and beff2 = bq + bext into parts[N*M + q] (hamiltonianactions.f90:240-241).
 template <typename R, int G>
 __global__ void __launch_bounds__(256) k_field(HamDev<R> h, const Quad<R> *__restrict__ src,
                                                Quad<R> *__restrict__ beff, double *en,
@@ -1794,10 +1794,11 @@ __device__ __forceinline__ R sq(R x) {
 
 // The energy difference of calculate_energy (montecarlo_common.f90:431-865)
 // once the exchange fields f of the U ensembles are known: exchange,
-// anisotropy, DM (nbf(j) = the site's j-th DM neighbour) and external field; de[k] = mub*(E_trial - E_current).  The exchange energy of the
-// current and the trial moment, -sum_j J_j m.m_j (512-520), is formed as -m.f
-// with the exchange field f = sum_j J_j m_j of site_field: the same quantity
-// with a third of the arithmetic, equal to the term-by-term sums to rounding.
+// anisotropy, DM (nbf(j) = the site's j-th DM neighbour) and external field;
+// de[k] = mub*(E_trial - E_current).  The exchange energy of the current and the
+// trial moment, -sum_j J_j m.m_j (512-520), is formed as -m.f with the exchange
+// field f = sum_j J_j m_j of site_field: the same quantity with a third of the
+// arithmetic, equal to the term-by-term sums to rounding.
 template <typename R, int U, typename F>
 __device__ __forceinline__ void mc_energy_diff(const HamDev<R> &h, const SiteClass &sc,
                                                const Quad<R> *__restrict__ s, int e0, F &&nbf,

@@ -133,10 +133,11 @@ inline double res_idle_waves(int64_t waves, int64_t items, double weight) {
 // Whether a resident launch keeps its lists in LDS beside `base` bytes of
 // state: where they fit and do not make the workgroups take turns on a CU that
 // would hold several at once without them (`lds` bytes and `cu_waves` wavefronts
-// a CU, which the kernel's registers allow; 256 CUs).  1000 systems of 1024 sites with 58 neighbours, lists of 119 KB in
-// LDS (one workgroup a CU, four rounds) -> in global memory, us a sweep: FP32
-// Metropolis 327 -> 83, heat bath 370 -> 88, FP64 360 -> 86 (colour by colour
-// 180, 186, 283); 260 systems 97 -> 63, 186 -> 80, 169 -> 79.
+// a CU, which the kernel's registers allow; 256 CUs).  1000 systems of 1024
+// sites with 58 neighbours, lists of 119 KB in LDS (one workgroup a CU, four
+// rounds) -> in global memory, us a sweep: FP32 Metropolis 327 -> 83, heat bath
+// 370 -> 88, FP64 360 -> 86 (colour by colour 180, 186, 283); 260 systems
+// 97 -> 63, 186 -> 80, 169 -> 79.
 inline bool res_lists_in_lds(int64_t systems, int threads, int cu_waves, size_t base,
                              size_t lists, size_t lds) {
   if (base + lists > lds) return false;
