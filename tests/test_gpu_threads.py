@@ -3,6 +3,8 @@ time, whatever launch limits their kernels share.
 
 The dynamic LDS limit of a kernel belongs to the process, so a context whose
 systems need little LDS must not take it from one whose systems need much."""
+import ctypes as C
+import re
 import threading
 
 import numpy as np
@@ -92,3 +94,59 @@ def test_tile_shapes_in_threads():
     got = _in_threads([lambda a=a: run(*a) for a in sizes])
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+def _hip_calls():
+    """Ordinary calls of a program's other threads, which HIP refuses while any
+    stream of the process is being captured."""
+    hip = C.CDLL(re.search(r"\S*libamdhip64\.so\S*", open("/proc/self/maps").read()).group(0))
+    buf, host = C.c_void_p(), (C.c_char * 4096)()
+    assert hip.hipMalloc(C.byref(buf), C.c_size_t(4096)) == 0
+
+    def malloc():
+        p = C.c_void_p()
+        return hip.hipMalloc(C.byref(p), C.c_size_t(1 << 16)) or hip.hipFree(p)
+    return {"device": hip.hipDeviceSynchronize, "malloc": malloc,
+            "copy": lambda: hip.hipMemcpy(buf, host, C.c_size_t(4096), 1),
+            "legacy": lambda: hip.hipStreamSynchronize(None)}
+
+
+@pytest.mark.parametrize("asked", [0, 64])
+@pytest.mark.parametrize("call", ["device", "malloc", "copy", "legacy"])
+def test_other_threads_calls_while_graphs_are_built(call, asked):
+    """Steps that are replayed, asked for or not, neither fail nor make another
+    thread's calls fail while their graphs are built."""
+    def run(graph):
+        n = 1000
+        i = np.arange(n)
+        nl = np.stack([(i + 1) % n, (i - 1) % n], axis=1).astype(np.int32) + 1
+        eng = U.Engine(n, 1)
+        eng.set_exchange(nl, np.full(n, 2, np.int32), np.full((n, 2), 3.0))
+        eng.set_moments(CF.random_unit(n, np.random.default_rng(3), 1), np.ones((1, n)))
+        eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+        if graph:
+            eng.set_graph_steps(asked)
+        else:
+            eng.set_kernel_timing(True)
+        for k in range(12):
+            eng.set_llg(0.1, 100.0 + k, 1e-16)       # the graph of the last turn is stale
+            eng.sd_steps(5, 2048 if not asked else 64)
+            eng.sd_steps(5, 128)
+        assert (eng.launch_counts()["llg_graph"] > 0) == graph
+        return eng.get_moments()[0]
+
+    want = run(False)
+    hip_call, stop, codes = _hip_calls()[call], threading.Event(), set()
+
+    def other():
+        while not stop.is_set():
+            codes.add(hip_call())
+    t = threading.Thread(target=other)
+    t.start()
+    try:
+        got = run(True)
+    finally:
+        stop.set()
+        t.join()
+    assert np.array_equal(got, want)
+    assert codes == {0}

@@ -233,15 +233,15 @@ struct uasd_ctx {
   DevBuf seg_partial, seg_out, acc;
   int64_t acc_samples = 0;
 
-  // captured step graphs: replayed for runs of graph_steps LLG steps / MC
+  // step graphs: replayed for runs of graph_steps LLG steps / MC
   // sweeps; the Philox counters then live in ctr (0 LLG step, 1 MC sweep).
   int graph_steps = 0;
-  uint64_t gen = 0;           // bumped whenever a captured graph may be stale
+  uint64_t gen = 0;           // bumped whenever a recorded graph may be stale
   uint64_t graphs_gen = 0;
   DevBuf ctr;
   bool ctr_valid[2] = {false, false};
   uint64_t ctr_val[2] = {0, 0};
-  bool capturing = false;
+  uasd::Recording *rec = nullptr;  // while a graph of steps or sweeps is built
   bool replays_off = false;   // an automatic replay failed on this stream
   struct Graph {
     hipGraph_t g = nullptr;
@@ -737,7 +737,7 @@ hipEvent_t take_event(uasd_ctx *c) {
 }
 
 void tic(uasd_ctx *c, int kind) {
-  if (!c->timing || c->capturing) return;
+  if (!c->timing || c->rec) return;
   if (c->timing_tick[kind]++ % c->timing_every != 0) return;
   c->cur = take_event(c);
   // a start event that could not be recorded times nothing: back to the pool
@@ -748,7 +748,7 @@ void tic(uasd_ctx *c, int kind) {
 }
 
 int toc(uasd_ctx *c, int kind) {
-  if (!c->timing || c->capturing || !c->cur) return UASD_OK;
+  if (!c->timing || c->rec || !c->cur) return UASD_OK;
   hipEvent_t b = take_event(c);
   if (!b) return fail(UASD_ERR_HIP, "hipEventCreate failed");
   HIP_TRY(hipEventRecord(b, c->stream));
@@ -759,7 +759,7 @@ int toc(uasd_ctx *c, int kind) {
 
 // Event pair around a whole stepping call (kind 6), on the context stream.
 int region_tic(uasd_ctx *c) {
-  if (!c->timing_region || c->capturing) return UASD_OK;
+  if (!c->timing_region || c->rec) return UASD_OK;
   c->region_cur = take_event(c);
   if (!c->region_cur) return fail(UASD_ERR_HIP, "hipEventCreate failed");
   const hipError_t err = hipEventRecord(c->region_cur, c->stream);
@@ -781,9 +781,12 @@ int region_toc(uasd_ctx *c) {
   return UASD_OK;
 }
 
+// Where the launches of steps and sweeps go.
+uasd::Queue queue(const uasd_ctx *c) { return {c->stream, c->rec}; }
+
 // One launch of `kind` that runs now (not one recorded into a graph).
 void count(uasd_ctx *c, int kind) {
-  if (!c->capturing) c->launches[kind] += 1;
+  if (!c->rec) c->launches[kind] += 1;
 }
 
 int resolve_timing(uasd_ctx *c) {
@@ -998,7 +1001,7 @@ int ready_for_llg(uasd_ctx *c) {
 }
 
 // Quad arrays in c->spins: 0 e (emom), 1 p (emom2), 2 b2 (b2eff).
-// step_off >= 0: inside a graph capture, the step is *ctr[0] + step_off.
+// step_off >= 0: inside a recorded graph, the step is *ctr[0] + step_off.
 bool sde_supported(int alg) {
   return alg == UASD_SDE_MIDPOINT || alg == UASD_SDE_HEUN || alg == UASD_SDE_DEPONDT ||
          alg == UASD_SDE_SIB || alg == UASD_SDE_SPHMID;
@@ -1033,14 +1036,14 @@ int run_llg_half(uasd_ctx *c, int alg, int half, bool fused, bool write_e,
       uasd::TileDev t;
       if (int r = make_tile(c, c->tune[0].tile, t)) return r;
       tic(c, half);
-      HIP_TRY(uasd::launch_llg_tile<R>(c->stream, t, c->tune[0].pipe, alg, half, h, prm, e, p, b2,
+      HIP_TRY(uasd::launch_llg_tile<R>(queue(c), t, c->tune[0].pipe, alg, half, h, prm, e, p, b2,
                                        out));
       count(c, UASD_LAUNCH_LLG_TILE);
       return toc(c, half);
     }
   }
   tic(c, half);
-  HIP_TRY(uasd::launch_llg<R>(c->stream,
+  HIP_TRY(uasd::launch_llg<R>(queue(c),
                               uasd::default_tune(c->tune[0], (int64_t)c->N * c->M, c->W), alg,
                               half, fused, h, prm, e, p, b2, beff, out));
   count(c, UASD_LAUNCH_LLG_LIST);
@@ -1939,39 +1942,37 @@ void destroy_graphs(uasd_ctx *c) {
   c->graphs.clear();
 }
 
-// Records what body() enqueues on the context stream and instantiates it.
-// Graphs that nobody asked for are recorded on the context's own stream, which
-// nothing else uses or waits for: a caller's may not be capturable, or other
-// threads' work may be ordered with it.
+// Whether the context stream is known not to be capturing.
+bool stream_free(uasd_ctx *c) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(c->stream, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // not known: the next launch's error is its own
+  return false;
+}
+
+// Builds the graph of what body() enqueues and instantiates it.  Not for a
+// stream that a caller captures: its replays would not move the host's counter.
 template <typename F>
-int capture_graph(uasd_ctx *c, F &&body, uasd_ctx::Graph &out) {
-  const hipStream_t run = c->stream, rec = c->graph_steps > 0 ? run : c->own_stream;
-  HIP_TRY(hipStreamBeginCapture(rec, hipStreamCaptureModeThreadLocal));
-  c->capturing = true;
-  c->stream = rec;
+int record_graph(uasd_ctx *c, F &&body, uasd_ctx::Graph &out) {
+  if (!stream_free(c))
+    return fail(UASD_ERR_HIP, "graphs of steps or sweeps need a stream that is not being captured");
+  uasd::Recording rec;
+  HIP_TRY(hipGraphCreate(&rec.graph, 0));
+  c->rec = &rec;
   const int r = body();
-  c->stream = run;
-  c->capturing = false;
-  hipGraph_t g = nullptr;
-  const hipError_t e = hipStreamEndCapture(rec, &g);
-  if (r) {
-    if (g) (void)hipGraphDestroy(g);
-    return r;
-  }
-  if (e != hipSuccess)
-    return fail(UASD_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
+  c->rec = nullptr;
   hipGraphExec_t x = nullptr;
-  const hipError_t e2 = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-  if (e2 != hipSuccess) {
-    (void)hipGraphDestroy(g);
-    return fail(UASD_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e2));
+  const hipError_t e = r ? hipSuccess : hipGraphInstantiate(&x, rec.graph, nullptr, nullptr, 0);
+  if (r || e != hipSuccess) {
+    (void)hipGraphDestroy(rec.graph);
+    return r ? r : fail(UASD_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   }
-  out.g = g;
+  out.g = rec.graph;
   out.exec = x;
   return UASD_OK;
 }
 
-// Replays graph `key` (capturing it on first use), which advances device
+// Replays graph `key` (built on first use), which advances device
 // counter idx by K.  The device counter is first set to host_ctr when they
 // differ (after eager steps), with a kernel, so no memset or copy node is
 // ever recorded.
@@ -1988,11 +1989,11 @@ int replay_graph(uasd_ctx *c, const std::tuple<int, int, int, uint64_t> &key, in
   auto it = c->graphs.find(key);
   if (it == c->graphs.end()) {
     uasd_ctx::Graph gr;
-    if (int r = capture_graph(c, body, gr)) return r;
+    if (int r = record_graph(c, body, gr)) return r;
     it = c->graphs.emplace(key, gr).first;
   }
   if (!c->ctr_valid[idx] || c->ctr_val[idx] != host_ctr) {
-    HIP_TRY(uasd::launch_counter(c->stream, idx, c->ctr.as<uint64_t>(), host_ctr, 0));
+    HIP_TRY(uasd::launch_counter(queue(c), idx, c->ctr.as<uint64_t>(), host_ctr, 0));
     c->ctr_valid[idx] = true;
   }
   tic(c, timer);
@@ -2031,14 +2032,6 @@ int uasd_sd_steps(uasd_ctx *c, int alg, int64_t nsteps) {
 
 namespace {
 
-// Whether the context stream is known not to be capturing.
-bool stream_free(uasd_ctx *c) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(c->stream, &st) == hipSuccess) return st == hipStreamCaptureStatusNone;
-  (void)hipGetLastError();  // not known: the next launch's error is its own
-  return false;
-}
-
 // An automatic replay that failed: nothing of it ran, so the call goes on with
 // single launches, and no other replay is tried on this stream.
 void replay_failed(uasd_ctx *c) {
@@ -2064,7 +2057,7 @@ int launched_tile(uasd_ctx *c) {
   return tile_fits(c, c->tune[0].tile) ? c->tune[0].tile : 0;
 }
 
-// Deviates of n steps (from the context's step, or inside a capture from
+// Deviates of n steps (from the context's step, or inside a graph from
 // *ctr[0] + step_off) into c->nsave.
 template <typename R>
 int draw_ahead(uasd_ctx *c, int n, int64_t step_off) {
@@ -2073,12 +2066,12 @@ int draw_ahead(uasd_ctx *c, int n, int64_t step_off) {
     prm.step = (uint64_t)step_off;
     prm.step_dev = c->ctr.as<uint64_t>();
   }
-  HIP_TRY(uasd::launch_draw<R>(c->stream, ham_view<R>(c), prm, n, quads<R>(c, c->nsave)));
+  HIP_TRY(uasd::launch_draw<R>(queue(c), ham_view<R>(c), prm, n, quads<R>(c, c->nsave)));
   count(c, UASD_LAUNCH_DRAW);
   return UASD_OK;
 }
 
-// n LLG steps launched one by one; in_graph: inside a capture, counted from
+// n LLG steps launched one by one; in_graph: inside a graph, counted from
 // the device counter.
 int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
   int K = llg_view<double>(c).noise_mode == UASD_NOISE_PHILOX ? steps_ahead(c) : 1;
@@ -2154,7 +2147,7 @@ int sd_steps_run(uasd_ctx *c, int alg, int64_t nsteps) {
   auto replay = [&](int K) -> int {
     auto body = [&]() -> int {
       if (int r = llg_steps(c, alg, K, true)) return r;
-      HIP_TRY(uasd::launch_counter(c->stream, 0, c->ctr.as<uint64_t>(), (uint64_t)K, 1));
+      HIP_TRY(uasd::launch_counter(queue(c), 0, c->ctr.as<uint64_t>(), (uint64_t)K, 1));
       return UASD_OK;
     };
     for (; nsteps - s >= K; s += K)
@@ -2376,11 +2369,11 @@ static int mc_resident(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
     const int n = (int)std::min(kResSweeps, nsweeps - s);
     tic(c, 3);
     if (c->prec == UASD_FP64)
-      HIP_TRY(uasd::launch_mc_resident<double>(c->stream, ham_view<double>(c), mp, c->res.dev, n,
+      HIP_TRY(uasd::launch_mc_resident<double>(queue(c), ham_view<double>(c), mp, c->res.dev, n,
                                                (size_t)c->lds_max, quads<double>(c, c->spins, 0),
                                                quads<double>(c, c->spins, 1)));
     else
-      HIP_TRY(uasd::launch_mc_resident<float>(c->stream, ham_view<float>(c), mp, c->res.dev, n,
+      HIP_TRY(uasd::launch_mc_resident<float>(queue(c), ham_view<float>(c), mp, c->res.dev, n,
                                               (size_t)c->lds_max, quads<float>(c, c->spins, 0),
                                                quads<float>(c, c->spins, 1)));
     count(c, UASD_LAUNCH_MC_RESIDENT);
@@ -2413,10 +2406,10 @@ static int mc_run(uasd_ctx *c, uasd::MCParams mp, int64_t nsweeps) {
       mp.sstride = c->color_stride[col];
       tic(c, 3);
       if (c->prec == UASD_FP64) {
-        HIP_TRY(uasd::launch_mc<double>(c->stream, mc_tune(c, mp.nsites), ham_view<double>(c), mp,
+        HIP_TRY(uasd::launch_mc<double>(queue(c), mc_tune(c, mp.nsites), ham_view<double>(c), mp,
                                         quads<double>(c, c->spins, 0)));
       } else {
-        HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, mp.nsites), ham_view<float>(c), mp,
+        HIP_TRY(uasd::launch_mc<float>(queue(c), mc_tune(c, mp.nsites), ham_view<float>(c), mp,
                                        quads<float>(c, c->spins, 0)));
       }
       count(c, UASD_LAUNCH_MC_COLOUR);
@@ -2461,15 +2454,15 @@ int mc_sweeps_run(uasd_ctx *c, char mode, const uasd::MCParams &mp, int64_t nswe
           g.site0 = c->color_start[col];
           g.sstride = c->color_stride[col];
           if (c->prec == UASD_FP64) {
-            HIP_TRY(uasd::launch_mc<double>(c->stream, mc_tune(c, g.nsites), ham_view<double>(c), g,
+            HIP_TRY(uasd::launch_mc<double>(queue(c), mc_tune(c, g.nsites), ham_view<double>(c), g,
                                             quads<double>(c, c->spins, 0)));
           } else {
-            HIP_TRY(uasd::launch_mc<float>(c->stream, mc_tune(c, g.nsites), ham_view<float>(c), g,
+            HIP_TRY(uasd::launch_mc<float>(queue(c), mc_tune(c, g.nsites), ham_view<float>(c), g,
                                            quads<float>(c, c->spins, 0)));
           }
         }
       }
-      HIP_TRY(uasd::launch_counter(c->stream, 1, c->ctr.as<uint64_t>(), (uint64_t)K, 1));
+      HIP_TRY(uasd::launch_counter(queue(c), 1, c->ctr.as<uint64_t>(), (uint64_t)K, 1));
       return UASD_OK;
     };
     for (; nsweeps - s >= K; s += K)

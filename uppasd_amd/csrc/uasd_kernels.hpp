@@ -2655,7 +2655,7 @@ __global__ void k_accumulate(int nseg, int M, const int *__restrict__ seg_n,
 }
 
 // Graph support: the step / sweep counters live in device memory while a
-// captured graph runs; one thread adds or sets them (a vector global store).
+// recorded graph runs; one thread adds or sets them (a vector global store).
 template <int I>
 __global__ void k_counter(uint64_t *ctr, uint64_t value, int add) {
   if (blockIdx.x == 0 && threadIdx.x == 0) ctr[I] = add ? ctr[I] + value : value;

@@ -15,11 +15,7 @@ hipError_t launch_accumulate(hipStream_t s, int nseg, int M, const int *seg_n, c
   return hipGetLastError();
 }
 
-hipError_t launch_counter(hipStream_t s, int idx, uint64_t *ctr, uint64_t value, int add) {
-  if (idx == 0)
-    hipLaunchKernelGGL(k_counter<0>, dim3(1), dim3(64), 0, s, ctr, value, add);
-  else
-    hipLaunchKernelGGL(k_counter<1>, dim3(1), dim3(64), 0, s, ctr, value, add);
-  return hipGetLastError();
+hipError_t launch_counter(Queue s, int idx, uint64_t *ctr, uint64_t value, int add) {
+  return enqueue(s, idx == 0 ? k_counter<0> : k_counter<1>, dim3(1), dim3(64), 0, ctr, value, add);
 }
 }  // namespace uasd

@@ -36,7 +36,7 @@ hipError_t launch_field(hipStream_t s, const Tune &t, const HamDev<R> &h, const 
 }
 
 template <typename R, int ALG, int HALF, bool FUSED>
-static hipError_t llg_one(hipStream_t s, const Tune &t, const HamDev<R> &h,
+static hipError_t llg_one(Queue s, const Tune &t, const HamDev<R> &h,
                           const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p, Quad<R> *b2,
                           const Quad<R> *beff, Quad<R> *out) {
   const int64_t n = (int64_t)h.N * h.M;
@@ -44,19 +44,16 @@ static hipError_t llg_one(hipStream_t s, const Tune &t, const HamDev<R> &h,
   const dim3 grid(grid_for(n, t.block)), block(t.block);
   const HamDev<R> hh = tuned(h, t);
   if (!FUSED) {  // no gather: one instance
-    hipLaunchKernelGGL((k_llg<R, ALG, HALF, false, 4>), grid, block, 0, s, hh, prm, e, p, b2,
-                       beff, out);
-    return hipGetLastError();
+    return enqueue(s, k_llg<R, ALG, HALF, false, 4>, grid, block, 0, hh, prm, e, p, b2, beff, out);
   }
   return with_gather(t, [&](auto g) {
-    hipLaunchKernelGGL((k_llg<R, ALG, HALF, true, decltype(g)::value>), grid, block, 0, s, hh,
-                       prm, e, p, b2, beff, out);
-    return hipGetLastError();
+    return enqueue(s, k_llg<R, ALG, HALF, true, decltype(g)::value>, grid, block, 0, hh, prm, e, p,
+                   b2, beff, out);
   });
 }
 
 template <typename R>
-hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fused,
+hipError_t launch_llg(Queue s, const Tune &t, int alg, int half, bool fused,
                       const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p,
                       Quad<R> *b2, const Quad<R> *beff, Quad<R> *out) {
   if (!tune_valid(t)) return hipErrorInvalidValue;
@@ -88,18 +85,17 @@ hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fuse
 }
 
 template <typename R>
-hipError_t launch_draw(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
+hipError_t launch_draw(Queue s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
                        Quad<R> *out) {
   const int64_t n = (int64_t)h.N * h.M;
   if (n == 0 || steps <= 0) return hipSuccess;
   const int block = n <= 64 * 256 ? 64 : kBlock;
-  hipLaunchKernelGGL((k_draw<R>), dim3((unsigned)((n + block - 1) / block), (unsigned)steps),
-                     dim3(block), 0, s, h, prm, steps, out);
-  return hipGetLastError();
+  return enqueue(s, k_draw<R>, dim3((unsigned)((n + block - 1) / block), (unsigned)steps),
+                 dim3(block), 0, h, prm, steps, out);
 }
 
 template <typename R>
-hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
+hipError_t launch_mc(Queue s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
                      Quad<R> *spins) {
   const int64_t n = (int64_t)mp.nsites * h.M;
   if (n == 0) return hipSuccess;
@@ -112,18 +108,11 @@ hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCP
   return with_gather(t, [&](auto g) {
     constexpr int G = decltype(g)::value;
     const dim3 grid(grid_for(two ? n / 2 : n, t.block)), block(t.block);
-    if (mp.heat_bath) {
-      if (two)
-        hipLaunchKernelGGL((k_mc_colour<R, G, 2, true>), grid, block, 0, s, hh, m, spins);
-      else
-        hipLaunchKernelGGL((k_mc_colour<R, G, 1, true>), grid, block, 0, s, hh, m, spins);
-    } else {
-      if (two)
-        hipLaunchKernelGGL((k_mc_colour<R, G, 2, false>), grid, block, 0, s, hh, m, spins);
-      else
-        hipLaunchKernelGGL((k_mc_colour<R, G, 1, false>), grid, block, 0, s, hh, m, spins);
-    }
-    return hipGetLastError();
+    if (mp.heat_bath)
+      return two ? enqueue(s, k_mc_colour<R, G, 2, true>, grid, block, 0, hh, m, spins)
+                 : enqueue(s, k_mc_colour<R, G, 1, true>, grid, block, 0, hh, m, spins);
+    return two ? enqueue(s, k_mc_colour<R, G, 2, false>, grid, block, 0, hh, m, spins)
+               : enqueue(s, k_mc_colour<R, G, 1, false>, grid, block, 0, hh, m, spins);
   });
 }
 
@@ -161,19 +150,18 @@ hipError_t launch_llg_resident(hipStream_t s, int alg, const HamDev<R> &h, const
 }
 
 template <typename R, bool HB, bool TRL, bool LNB>
-static hipError_t mc_resident_one(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
+static hipError_t mc_resident_one(Queue s, const HamDev<R> &h, const MCParams &mp,
                                   const ResDev &rd, int nsweeps, size_t bytes, int threads,
                                   Quad<R> *spins, Quad<R> *trials) {
   static LdsLimit limit;
   const hipError_t err = limit.raise((const void *)&k_mc_resident<R, HB, TRL, LNB>, bytes);
   if (err != hipSuccess) return err;
-  hipLaunchKernelGGL((k_mc_resident<R, HB, TRL, LNB>), dim3((unsigned)(rd.ncomp * h.M)),
-                     dim3(threads), bytes, s, h, mp, rd, nsweeps, spins, trials);
-  return hipGetLastError();
+  return enqueue(s, k_mc_resident<R, HB, TRL, LNB>, dim3((unsigned)(rd.ncomp * h.M)),
+                 dim3(threads), bytes, h, mp, rd, nsweeps, spins, trials);
 }
 
 template <typename R>
-hipError_t launch_mc_resident(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
+hipError_t launch_mc_resident(Queue s, const HamDev<R> &h, const MCParams &mp,
                               const ResDev &rd, int nsweeps, size_t lds, Quad<R> *spins,
                               Quad<R> *trials) {
   const size_t sp = res_lds_spins(sizeof(R), rd.nmax), lists = res_lds_lists(rd.nmax, h.W + h.Wd);
@@ -206,7 +194,7 @@ hipError_t launch_mc_resident(hipStream_t s, const HamDev<R> &h, const MCParams 
 }
 
 template <typename R>
-hipError_t launch_llg_tile(hipStream_t s, TileDev t, int pipe, int alg, int half,
+hipError_t launch_llg_tile(Queue s, TileDev t, int pipe, int alg, int half,
                            const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e,
                            Quad<R> *p, Quad<R> *b2, Quad<R> *out) {
   switch (alg) {
@@ -292,19 +280,19 @@ hipError_t launch_energy_terms(hipStream_t s, const HamDev<R> &h, int nseg, int 
 #define UASD_INSTANTIATE(R)                                                                   \
   template hipError_t launch_field<R>(hipStream_t, const Tune &, const HamDev<R> &,           \
                                       const Quad<R> *, Quad<R> *, double *, Quad<R> *);       \
-  template hipError_t launch_llg<R>(hipStream_t, const Tune &, int, int, bool,                \
+  template hipError_t launch_llg<R>(Queue, const Tune &, int, int, bool,                \
                                     const HamDev<R> &, const LLGDev<R> &, const Quad<R> *,    \
                                     Quad<R> *, Quad<R> *, const Quad<R> *, Quad<R> *);        \
-  template hipError_t launch_draw<R>(hipStream_t, const HamDev<R> &, const LLGDev<R> &, int,   \
+  template hipError_t launch_draw<R>(Queue, const HamDev<R> &, const LLGDev<R> &, int,   \
                                      Quad<R> *);                                              \
-  template hipError_t launch_mc<R>(hipStream_t, const Tune &, const HamDev<R> &,              \
+  template hipError_t launch_mc<R>(Queue, const Tune &, const HamDev<R> &,              \
                                    const MCParams &, Quad<R> *);                              \
   template hipError_t launch_llg_resident<R>(hipStream_t, int, const HamDev<R> &,             \
                                              const LLGDev<R> &, const ResDev &, int, size_t,  \
                                              Quad<R> *);                                      \
-  template hipError_t launch_mc_resident<R>(hipStream_t, const HamDev<R> &, const MCParams &,  \
+  template hipError_t launch_mc_resident<R>(Queue, const HamDev<R> &, const MCParams &,  \
                                             const ResDev &, int, size_t, Quad<R> *, Quad<R> *); \
-  template hipError_t launch_llg_tile<R>(hipStream_t, TileDev, int, int, int,              \
+  template hipError_t launch_llg_tile<R>(Queue, TileDev, int, int, int,              \
                                          const HamDev<R> &, const LLGDev<R> &,                \
                                          const Quad<R> *, Quad<R> *, Quad<R> *, Quad<R> *);   \
   template hipError_t launch_reduce<R>(hipStream_t, int, int, const Quad<R> *, const double *, \

@@ -40,6 +40,47 @@ struct LdsLimit {
   }
 };
 
+// A graph under construction: its kernels run one after the other.
+struct Recording {
+  hipGraph_t graph = nullptr;
+  hipGraphNode_t last = nullptr;
+};
+
+// Where a launch goes: to a stream, or to the end of a graph.  Graphs are built
+// node by node, not captured from a stream: while any stream of the process is
+// capturing, HIP refuses ordinary calls of other threads (hipDeviceSynchronize,
+// legacy-stream copies), which in turn break the capture.
+struct Queue {
+  hipStream_t stream;
+  Recording *rec = nullptr;
+};
+
+template <typename T>
+struct Same {
+  using type = T;
+};
+
+template <typename... P>
+hipError_t enqueue(const Queue &q, void (*kern)(P...), dim3 grid, dim3 block, size_t lds,
+                   typename Same<P>::type... args) {
+  if (!q.rec) {
+    hipLaunchKernelGGL(kern, grid, block, lds, q.stream, args...);
+    return hipGetLastError();
+  }
+  void *params[] = {(void *)&args...};
+  hipKernelNodeParams n{};
+  n.func = (void *)kern;
+  n.gridDim = grid;
+  n.blockDim = block;
+  n.sharedMemBytes = (unsigned)lds;
+  n.kernelParams = params;  // copied by the call
+  hipGraphNode_t node = nullptr;
+  const hipError_t err =
+      hipGraphAddKernelNode(&node, q.rec->graph, &q.rec->last, q.rec->last ? 1 : 0, &n);
+  if (err == hipSuccess) q.rec->last = node;
+  return err;
+}
+
 // Launch shape of the gathering kernels (chosen by the autotuner):
 //   gather  neighbours whose loads are issued together: 2, 4, 8 or 16
 //   block   workgroup size: 64, 128 or 256
@@ -110,7 +151,7 @@ hipError_t launch_field(hipStream_t s, const Tune &t, const HamDev<R> &h, const 
 
 // alg: 1 midpoint / 5 Depondt; half: 0 predictor, 1 corrector
 template <typename R>
-hipError_t launch_llg(hipStream_t s, const Tune &t, int alg, int half, bool fused,
+hipError_t launch_llg(Queue s, const Tune &t, int alg, int half, bool fused,
                       const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p,
                       Quad<R> *b2, const Quad<R> *beff, Quad<R> *out);
 
@@ -160,18 +201,18 @@ inline size_t res_lds_llg(size_t rsize, int nmax) { return 12 * rsize * (size_t)
 
 // Deviates of `steps` steps from prm.step on into as many quad arrays of out.
 template <typename R>
-hipError_t launch_draw(hipStream_t s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
+hipError_t launch_draw(Queue s, const HamDev<R> &h, const LLGDev<R> &prm, int steps,
                        Quad<R> *out);
 
 template <typename R>
-hipError_t launch_mc(hipStream_t s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
+hipError_t launch_mc(Queue s, const Tune &t, const HamDev<R> &h, const MCParams &mp,
                      Quad<R> *spins);
 
 // nsweeps sweeps of every system with k_mc_resident; lds = LDS bytes a
 // workgroup may use, trials = N*M quads of scratch for the trial moves that do
 // not fit in them (not read before they are written).
 template <typename R>
-hipError_t launch_mc_resident(hipStream_t s, const HamDev<R> &h, const MCParams &mp,
+hipError_t launch_mc_resident(Queue s, const HamDev<R> &h, const MCParams &mp,
                               const ResDev &rd, int nsweeps, size_t lds, Quad<R> *spins,
                               Quad<R> *trials);
 
@@ -185,12 +226,12 @@ inline size_t res_lds_spins(size_t rsize, int nmax) {
 // Fused LLG half-step with the LDS-tiled stencil kernel, work units (tile,
 // ensemble).
 template <typename R>
-hipError_t launch_llg_tile(hipStream_t s, TileDev t, int pipe, int alg, int half,
+hipError_t launch_llg_tile(Queue s, TileDev t, int pipe, int alg, int half,
                            const HamDev<R> &h, const LLGDev<R> &prm, const Quad<R> *e,
                            Quad<R> *p, Quad<R> *b2, Quad<R> *out);
 // The same for one solver; uasd_tile.hip instantiates each (R, ALG).
 template <typename R, int ALG>
-hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, const HamDev<R> &h,
+hipError_t launch_llg_tile_alg(Queue s, TileDev t, int pipe, int half, const HamDev<R> &h,
                                const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p, Quad<R> *b2,
                                Quad<R> *out);
 // LDS bytes the tile kernel needs for a halo tile of hv cells
@@ -230,7 +271,7 @@ hipError_t launch_energy_terms(hipStream_t s, const HamDev<R> &h, int nseg, int 
                                double *partial, double *out);
 
 // ctr[idx] = value (add = 0) or ctr[idx] += value (add = 1), on the stream.
-hipError_t launch_counter(hipStream_t s, int idx, uint64_t *ctr, uint64_t value, int add);
+hipError_t launch_counter(Queue s, int idx, uint64_t *ctr, uint64_t value, int add);
 
 // Appends one cumulant sample per (segment, ensemble) from out of launch_segsum.
 hipError_t launch_accumulate(hipStream_t s, int nseg, int M, const int *seg_n,

@@ -6,7 +6,7 @@
 namespace uasd {
 
 template <typename R, int ALG>
-hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, const HamDev<R> &h,
+hipError_t launch_llg_tile_alg(Queue s, TileDev t, int pipe, int half, const HamDev<R> &h,
                                const LLGDev<R> &prm, const Quad<R> *e, Quad<R> *p, Quad<R> *b2,
                                Quad<R> *out) {
   // work units: (tile, ensemble) pairs
@@ -55,17 +55,15 @@ hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, con
   };
 #define UASD_TILE_CASE(H, PL, F, E)                                                             \
   if (half == H && plane == PL && full == F && ens == E) {                                      \
-    const void *kern = (const void *)&k_llg_tile<R, ALG, H, PL, F, E>;                          \
+    const auto kern = k_llg_tile<R, ALG, H, PL, F, E>;                                          \
     static LdsLimit limit;                                                                      \
     static Slots slots;                                                                         \
-    hipError_t err = limit.raise(kern, lds);                                                    \
-    if (err == hipSuccess) err = units_per_wg(kern, slots);                                     \
+    hipError_t err = limit.raise((const void *)kern, lds);                                      \
+    if (err == hipSuccess) err = units_per_wg((const void *)kern, slots);                       \
     if (err != hipSuccess) return err;                                                          \
     const int nwg = (nunits + t.per - 1) / t.per;                                               \
     const dim3 grid((nwg + kXCD - 1) / kXCD * kXCD), block(threads);                            \
-    hipLaunchKernelGGL((k_llg_tile<R, ALG, H, PL, F, E>), grid, block, lds, s, tile_ham(h), prm, \
-                       t, e, p, b2, out);                                                       \
-    return hipGetLastError();                                                                   \
+    return enqueue(s, kern, grid, block, lds, tile_ham(h), prm, t, e, p, b2, out);              \
   }
 #define UASD_TILE_FULL(H, PL)                                                                   \
   UASD_TILE_CASE(H, PL, false, false)                                                           \
@@ -86,7 +84,7 @@ hipError_t launch_llg_tile_alg(hipStream_t s, TileDev t, int pipe, int half, con
   return hipErrorInvalidValue;
 }
 
-template hipError_t launch_llg_tile_alg<UASD_REAL, UASD_ALG>(hipStream_t, TileDev, int, int,
+template hipError_t launch_llg_tile_alg<UASD_REAL, UASD_ALG>(Queue, TileDev, int, int,
                                                              const HamDev<UASD_REAL> &,
                                                              const LLGDev<UASD_REAL> &,
                                                              const Quad<UASD_REAL> *,
