@@ -401,3 +401,27 @@ def test_largest_resident_systems(kind, n, resident):
     eng.sd_steps(5, 8) if kind == "llg" else eng.mc_sweeps(kind, 300.0, 2, 9)
     c = eng.launch_counts()
     assert (c["llg_resident" if kind == "llg" else "mc_resident"] == 1) == resident
+
+
+@pytest.mark.parametrize("kind", ["llg", "mc"])
+def test_tuned_batches_stay_resident(kind):
+    """A search over calls of one sweep or three steps, whose resident launches
+    are mostly the loading of their systems, does not cost a batch of small
+    systems the resident launches of its longer calls."""
+    rng = np.random.default_rng(7)
+    reps = [CF.bcc_alloy(L, rng.integers(0, 2, 2 * L ** 3)) for L in (5, 6, 7, 5, 6, 7, 5, 6)] \
+        if kind == "mc" else [CF.bcc_shells(L, [1.34, 0.77], moment=2.2) for L in (4, 5, 6, 4, 5, 6)]
+    j = Bt.join(reps)
+    M = 32 if kind == "mc" else 1
+    eng = Bt.engine_for(j, M, "fp32")
+    eng.set_moments(CF.random_unit(j.natom, rng, M), np.broadcast_to(j.mmom, (M, j.natom)))
+    eng.set_llg(0.1, 300.0, 1e-16)
+    eng.set_noise(U.UASD_NOISE_PHILOX, 3)
+    if kind == "mc":
+        eng.autotune_mc("M", np.linspace(200.0, 1600.0, M))
+    else:
+        eng.autotune_llg(5)
+    before = eng.launch_counts()
+    eng.mc_sweeps("M", np.linspace(200.0, 1600.0, M), 20, 5) if kind == "mc" else eng.sd_steps(5, 20)
+    after = eng.launch_counts()
+    assert {k for k in after if after[k] > before[k]} - {"draw"} == {kind + "_resident"}
