@@ -160,3 +160,35 @@ def test_colour_pass_with_scalar_couplings(mode, precision):
         out.append(eng.get_moments()[0][:, :n])
     for e in out[1:]:
         assert np.array_equal(e, out[0])
+
+
+def test_no_room_for_resident_tables():
+    """On a device filled after a context's set-up, systems whose resident tables
+    find no room are launched, with the same results."""
+    import ctypes as C
+    import re
+    s = Bt.join([_circulant(512, 70) for _ in range(32)])       # lists of 4.6 MB
+    out = []
+    for full in (False, True):
+        eng = Bt.engine_for(s, 1, "fp64")
+        eng.set_moments(CF.random_unit(s.natom, np.random.default_rng(3), 1), s.mmom[None])
+        eng.set_llg(0.1, 0.0, 1e-16)
+        eng.field(with_energy=True)
+        hip = C.CDLL(re.search(r"\S*libamdhip64\.so\S*", open("/proc/self/maps").read()).group(0))
+        held, size = [], 1 << 35 if full else 0
+        try:
+            while size >= 1 << 21:
+                p = C.c_void_p()
+                if hip.hipMalloc(C.byref(p), C.c_size_t(size)) == 0:
+                    held.append(p)
+                else:
+                    hip.hipGetLastError()
+                    size //= 2
+            eng.sd_steps(5, 12)
+            c = eng.launch_counts()
+            out.append(eng.get_moments()[0])
+        finally:
+            for p in held:
+                hip.hipFree(p)
+        assert (c["llg_resident"], c["llg_list"]) == ((0, 24) if full else (1, 0))
+    assert np.array_equal(out[0], out[1])

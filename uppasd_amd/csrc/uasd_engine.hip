@@ -911,7 +911,10 @@ int build_llg_resident(uasd_ctx *c) {
   std::memcpy(all.data(), cls.data(), ooff);
   std::memcpy(all.data() + ooff, off.data(), off.size() * sizeof(int));
   std::memcpy(all.data() + onb, nb.data(), nb.size() * sizeof(uint16_t));
-  if (int e = upload_raw(c, r.buf, all)) return e;
+  if (upload_raw(c, r.buf, all)) {  // no room for tables that the launched kernels do not need
+    (void)hipGetLastError();
+    return UASD_OK;
+  }
   const char *base = r.buf.as<char>();
   r.dev = uasd::ResDev{};
   r.dev.ncomp = ncomp;
@@ -2258,7 +2261,10 @@ static int build_resident(uasd_ctx *c) {
                optr = put(ptr.data(), ptr.size() * sizeof(int)),
                osite = put(site.data(), site.size() * sizeof(int)),
                onb = put(nb.data(), nb.size() * sizeof(uint16_t));
-  if (int e = upload_raw(c, r.buf, all)) return e;
+  if (upload_raw(c, r.buf, all)) {  // no room for tables that the launched kernels do not need
+    (void)hipGetLastError();
+    return UASD_OK;
+  }
   const char *base = r.buf.as<char>();
   r.dev = uasd::ResDev{ncomp,
                        ncol,
