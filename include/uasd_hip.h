@@ -158,14 +158,15 @@ int uasd_evolve_second_host(uasd_ctx *ctx, int sdealgh, const double *beff,
  * -> field -> evolve_second -> moment_update, fused into two kernels/step, or
  * for systems of up to 512 sites into one launch of 4 to 64 steps. */
 int uasd_sd_steps(uasd_ctx *ctx, int sdealgh, int64_t nsteps);
-/* Graph-captured stepping (no reference counterpart: the reference has no
- * launches to capture): with steps_per_graph = K > 0, uasd_sd_steps and
+/* Stepping by graph replays (no reference counterpart: the reference has no
+ * launches to replay): with steps_per_graph = K > 0, uasd_sd_steps and
  * uasd_mc_sweeps replay a hipGraph of K steps (K sweeps) for every full run of
  * K, and launch the rest one by one; the numbers are the same either way.
  * The Philox counters then advance on the device.  0 (the default) leaves it
  * to the library, which replays the steps or sweeps of small systems once
  * enough of them have run under unchanged settings (not while kernels are
- * timed or the stream is being captured). */
+ * timed or the stream is being captured).  Graphs are built without capturing
+ * a stream, so other threads' calls are not disturbed. */
 int uasd_set_graph_steps(uasd_ctx *ctx, int steps_per_graph);
 /* Field of the resident moments into a host array (NULL skips the copy). */
 int uasd_effective_field(uasd_ctx *ctx, double *beff, double *energy);

@@ -2102,9 +2102,9 @@ int llg_steps(uasd_ctx *c, int alg, int64_t n, bool in_graph) {
 // 0.4-1.6 us shorter than an enqueued one (its arguments already lie in device
 // memory): 432 sites, 14 neighbours, FP64 13.3 -> 10.3 us a step, FP32 11.9 ->
 // 8.6; 16,000 sites 14.3 -> 11.7; 65,536 sites (film) FP32 14.8 -> 13.0, FP64
-// 16.7 -> 15.6; nothing from 2^18 items on.  Capturing costs 25 us a launch
-// (4 ms for 80 steps), which 2048 steps or 512 sweeps would have repaid, hence
-// `after`.
+// 16.7 -> 15.6; nothing from 2^18 items on.  Building a graph costs 3.3 us a
+// launch (430 us for 64 steps) and the process's first 3.6 ms more, which 2048
+// steps or 512 sweeps would have repaid, hence `after`.
 bool repeats_pay(uasd_ctx *c, int kind, int alg, uint64_t seed, int64_t items, int64_t n,
                  int64_t after) {
   if (c->graph_steps > 0 || c->timing || c->replays_off || items > 131072) return false;
