@@ -176,3 +176,32 @@ def test_settings_changed_while_replays_run(asked):
         assert n == ((4 * 2688 // 64 if asked else 4 * 10) if replayed else 0)
         out.append(eng.get_moments()[0])
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("kind", ["tile", "resident"])
+def test_graphs_of_kernels_with_much_lds(kind, precision):
+    """Graph nodes of kernels that ask for more than 64 KB of LDS: the tile
+    kernel and resident sweeps, replays against launches."""
+    L, shells = ((16, 16, 16), CF.bcc5_couplings()) if kind == "tile" else ((12, 12, 12), [1.34, 0.77])
+    s = CF.bcc_shells(L, shells, moment=2.2)
+    N, out = s["lattice"].natom, []
+    for graph in (0, 4):
+        eng = U.Engine(N, 1, precision, site_order=2)
+        eng.set_lattice_dims(2, *L)
+        eng.set_exchange(s["nlist"], s["nlistsize"], s["ncoup"])
+        eng.set_moments(CF.random_unit(N, np.random.default_rng(3), 1), s["mmom"][None])
+        eng.set_llg(0.1, 300.0, 1e-16)
+        eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+        eng.set_graph_steps(graph)
+        if kind == "tile":
+            eng.set_tuning(eng.TUNE_LLG, 4, 256 | (4 << 18) | 0x400000)
+            assert eng.llg_tile() == 4
+        for k in (4, 9, 3):
+            eng.sd_steps(1, k) if kind == "tile" else eng.mc_sweeps("M", 400.0, k, 5)
+            eng.measure()
+        c = eng.launch_counts()
+        assert c["llg_graph"] + c["mc_graph"] == (3 if graph else 0)
+        assert (c["llg_tile"] > 0) == (kind == "tile") and (c["mc_resident"] > 0) != (kind == "tile")
+        out.append(eng.get_moments()[0])
+    assert np.array_equal(out[0], out[1])

@@ -150,3 +150,26 @@ def test_other_threads_calls_while_graphs_are_built(call, asked):
         t.join()
     assert np.array_equal(got, want)
     assert codes == {0}
+
+
+def test_replays_in_threads():
+    """Contexts on four threads whose steps and sweeps are replayed, their graphs
+    built and dropped side by side."""
+    def run(n, alg):
+        i = np.arange(n)
+        nl = np.stack([(i + 1) % n, (i - 1) % n], axis=1).astype(np.int32) + 1
+        eng = U.Engine(n, 1)
+        eng.set_exchange(nl, np.full(n, 2, np.int32), np.full((n, 2), 3.0))
+        eng.set_moments(CF.random_unit(n, np.random.default_rng(n), 1), np.ones((1, n)))
+        eng.set_noise(U.UASD_NOISE_PHILOX, 7)
+        eng.set_graph_steps(16)
+        for k in range(20):
+            eng.set_llg(0.1, 100.0 + k, 1e-16)
+            eng.sd_steps(alg, 40)
+            eng.mc_sweeps("M", 400.0, 20, k)
+        return eng.get_moments()[0]
+    jobs = [(1000, 5), (777, 1), (20000, 4), (12000, 5)]
+    want = [run(*a) for a in jobs]
+    got = _in_threads([lambda a=a: run(*a) for a in jobs])
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
